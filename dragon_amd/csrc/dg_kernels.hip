@@ -9,6 +9,7 @@
 // R of reconstruction and Riemann solves (double: drop-in; float: the mixed
 // form, whose state, accumulation, pressure recovery and CT stay double).
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "dg_kernels.hpp"
@@ -1588,6 +1589,22 @@ static Box face_box(int D, const Ext& ce, int ax, int along_lo, int along_hi_inc
     return make_box(D, lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]);
 }
 
+// Faces per walker of the strided-axis sweeps.  A walker of c faces rebuilds
+// one cell more than it has faces, which costs about 1/c of half a face's
+// work, and the launch ends with about half a round of resident walkers (two
+// waves per SIMD in FP64, four in FP32), which costs half of c faces' time.
+// With F faces and R resident walkers the sum F/R (1 + 1/2c) + c/2 is least
+// near c = sqrt(F/R); measured, the half round costs a quarter of that, and
+// c = sqrt(2 F/R) lies within 10% of the best of 1..33 at every size tried
+// (64^3 to 240 x 200 x 261, 128^2 to 2048^2, both forms; 33 at 512^3).  With
+// at least 16 faces each, as before, small grids had fewer walkers than the
+// chip holds: x sweeps of 128^2 in FP64 102 -> 16 us, 771 x 530 123 -> 55 us,
+// 64 x 32 x 32 88 -> 18 us, 2048^2 mixed 174 -> 155 us.
+static long march_chunk(long faces, bool fp64) {
+    const double resident = fp64 ? 131072.0 : 262144.0;
+    return std::max(1L, (long)(std::sqrt(2.0 * (double)faces / resident) + 0.5));
+}
+
 // One sweep launch for axis AX over the face box b.
 template <int D, bool MHD, class R, bool FINAL, int AX>
 static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, hipStream_t s) {
@@ -1613,17 +1630,10 @@ static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, 
         a.chunk = 63;
         hipLaunchKernelGGL((k_sweep_wave<D, MHD, R, AX, FINAL>), dim3(blocks(waves * 64)), dim3(256), 0, s, a);
     } else {
-        // Walkers of at least 16 faces (one extra cell rebuild per walker),
-        // ~2^22 of them where the grid allows: with 2 resident waves per SIMD
-        // that is ~32 rounds of waves, so the last, partial round costs
-        // little.  (A walker per whole line, 4161 waves at 512^3, ran as two
-        // full rounds and a third of 65 waves.)
-        const long want = 1L << 22;
-        long nch = (want + ntrans - 1) / ntrans;
-        long chunk = c.march_chunk > 0 ? c.march_chunk : (len + nch - 1) / nch;
-        if (c.march_chunk <= 0 && chunk < 16) chunk = 16;
+        const long chunk0 = march_chunk(len * ntrans, sizeof(R) == 8);
+        long chunk = c.march_chunk > 0 ? c.march_chunk : chunk0;
         if (chunk > len) chunk = len;
-        nch = (len + chunk - 1) / chunk;
+        const long nch = (len + chunk - 1) / chunk;
         a.chunk = (int)chunk;
         if constexpr (!march_window<R>()) {
             if (c.march_window) {
