@@ -1193,15 +1193,21 @@ KB __attribute__((amdgpu_waves_per_eu(emf_tiled_waves<FT>()))) __global__ void k
     }
 }
 
-// i-planes per workgroup of the tiled EMF (one extra plane is read per run)
-constexpr int EMF_IPLANES = 32;
+// i-planes per workgroup of the tiled EMF (one extra plane is read per run):
+// at most 32, fewer where the planes of a grid would make less than four
+// workgroups per CU (planes follow each other at about 1.4 us each: EMF of
+// 64 x 32 x 32 cells 47 us with 32, 9 us with 2).
+constexpr long EMF_IPLANES = 32, EMF_IPLANES_LEAST = 2, EMF_WORKGROUPS = 1024;
 static void emf3_tiled(const FSoa& FX, const FSoa& FY, const FSoa& FZ, const ERef& ref, const Ext& ce, const Ext& fe, const Box& eb,
                        int upwind, ET* Ex, ET* Ey, ET* Ez, hipStream_t s) {
     using T = EmfTile;
     const long nkt = (eb.hi[2] - eb.lo[2] + T::TK - 1) / T::TK, njt = ((eb.hi[1] - eb.lo[1] + T::TJ - 1) / T::TJ + 3) / 4 * 4;  // runs of 4
-    const long nic = (eb.hi[0] - eb.lo[0] + EMF_IPLANES - 1) / EMF_IPLANES;
-    if (nkt <= 0 || njt <= 0 || nic <= 0) return;
-    hipLaunchKernelGGL(k_emf3_tiled, dim3((unsigned)(nkt * njt * nic)), dim3(256), 0, s, FX, FY, FZ, ref, ce, fe, eb, upwind, EMF_IPLANES,
+    const long ni = eb.hi[0] - eb.lo[0];
+    if (nkt <= 0 || njt <= 0 || ni <= 0) return;
+    const long runs = std::max((ni + EMF_IPLANES - 1) / EMF_IPLANES,
+                               std::min((EMF_WORKGROUPS + nkt * njt - 1) / (nkt * njt), (ni + EMF_IPLANES_LEAST - 1) / EMF_IPLANES_LEAST));
+    const long planes = (ni + runs - 1) / runs, nic = (ni + planes - 1) / planes;
+    hipLaunchKernelGGL(k_emf3_tiled, dim3((unsigned)(nkt * njt * nic)), dim3(256), 0, s, FX, FY, FZ, ref, ce, fe, eb, upwind, (int)planes,
                        Ex, Ey, Ez);
 }
 
