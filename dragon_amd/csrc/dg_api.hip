@@ -399,6 +399,34 @@ static void apply_one(dg_grid* g, const dg_bc& b) {
     }
 }
 
+// The implicit Outflow `imp` and then the list in one launch; false (nothing
+// done) where its passes do not fit one (launch_bc_list).
+static bool apply_list(dg_grid* g, const dg_bc& imp) {
+    const int D = g->d.dim;
+    const bool faces = g->d.mhd && D >= 2;
+    BCListArgs a{};
+    a.W = soa(g->W, g->ce.size);
+    for (int q = 0; q < 3; q++) a.B[q] = faces ? g->B + q * g->fe.size : nullptr;
+    a.ce = g->ce; a.fe = g->fe;
+    a.dim = D; a.nf = g->d.mhd ? 8 : 5;
+    auto add = [&](const dg_bc& b) {
+        if (b.kind == DG_BC_IGNORE) return true;
+        for (int ax = 0; ax < D; ax++)
+            for (int side = 0; side < 2; side++) {
+                if (!(b.faces >> (2 * ax + side) & 1)) continue;
+                if (!b.corners || a.npass == 6) return false;
+                BCPass& p = a.p[a.npass++];
+                p.axis = ax; p.side = side; p.kind = b.kind; p.gated = b.gated;
+                for (int q = 0; q < 8; q++) p.st[q] = b.state[q];
+            }
+        return true;
+    };
+    if (!add(imp)) return false;
+    for (auto& b : g->bcs)
+        if (!add(b)) return false;
+    return launch_bc_list(a, g->s);
+}
+
 // One element applied alone, without the list's implicit Outflow: the step
 // by which a caller interleaves device elements with elements it evaluates
 // itself on the host (user GhostFill subclasses).
@@ -432,8 +460,10 @@ int dg_apply_boundary(dg_grid* g) {
     dg_bc imp{};
     imp.kind = DG_BC_OUTFLOW; imp.faces = uncovered; imp.corners = 1; imp.gated = 0;
     tm_record(g, -1);
-    apply_one(g, imp);
-    for (auto& b : g->bcs) apply_one(g, b);
+    if (!apply_list(g, imp)) {
+        apply_one(g, imp);
+        for (auto& b : g->bcs) apply_one(g, b);
+    }
     tm_record(g, K_BC);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(g, DG_ERR_HIP, hipGetErrorString(e));

@@ -284,6 +284,181 @@ KB __global__ void k_bc_faces_periodic_g(BCArgs a) {
     else { fget(a.B, at(g - 1), v); fset(a.B, at(n - 1 + g), v); }
 }
 
+// The whole list in one launch, one thread per ghost cell and field or per
+// boundary face and component.  A thread walks the passes from the last to the
+// first; a pass that would have written its point moves the point to where
+// that pass read it (along its axis), and the signs, the inflow gate and the
+// extrapolation it meets are applied to the value found at the end.  No pass
+// writes a point that the walk ends at: each face has at most one pass, a
+// periodic axis no other, and the passes read interior points along their axis
+// (axes of at least ng + 2 cells; launch_bc_list).  The passes as launches of
+// their own, with their ghost loops, cost 8 us each at any size (a chain of
+// dependent loads and stores per thread, and the gap to the next launch):
+// boundary of 128^2 2D MHD 33 -> 9 us, 64 x 32 x 32 3D MHD 74 -> 12 us,
+// 771 x 530 with outflow 59 -> 10 us.
+struct BCShell {  // the points of the launch: [-wl, 0) and [n, n + wh) along an axis, earlier axes inside, later ones whole
+    int dim, n[3], wl, wh;
+    // extent along d of the slabs of axis ax
+    __host__ __device__ __forceinline__ unsigned width(int d, int ax) const {
+        return d >= dim ? 1u : d == ax ? (unsigned)(wl + wh) : d < ax ? (unsigned)n[d] : (unsigned)(n[d] + wl + wh);
+    }
+    __host__ __device__ __forceinline__ unsigned slab(int ax) const { return ax >= dim ? 0u : width(0, ax) * width(1, ax) * width(2, ax); }
+    __host__ __device__ unsigned count() const { return slab(0) + slab(1) + slab(2); }
+    __device__ __forceinline__ void point(unsigned t, int& i, int& j, int& k) const {
+        int ax = 0;
+        const unsigned s0 = slab(0), s1 = slab(1);
+        if (t >= s0) { t -= s0; ax = 1; if (t >= s1) { t -= s1; ax = 2; } }
+        auto coord = [&](int d) {
+            const unsigned w = width(d, ax);
+            const int r = (int)(t % w);
+            t /= w;
+            return d >= dim ? 0 : d == ax ? (r < wl ? r - wl : n[d] + r - wl) : d < ax ? r : r - wl;
+        };
+        k = coord(2);
+        j = coord(1);
+        i = coord(0);
+    }
+};
+__host__ __device__ inline BCShell cell_shell(const Ext& ce, int dim) { return BCShell{dim, {ce.n[0], ce.n[1], ce.n[2]}, ce.g, ce.g}; }
+// Faces 0 .. n of an axis of n cells: face n is written by most kinds and
+// face 0 by a fixed normal component, so both belong to the shell; indices are
+// shifted by one (point() counts from face 1).
+__host__ __device__ inline BCShell face_shell(const Ext& ce, int dim) {
+    return BCShell{dim, {ce.n[0] - 1, ce.n[1] - 1, ce.n[2] - 1}, ce.g + 1, ce.g + 1};
+}
+// Fields [f0, f1) of the t-th ghost cell.
+__device__ __forceinline__ void bc_list_cell(const BCListArgs& a, const Ext& ce, unsigned t, int f0, int f1) {
+    int i, j, k;
+    cell_shell(ce, a.dim).point(t, i, j, k);
+    const long dst = ce.at(i, j, k);
+    unsigned neg = 0, in_lo = 0, in_hi = 0;  // per field: sign change, inflow through a low / high face dropped
+    bool hit = false;
+    int fixed = -1;  // the pass whose state the cell takes
+    for (int q = a.npass - 1; q >= 0 && fixed < 0; q--) {
+        const BCPass& p = a.p[q];
+        const int ax = p.axis, n = ax == 0 ? ce.n[0] : ax == 1 ? ce.n[1] : ce.n[2], x = ax == 0 ? i : ax == 1 ? j : k;
+        if (p.side == 0 ? x >= 0 : x < n) continue;
+        hit = true;
+        int y = x;
+        if (p.kind == 0) {
+            y = p.side == 0 ? 0 : n - 1;
+            if (p.gated) (p.side == 0 ? in_lo : in_hi) |= 1u << (F_VX + ax);
+        } else if (p.kind == 1) {
+            y = p.side == 0 ? x + n : x - n;
+        } else if (p.kind == 2) {
+            y = p.side == 0 ? -1 - x : 2 * n - 1 - x;
+            neg ^= (1u << (F_VX + ax)) | (7u << F_BX & ~(1u << (F_BX + ax)));
+        } else {
+            fixed = q;
+        }
+        if (ax == 0) i = y; else if (ax == 1) j = y; else k = y;
+    }
+    if (!hit) return;
+    const long src = ce.at(i, j, k);
+    auto finish = [&](int f, double v) {
+        if (neg >> f & 1) v *= -1;
+        if ((in_lo >> f & 1 && v > 0) || (in_hi >> f & 1 && v < 0)) v = 0;
+        a.W(f, dst) = v;
+    };
+    if (f1 - f0 == 1) {
+        finish(f0, fixed >= 0 ? a.p[fixed].st[f0] : a.W(f0, src));
+        return;
+    }
+    double v[8];  // read before any is written, so that the reads overlap
+#pragma unroll
+    for (int f = 0; f < 8; f++)
+        if (f < f1) v[f] = fixed >= 0 ? a.p[fixed].st[f] : a.W(f, src);
+#pragma unroll
+    for (int f = 0; f < 8; f++)
+        if (f < f1) finish(f, v[f]);
+}
+__device__ __forceinline__ void bc_list_face(const BCListArgs& a, const Ext& ce, const Ext& fe, unsigned t, int c) {
+    int i, j, k;
+    face_shell(ce, a.dim).point(t, i, j, k);
+    i++;
+    if (a.dim >= 2) j++;
+    if (a.dim >= 3) k++;
+    double* const B = c == 0 ? a.B[0] : c == 1 ? a.B[1] : a.B[2];
+    const long dst = fe.at(i, j, k);
+    const int ng = ce.g;
+    double v = 0, sgn = 1;
+    int ext = 0, exg = 0;  // extrapolation of the normal component: side + 1, faces beyond the last one kept
+    bool hit = false, fixed = false;
+    for (int q = a.npass - 1; q >= 0 && !fixed; q--) {
+        const BCPass& p = a.p[q];
+        const int ax = p.axis, n = ax == 0 ? ce.n[0] : ax == 1 ? ce.n[1] : ce.n[2], x = ax == 0 ? i : ax == 1 ? j : k;
+        const bool normal = c == ax;
+        int y = x;
+        if (p.side == 0) {
+            if (x > 0 || (x == 0 && !(p.kind == 3 && normal))) continue;
+            if (p.kind == 0) {
+                y = 0;
+                if (normal) { ext = 1; exg = -x; }
+            } else if (p.kind == 1) {
+                y = x + n;
+            } else if (p.kind == 2) {
+                y = normal ? -x : -x - 1;
+                if (!normal) sgn = -sgn;
+            }
+        } else {
+            if (x < n || (p.kind == 0 && normal && x == n) || ((p.kind == 1 || p.kind == 3) && x == n + ng)) continue;
+            if (p.kind == 0) {
+                y = normal ? n : n - 1;
+                if (normal) { ext = 2; exg = x - n; }
+            } else if (p.kind == 1) {
+                y = x - n;
+            } else if (p.kind == 2) {
+                y = x == n ? n - 1 : normal ? 2 * n - x : 2 * n - x - 1;
+                if (x == n || !normal) sgn = -sgn;
+            }
+        }
+        hit = true;
+        if (p.kind == 3) {
+            v = p.st[F_BX + c];
+            fixed = true;
+            ext = 0;  // the extrapolation of equal values
+        }
+        if (ax == 0) i = y; else if (ax == 1) j = y; else k = y;
+    }
+    if (!hit) return;
+    if (!fixed) {
+        const long m = fe.at(i, j, k), s = c == 0 ? fe.s[0] : c == 1 ? fe.s[1] : fe.s[2];
+        v = ld32(B, m);
+        if (ext) {
+            double u = ld32(B, ext == 1 ? m + s : m - s);
+            for (int g = 0; g < exg; g++) {
+                const double w = 2 * v - u;
+                u = v;
+                v = w;
+            }
+        }
+    }
+    if (sgn < 0) v *= -1;
+    B[dst] = v;
+}
+// WHOLE: a thread per point instead of per point and field.  The point's
+// index costs more than a field's copy, so large shells take it (boundary of
+// 384^3 3D MHD 244 us against 341, 64^3 (81 thousand ghost cells) 16 against
+// 19); small ones need the threads (2048^2, 49 thousand: 11 us against 14).
+template <bool WHOLE>
+__device__ __forceinline__ void bc_list_body(const BCListArgs& a, const Ext& ce, const Ext& fe, unsigned t) {
+    if (WHOLE) {
+        if (t < a.ncell) bc_list_cell(a, ce, t, 0, a.nf);
+        else if (t - a.ncell < a.nface)
+            for (int c = 0; c < 3; c++) bc_list_face(a, ce, fe, t - a.ncell, c);
+        return;
+    }
+    const unsigned cells = a.ncell * (unsigned)a.nf;
+    if (t < cells) {
+        const int f = (int)(t / a.ncell);
+        bc_list_cell(a, ce, t % a.ncell, f, f + 1);
+    } else if (t - cells < 3 * a.nface) {
+        bc_list_face(a, ce, fe, (t - cells) % a.nface, (int)((t - cells) / a.nface));
+    }
+}
+template <bool WHOLE>
+KB __global__ void k_bc_list(BCListArgs a) { bc_list_body<WHOLE>(a, a.ce, a.fe, (unsigned)tid()); }
+
 // ==================================================================== CFL
 // Max signal speed over cells [-1, n+1)^D (CFL.cpp:113-162); wave64
 // shuffles then one atomicMax per block on the (non-negative) FP64 bits.
@@ -1536,6 +1711,37 @@ void launch_bc(const BCArgs& a, bool faces, hipStream_t s) {
     else if (contiguous)
         hipLaunchKernelGGL(k_bc_cells_g, dim3(blocks(n * (a.kind == 1 ? 2 : 1) * a.ce.g)), dim3(256), 0, s, a);
     else hipLaunchKernelGGL(k_bc_cells, dim3(blocks(n)), dim3(256), 0, s, a);
+}
+
+constexpr unsigned BC_WHOLE = 65536;  // ghost cells from which a thread copies every field of one
+// False where the list does not fit k_bc_list: an axis with a pass and fewer
+// than ng + 2 cells, two passes on one face, a periodic axis with another
+// pass, or more threads than 32 bits count.
+bool launch_bc_list(BCListArgs& a, hipStream_t s) {
+    if (a.npass == 0) return true;
+    int on[3] = {0, 0, 0}, periodic[3] = {0, 0, 0};
+    for (int q = 0; q < a.npass; q++) {
+        const BCPass& p = a.p[q];
+        if (a.ce.n[p.axis] < a.ce.g + 2 || (on[p.axis] >> p.side & 1)) return false;
+        on[p.axis] |= 1 << p.side;
+        periodic[p.axis] += p.kind == 1;
+    }
+    for (int d = 0; d < 3; d++)
+        if (periodic[d] == 1) return false;
+    for (int d = 0; d < a.dim; d++)
+        if (a.ce.n[d] < 2) return false;
+    const bool faces = a.B[0] != nullptr;
+    double cells = 0, fcs = 0;  // upper bounds of the counts
+    for (int d = 0; d < a.dim; d++) {
+        cells += (double)a.ce.size / (a.ce.n[d] + 2 * a.ce.g) * 2 * a.ce.g;
+        fcs += (double)a.fe.size / (a.fe.n[d] + 2 * a.fe.g) * 2 * (a.fe.g + 1);
+    }
+    if (cells * a.nf + fcs * 3 > 2e9) return false;
+    a.ncell = cell_shell(a.ce, a.dim).count();
+    a.nface = faces ? face_shell(a.ce, a.dim).count() : 0;
+    if (a.ncell >= BC_WHOLE) hipLaunchKernelGGL(k_bc_list<true>, dim3(blocks((long)a.ncell + a.nface)), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_bc_list<false>, dim3(blocks((long)a.ncell * a.nf + 3L * a.nface)), dim3(256), 0, s, a);
+    return true;
 }
 
 void launch_fill_u64(unsigned long long* p, unsigned long long v, int n, hipStream_t s) {

@@ -57,6 +57,20 @@ struct BCArgs {
     double st[8];
     int lo[2], hi[2];                           // transverse ranges
 };
+// A whole boundary list as one launch (k_bc_list): its passes in the list's
+// order, at most one per face, every one over the full transverse range.
+struct BCPass {
+    int axis, side, kind, gated;  // side: 0 negative, 1 positive; kind as dg_bc
+    double st[8];
+};
+struct BCListArgs {
+    Soa W;
+    double* B[3];
+    Ext ce, fe;
+    int dim, nf, npass;
+    unsigned ncell, nface;  // ghost cells / boundary faces the launch covers
+    BCPass p[6];
+};
 // Batched 2D MHD patches (CTU + CT).  Every stage of the step is one launch
 // over all patches: a block table per work kind maps each workgroup to a
 // patch and the first work item it covers.  Pools hold every patch back to
@@ -131,6 +145,7 @@ struct BatchArgs {
     void launch_step(const StepCtx& c, hipStream_t s);                                                          \
     void launch_split_axis(const StepCtx& c, int ax, Soa in, Soa out, hipStream_t s);  /* one split sweep (hydro) */ \
     void launch_bc(const BCArgs& a, bool faces, hipStream_t s);                                                 \
+    bool launch_bc_list(BCListArgs& a, hipStream_t s);                                                          \
     void launch_cfl(const StepCtx& c, unsigned long long* out, hipStream_t s);                                  \
     void launch_cfl_tail(const StepCtx& c, long nparts, unsigned long long* out, hipStream_t s);                \
     void launch_init_B(int dim, Soa W, double* B, Ext ce, Ext fe, hipStream_t s);                               \
