@@ -125,6 +125,20 @@ __device__ __forceinline__ void cross(double ux, double uy, double uz, double vx
     wz = ux * vy - uy * vx;
 }
 
+// Step sizes: wave-uniform loads of words that no launch of the step writes.
+typedef const __attribute__((address_space(4))) StepDts* DtsPtr;
+__device__ __forceinline__ double dts(const StepDts* t, int q, bool half = false) {
+    DtsPtr c = (DtsPtr)t;
+    return half ? c->half[q] : c->full[q];
+}
+// The sweeps check this first; the short kernels once their loads are issued,
+// before they report or write the next state, and the EMF and the half-step
+// faces, which write scratch only, not at all: a wavefront that waits for the
+// word before its first load costs Faraday 3%.
+__device__ __forceinline__ bool stopped(const StepDts* t) { return ((DtsPtr)t)->stop != 0; }
+// A run of steps is over: the step before this launch failed, or no time is left.
+__device__ __forceinline__ bool run_over(const StepCtl* c) { return c->t.stop || c->err != ~0ull || !(c->left_next > c->tol); }
+
 // ===================================================================== BC
 // One thread per transverse index of a face; it runs the reference's ghost
 // loop (g = 1..ng) in order, since face-B extrapolation reads the ghost it
@@ -187,13 +201,17 @@ __device__ __forceinline__ void bc_cells_body(const BCArgs& a, long t) {
         else bc_cell(a, t0, t1, g, a.side);
     }
 }
-KB __global__ void k_bc_cells(BCArgs a) { bc_cells_body(a, tid()); }
+KB __global__ void k_bc_cells(BCArgs a) {
+    if (a.ctl && run_over(a.ctl)) return;
+    bc_cells_body(a, tid());
+}
 // The same with one thread per ghost cell, for the contiguous axis: the
 // cells a pass writes are distinct and, when the axis holds at least ng
 // cells, every cell it reads is interior, so the g loop has no order to
 // keep.  Neighbouring lanes then write neighbouring ghost cells of a line
 // instead of one cell per line each.
 KB __global__ void k_bc_cells_g(BCArgs a) {
+    if (a.ctl && run_over(a.ctl)) return;
     const int ng = a.ce.g, per = a.kind == 1 ? 2 * ng : ng;
     const int n1 = a.hi[0] - a.lo[0], n2 = a.hi[1] - a.lo[1];
     long t = tid();
@@ -266,10 +284,14 @@ __device__ __forceinline__ void bc_faces_body(const BCArgs& a, long t) {
         }
     }
 }
-KB __global__ void k_bc_faces(BCArgs a) { bc_faces_body(a, tid()); }
+KB __global__ void k_bc_faces(BCArgs a) {
+    if (a.ctl && run_over(a.ctl)) return;
+    bc_faces_body(a, tid());
+}
 // Periodic face pass on the contiguous axis, one thread per ghost face:
 // with at least ng cells along the axis every face it reads is interior.
 KB __global__ void k_bc_faces_periodic_g(BCArgs a) {
+    if (a.ctl && run_over(a.ctl)) return;
     const int ng = a.fe.g, per = 2 * ng;
     const int n1 = a.hi[0] - a.lo[0], n2 = a.hi[1] - a.lo[1];
     long t = tid();
@@ -457,7 +479,10 @@ __device__ __forceinline__ void bc_list_body(const BCListArgs& a, const Ext& ce,
     }
 }
 template <bool WHOLE>
-KB __global__ void k_bc_list(BCListArgs a) { bc_list_body<WHOLE>(a, a.ce, a.fe, (unsigned)tid()); }
+KB __global__ void k_bc_list(BCListArgs a) {
+    if (a.ctl && run_over(a.ctl)) return;
+    bc_list_body<WHOLE>(a, a.ce, a.fe, (unsigned)tid());
+}
 
 // ==================================================================== CFL
 // Max signal speed over cells [-1, n+1)^D (CFL.cpp:113-162); wave64
@@ -505,11 +530,78 @@ __device__ __forceinline__ void block_max_store(double m, double* part) {
         part[blockIdx.x] = b;
     }
 }
+// Begins the next step of a run: dt = min(time left, cfl) from the gathered
+// maximum (D: dimension, 0: no CFL), and the words of the step cleared.  One
+// thread, once every workgroup has added its maximum.
+__device__ __forceinline__ void ctl_advance(StepCtl* c, int D, double coeff, double dx, double dy, double dz) {
+    const double left = c->left_next;
+    double t1 = left;
+    if (D) {
+        const double m = __longlong_as_double((long long)__hip_atomic_load(&c->vmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (!(m > 0)) {
+            c->why = CTL_NO_SPEED;
+            c->t.stop = 1;
+            return;
+        }
+        const double t = D == 1 ? coeff * dx / m : coeff / m;
+        t1 = t < left ? t : left;
+    }
+    const double q[3] = {t1 / dx, t1 / dy, t1 / dz};
+    for (int k = 0; k < 3; k++) { c->t.full[k] = q[k]; c->t.half[k] = 0.5 * q[k]; }
+    c->dt = t1;
+    c->left = left;
+    c->left_next = left - t1;
+    c->ring[c->count & (CTL_RING - 1)] = t1;
+    c->count += 1;
+    c->err = ~0ull;
+    c->vmax = 0ull;
+    c->ticket = 0;
+}
+__global__ void k_ctl_set(StepCtl* c, double dt, double dx, double dy, double dz) {
+    c->t.stop = 0;
+    c->left_next = dt;
+    c->count = 0;
+    ctl_advance(c, 0, 0, dx, dy, dz);
+}
+__global__ void k_ctl_begin(StepCtl* c, double left, double tol) {
+    c->t.stop = 0;
+    c->left = c->left_next = left;
+    c->tol = tol;
+    c->err = ~0ull;
+    c->vmax = 0ull;
+    c->ticket = 0;
+    c->count = c->why = 0;
+}
+__global__ void k_ctl_next(StepCtl* c, double dx, double dy, double dz) {
+    if (run_over(c)) c->t.stop = 1;
+    else ctl_advance(c, 0, 0, dx, dy, dz);
+}
+// The end of a CFL pass: the workgroup's maximum b (thread 0) into *out, or in
+// a run into the run's word, whose last workgroup begins the step.
+__device__ __forceinline__ void cfl_finish(double b, unsigned long long* out, StepCtl* run, int D, double coeff, double dx, double dy, double dz) {
+    if (!run) {
+        if (b > 0) atomicMax(out, (unsigned long long)__double_as_longlong(b));
+        return;
+    }
+    // The maximum has reached memory when its old value is back; only then is
+    // the workgroup counted.  (A fence would also write back the XCD's L2, in
+    // each workgroup: 2048^2 2D MHD 80 us more a step.)
+    const unsigned long long was = b > 0 ? atomicMax(&run->vmax, (unsigned long long)__double_as_longlong(b)) : 0ull;
+    asm volatile("s_waitcnt vmcnt(0)" ::"v"(was) : "memory");
+    if (atomicAdd(&run->ticket, 1u) == gridDim.x - 1) ctl_advance(run, D, coeff, dx, dy, dz);
+}
+// True (all threads) where a run is over; its first workgroup marks it.
+__device__ __forceinline__ bool cfl_run_over(StepCtl* run) {
+    if (!run || !run_over(run)) return false;
+    if (blockIdx.x == 0 && threadIdx.x == 0) run->t.stop = 1;
+    return true;
+}
 // CFL of the committed state from the maxima the apply pass left over the
 // interior plus a scan of the ghost layer 1 (the shell of [-1, n+1)^D).
 template <int D, bool MHD>
 KB __global__ void k_cfl_tail(Soa W, Ext ce, const double* part, long nparts, Phys ph, int mode, double dx, double dy, double dz,
-                              unsigned long long* out) {
+                              unsigned long long* out, StepCtl* run, double coeff) {
+    if (cfl_run_over(run)) return;
     const long n0 = ce.n[0], n1 = ce.n[1], n2 = ce.n[2];
     // shell slabs: x faces (i = -1, n0) over the full transverse range, then y, then z faces inside
     const long sx = D == 3 ? (n1 + 2) * (n2 + 2) : (D == 2 ? n1 + 2 : 1);
@@ -549,11 +641,13 @@ KB __global__ void k_cfl_tail(Soa W, Ext ce, const double* part, long nparts, Ph
     if (threadIdx.x == 0) {
         double b = wmax[0];
         for (int q = 1; q < (int)(blockDim.x >> 6); q++) b = dmax(b, wmax[q]);
-        if (b > 0) atomicMax(out, (unsigned long long)__double_as_longlong(b));
+        cfl_finish(b, out, run, D, coeff, dx, dy, dz);
     }
 }
 template <int D, bool MHD>
-KB __global__ void k_cfl(Soa W, Ext ce, Box box, Phys ph, int mode, double dx, double dy, double dz, unsigned long long* out) {
+KB __global__ void k_cfl(Soa W, Ext ce, Box box, Phys ph, int mode, double dx, double dy, double dz, unsigned long long* out,
+                         StepCtl* run, double coeff) {
+    if (cfl_run_over(run)) return;
     double m = 0;
     int i, j, k;
     const long cnt = box.count(), stride = (long)gridDim.x * blockDim.x;
@@ -567,7 +661,7 @@ KB __global__ void k_cfl(Soa W, Ext ce, Box box, Phys ph, int mode, double dx, d
     if (threadIdx.x == 0) {
         double b = part[0];
         for (int q = 1; q < (int)(blockDim.x >> 6); q++) b = dmax(b, part[q]);
-        if (b > 0) atomicMax(out, (unsigned long long)__double_as_longlong(b));
+        cfl_finish(b, out, run, D, coeff, dx, dy, dz);
     }
 }
 
@@ -577,7 +671,9 @@ KB __global__ void k_cfl(Soa W, Ext ce, Box box, Phys ph, int mode, double dx, d
 // layer along an axis get the first-order copy.
 template <int D, bool MHD, class R>
 KB __global__ void k_half(Soa W, double* Bx, double* By, double* Bz, Ext ce, Ext fe, Soa HS0, Soa HS1, Soa HS2, Soa HS3,
-                          Soa HS4, Soa HS5, double dt_dx, double dt_dy, double dt_dz, Phys ph) {
+                          Soa HS4, Soa HS5, const StepDts* ts, Phys ph) {
+    if (stopped(ts)) return;
+    const double dt_dx = dts(ts, 0), dt_dy = dts(ts, 1), dt_dz = dts(ts, 2);
     Box box = make_box(D, -ce.g, ce.n[0] + ce.g, -ce.g, ce.n[1] + ce.g, -ce.g, ce.n[2] + ce.g);
     int i, j, k;
     if (!box.point(tid(), i, j, k)) return;
@@ -627,7 +723,9 @@ KB __global__ void k_half(Soa W, double* Bx, double* By, double* Bz, Ext ce, Ext
 // ================================================================= fluxes
 // computeFlux_X/Y/Z (Unsplit.cpp:210-254): F[c] = Riemann(R[c - e], L[c]).
 template <int D, bool MHD, class R, int AX>
-KB __global__ void k_flux(Soa HL, Soa HR, FSoa F, Ext ce, Box box, double dt_d, Phys ph, unsigned long long* err, int stage) {
+KB __global__ void k_flux(Soa HL, Soa HR, FSoa F, Ext ce, Box box, const StepDts* ts, Phys ph, unsigned long long* err, int stage) {
+    if (stopped(ts)) return;
+    const double dt_d = dts(ts, AX);
     int i, j, k;
     if (!box.point(tid(), i, j, k)) return;
     const long m = ce.at(i, j, k);
@@ -659,11 +757,12 @@ struct SweepArgs {
     FSoa Fo;               // output fluxes of this axis
     Ext ce, fe;
     int lo[3], hi[3];      // faces [lo, hi) per dim; face f of axis AX sits between cells f-1 and f
-    double dt_d[3];
+    const StepDts* ts;
     Phys ph;
     unsigned long long* err;
-    int stage, chunk;
+    int stage, chunk, half;  // half: a step of dt / 2
     ET* eref[3];           // MHD predictor sweep along the contiguous axis: the cells' reference EMF cross(B, v) (else unused)
+    __device__ __forceinline__ double dt_d(int q) const { return dts(ts, q, half); }
 };
 // The MHD predictor sweep along the contiguous axis also writes each rebuilt
 // cell's reference EMF, cross(B, v) of the state it holds: its cells cover
@@ -733,7 +832,7 @@ __device__ __forceinline__ void ctu_correct(const SweepArgs& a, long m, long q, 
     auto fd = [&](int ax) { return usub<MHD>(load_u(a.Fp[ax], m, MHD), load_u(a.Fp[ax], m + ce.s[ax], MHD)); };
     if constexpr (!MHD) {  // correctState (hydro 2D): minus the transverse flux difference
         constexpr int T = AX == 0 ? 1 : 0;
-        U<double> t = umul<false>(usub<false>(load_u(a.Fp[T], m + ce.s[T], false), load_u(a.Fp[T], m, false)), 0.5 * a.dt_d[T]);
+        U<double> t = umul<false>(usub<false>(load_u(a.Fp[T], m + ce.s[T], false), load_u(a.Fp[T], m, false)), 0.5 * a.dt_d(T));
         L = prim_c<false>(usub<false>(cons_c<false>(L, ph), t), ph);
         Rr = prim_c<false>(usub<false>(cons_c<false>(Rr, ph), t), ph);
         return;
@@ -742,7 +841,7 @@ __device__ __forceinline__ void ctu_correct(const SweepArgs& a, long m, long q, 
         const long fx = fe.s[0], fy = fe.s[1], fz = fe.s[2];
         const double k8 = ph.k1_8pi;
         const P<double> Wc = load_p<double>(a.W, m, true);
-        const double dt_dx = a.dt_d[0], dt_dy = a.dt_d[1], dt_dz = a.dt_d[2];
+        const double dt_dx = a.dt_d(0), dt_dy = a.dt_d(1), dt_dz = a.dt_d(2);
         const ET *E0x = a.E0[0], *E0y = a.E0[1], *E0z = a.E0[2];
         U<double> corr;
         if (D == 2) {
@@ -814,20 +913,20 @@ __device__ __forceinline__ void cell_states_from(const SweepArgs& a, int i, int 
     long q = 0;
     if (MHD && D >= 2) {
         q = fe.at(i, j, k);
-        bx = (ld32(a.B[0], q + fe.s[0]) - ld32(a.B[0], q)) * a.dt_d[0];
-        by = (ld32(a.B[1], q + fe.s[1]) - ld32(a.B[1], q)) * a.dt_d[1];
-        if (D == 3) bz = (ld32(a.B[2], q + fe.s[2]) - ld32(a.B[2], q)) * a.dt_d[2];
+        bx = (ld32(a.B[0], q + fe.s[0]) - ld32(a.B[0], q)) * a.dt_d(0);
+        by = (ld32(a.B[1], q + fe.s[1]) - ld32(a.B[1], q)) * a.dt_d(1);
+        if (D == 3) bz = (ld32(a.B[2], q + fe.s[2]) - ld32(a.B[2], q)) * a.dt_d(2);
     }
     if (idx[AX] >= -g + 1 && idx[AX] < ce.n[AX] + g - 1) {
         if (AX == 0) {
-            muscl<MHD, R>(wl, L, wc, Rr, wr, R(a.dt_d[0]), R(bx), R(by), R(bz), a.ph);
+            muscl<MHD, R>(wl, L, wc, Rr, wr, R(a.dt_d(0)), R(bx), R(by), R(bz), a.ph);
         } else if (AX == 1) {
             P<R> l, r;
-            muscl<MHD, R>(swapXY(wl), l, swapXY(wc), r, swapXY(wr), R(a.dt_d[1]), R(by), R(bx), R(bz), a.ph);
+            muscl<MHD, R>(swapXY(wl), l, swapXY(wc), r, swapXY(wr), R(a.dt_d(1)), R(by), R(bx), R(bz), a.ph);
             L = swapXY(l); Rr = swapXY(r);
         } else {
             P<R> l, r;
-            muscl<MHD, R>(swapXZ(wl), l, swapXZ(wc), r, swapXZ(wr), R(a.dt_d[2]), R(bz), R(by), R(bx), a.ph);
+            muscl<MHD, R>(swapXZ(wl), l, swapXZ(wc), r, swapXZ(wr), R(a.dt_d(2)), R(bz), R(by), R(bx), a.ph);
             L = swapXZ(l); Rr = swapXZ(r);
         }
     } else {
@@ -869,7 +968,7 @@ __device__ __forceinline__ void face_flux(const SweepArgs& a, P<R> l, P<R> r, lo
     if (AX == 1) { l = swapXY(l); r = swapXY(r); }
     if (AX == 2) { l = swapXZ(l); r = swapXZ(r); }
     int fail = RF_OK;
-    U<R> f = riemann_x<MHD, R>(l, r, R(a.dt_d[AX]), a.ph, &fail);
+    U<R> f = riemann_x<MHD, R>(l, r, R(a.dt_d(AX)), a.ph, &fail);
     if (fail) report(a.err, a.stage, (unsigned long long)m, fail == RF_BAD_INPUT ? E_RIEMANN_INPUT : E_RIEMANN_SOLUTION);
     if (AX == 1) f = swapXY(f);
     if (AX == 2) f = swapXZ(f);
@@ -1017,10 +1116,14 @@ template <int D, int AX, class R, bool FINAL> constexpr int march_min_waves() {
 }
 template <int D, bool MHD, class R, int AX, bool FINAL>
 KS __attribute__((amdgpu_waves_per_eu(march_min_waves<D, AX, R, FINAL>()))) __global__ void k_sweep_march(SweepArgs a) {
+    if (stopped(a.ts)) return;
     sweep_march_body<D, MHD, R, AX, FINAL>(a, tid_xcd());
 }
 template <int D, bool MHD, class R, int AX, bool FINAL>
-KS __global__ void k_sweep_march_window(SweepArgs a) { sweep_march_body<D, MHD, R, AX, FINAL, true>(a, tid()); }
+KS __global__ void k_sweep_march_window(SweepArgs a) {
+    if (stopped(a.ts)) return;
+    sweep_march_body<D, MHD, R, AX, FINAL, true>(a, tid());
+}
 
 template <class R> __device__ __forceinline__ P<R> shfl_up1(const P<R>& w) {
     return P<R>{__shfl_up(w.rho, 1), __shfl_up(w.p, 1), __shfl_up(w.vx, 1), __shfl_up(w.vy, 1),
@@ -1092,6 +1195,7 @@ __device__ __forceinline__ void sweep_stream_body(const SweepArgs& a, int w, int
 template <class R> constexpr int wave_min_waves() { return DG_SWEEP_WAVES == 0 && sizeof(R) == 8 ? 3 : 1; }
 template <int D, bool MHD, class R, int AX, bool FINAL>
 KS __attribute__((amdgpu_waves_per_eu(wave_min_waves<R>()))) __global__ void k_sweep_wave(SweepArgs a) {
+    if (stopped(a.ts)) return;
     // the wavefront index is uniform: keep it in a scalar register
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     sweep_stream_body<D, MHD, R, AX, FINAL>(a, (int)block_xcd() * (int)(blockDim.x >> 6) + w, threadIdx.x & 63);
@@ -1101,7 +1205,9 @@ KS __attribute__((amdgpu_waves_per_eu(wave_min_waves<R>()))) __global__ void k_s
 // correctState (CTU.cpp:264-301): states along SAX corrected by the flux
 // difference of FAX.
 template <int D, class R>
-KB __global__ void k_correct(Soa HL, Soa HR, FSoa F, Ext ce, Box box, int fax, double dt_dL, Phys ph) {
+KB __global__ void k_correct(Soa HL, Soa HR, FSoa F, Ext ce, Box box, int fax, const StepDts* ts, Phys ph) {
+    if (stopped(ts)) return;
+    const double dt_dL = dts(ts, fax, true);
     int i, j, k;
     if (!box.point(tid(), i, j, k)) return;
     const long m = ce.at(i, j, k);
@@ -1114,8 +1220,10 @@ KB __global__ void k_correct(Soa HL, Soa HR, FSoa F, Ext ce, Box box, int fax, d
 // computeCTUFlux_X/Y/Z (CTU.cpp:306-370): a flux between states corrected by
 // the transverse flux T (3D hydro, 12-solve CTU).
 template <class R, int AX>
-KB __global__ void k_ctu_flux(Soa HL, Soa HR, FSoa T, FSoa F, Ext ce, Box box, int tax, double dt_d, double dt_t, Phys ph,
+KB __global__ void k_ctu_flux(Soa HL, Soa HR, FSoa T, FSoa F, Ext ce, Box box, int tax, const StepDts* ts, Phys ph,
                               unsigned long long* err, int stage) {
+    if (stopped(ts)) return;
+    const double dt_d = dts(ts, AX), dt_t = dts(ts, tax) / 3.0;
     int i, j, k;
     if (!box.point(tid(), i, j, k)) return;
     const long m = ce.at(i, j, k), e = ce.s[AX], te = ce.s[tax];
@@ -1391,7 +1499,7 @@ static void emf3_tiled(const FSoa& FX, const FSoa& FY, const FSoa& FZ, const ERe
 template <int D, class BO>
 __device__ __forceinline__ void faraday_body(const ET* Ex, const ET* Ey, const ET* Ez, const double* Bix, const double* Biy,
                                              const double* Biz, BO* Box_, BO* Boy, BO* Boz, const Ext& fe, int gg, double dt_dx,
-                                             double dt_dy, double dt_dz, long m) {
+                                             double dt_dy, double dt_dz, long m, const StepDts* gate = nullptr) {
     if (m >= fe.size) return;
     double bx = ld32(Bix, m), by = ld32(Biy, m), bz = ld32(Biz, m);
     // recover (i,j,k) of m
@@ -1414,15 +1522,17 @@ __device__ __forceinline__ void faraday_body(const ET* Ex, const ET* Ey, const E
         if (ixl && jy && kzl) by -= (ed(Ex, m + fe.s[2]) - ed(Ex, m)) * dt_dz - (ed(Ez, m + fe.s[0]) - ed(Ez, m)) * dt_dx;
         if (ixl && jyl && kz) bz -= (ed(Ey, m + fe.s[0]) - ed(Ey, m)) * dt_dx - (ed(Ex, m + fe.s[1]) - ed(Ex, m)) * dt_dy;
     }
+    if (gate && stopped(gate)) return;
     Box_[m] = BO(bx); Boy[m] = BO(by); Boz[m] = BO(bz);
 }
 // The final update writes FP64 face B; the half-step one (gg = 1) writes the
 // half-step faces in ET.
 template <int D, class BO>
 KB __global__ void k_faraday(const ET* Ex, const ET* Ey, const ET* Ez, const double* Bix, const double* Biy,
-                             const double* Biz, BO* Box_, BO* Boy, BO* Boz, Ext fe, int gg, double dt_dx, double dt_dy,
-                             double dt_dz) {
-    faraday_body<D, BO>(Ex, Ey, Ez, Bix, Biy, Biz, Box_, Boy, Boz, fe, gg, dt_dx, dt_dy, dt_dz, tid_xcd());
+                             const double* Biz, BO* Box_, BO* Boy, BO* Boz, Ext fe, int gg, const StepDts* ts) {
+    const bool h = gg != 0;
+    faraday_body<D, BO>(Ex, Ey, Ez, Bix, Biy, Biz, Box_, Boy, Boz, fe, gg, dts(ts, 0, h), dts(ts, 1, h), dts(ts, 2, h), tid_xcd(),
+                        ts);
 }
 
 // computeBodyField + shouldProtectThermal (B_fields.cpp:70-114, production
@@ -1458,7 +1568,8 @@ __device__ __forceinline__ void cell_B(const T* Bx, const T* By, const T* Bz, co
 template <int D>
 __device__ __forceinline__ void whalf_body(const Soa& W, const FSoa& FX, const FSoa& FY, const FSoa& FZ, const ET* Bhx, const ET* Bhy,
                                            const ET* Bhz, const Ext& ce, const Ext& fe, const Box& box, double hx, double hy, double hz,
-                                           const Phys& ph, ET* Ehx, ET* Ehy, ET* Ehz, unsigned long long* err, long t) {
+                                           const Phys& ph, ET* Ehx, ET* Ehy, ET* Ehz, unsigned long long* err, long t,
+                                           const StepDts* gate = nullptr) {
     int i, j, k;
     if (!box.point(t, i, j, k)) return;
     const long m = ce.at(i, j, k);
@@ -1467,6 +1578,7 @@ __device__ __forceinline__ void whalf_body(const Soa& W, const FSoa& FX, const F
     u = uadd<true>(u, umul<true>(usub<true>(load_u_nb<0>(FX, m), load_u_nb<0>(FX, m + ce.s[0])), hx));
     u = uadd<true>(u, umul<true>(usub<true>(load_u_nb<1>(FY, m), load_u_nb<1>(FY, m + ce.s[1])), hy));
     if (D == 3) u = uadd<true>(u, umul<true>(usub<true>(load_u_nb<2>(FZ, m), load_u_nb<2>(FZ, m + ce.s[2])), hz));
+    if (gate && stopped(gate)) return;
     if (!finite<true>(u)) report(err, ST_WHALF_NAN, (unsigned long long)m, E_NAN);
     w = prim<true>(u, ph);
     double cbx, cby, cbz;
@@ -1479,17 +1591,19 @@ __device__ __forceinline__ void whalf_body(const Soa& W, const FSoa& FX, const F
 }
 template <int D>
 KB __global__ void k_whalf(Soa W, FSoa FX, FSoa FY, FSoa FZ, const ET* Bhx, const ET* Bhy, const ET* Bhz, Ext ce,
-                           Ext fe, Box box, double hx, double hy, double hz, Phys ph, ET* Ehx, ET* Ehy, ET* Ehz,
+                           Ext fe, Box box, const StepDts* ts, Phys ph, ET* Ehx, ET* Ehy, ET* Ehz,
                            unsigned long long* err) {
-    whalf_body<D>(W, FX, FY, FZ, Bhx, Bhy, Bhz, ce, fe, box, hx, hy, hz, ph, Ehx, Ehy, Ehz, err, tid_xcd());
+    whalf_body<D>(W, FX, FY, FZ, Bhx, Bhy, Bhz, ce, fe, box, dts(ts, 0, true), dts(ts, 1, true), dts(ts, 2, true), ph, Ehx, Ehy, Ehz, err,
+                  tid_xcd(), ts);
 }
 
 // ctu_sweep_MHD corrections (CTU.cpp:65-129 3D, 162-202 2D), in place.
 template <int D>
 KB __global__ void k_ctu_mhd(Soa W, const double* Bx, const double* By, const double* Bz, const ET* Bhx, const ET* Bhy,
                              const ET* Bhz, const ET* E0x, const ET* E0y, const ET* E0z, FSoa FX, FSoa FY, FSoa FZ,
-                             Soa XL, Soa XR, Soa YL, Soa YR, Soa ZL, Soa ZR, Ext ce, Ext fe, Box box, double dt_dx, double dt_dy,
-                             double dt_dz, Phys ph) {
+                             Soa XL, Soa XR, Soa YL, Soa YR, Soa ZL, Soa ZR, Ext ce, Ext fe, Box box, const StepDts* ts, Phys ph) {
+    if (stopped(ts)) return;
+    const double dt_dx = dts(ts, 0), dt_dy = dts(ts, 1), dt_dz = dts(ts, 2);
     int i, j, k;
     if (!box.point(tid(), i, j, k)) return;
     const long m = ce.at(i, j, k), q = fe.at(i, j, k);
@@ -1563,7 +1677,7 @@ template <int D, bool MHD>
 __device__ __forceinline__ double apply_body(const Soa& W, const Soa& Wn, const FSoa& FX, const FSoa& FY, const FSoa& FZ, const double* Bnx,
                                              const double* Bny, const double* Bnz, const Ext& ce, const Ext& fe, double dt_dx, double dt_dy,
                                              double dt_dz, const Phys& ph, unsigned long long* err, long m, bool cfl = false, int cfl_mode = 1,
-                                             double cdx = 1, double cdy = 1, double cdz = 1) {
+                                             double cdx = 1, double cdy = 1, double cdz = 1, const StepDts* gate = nullptr) {
     if (m >= ce.size) return 0.0;
     const int nf = MHD ? 8 : 5;
     unsigned r = (unsigned)m;
@@ -1574,6 +1688,7 @@ __device__ __forceinline__ double apply_body(const Soa& W, const Soa& Wn, const 
     i = (int)r - ce.g;
     const bool interior = i >= 0 && i < ce.n[0] && j >= 0 && j < ce.n[1] && k >= 0 && k < ce.n[2];
     if (!interior) {
+        if (gate && stopped(gate)) return 0.0;
         for (int f = 0; f < nf; f++) st_nt(Wn, f, m, W(f, m));
         return 0.0;
     }
@@ -1588,6 +1703,7 @@ __device__ __forceinline__ double apply_body(const Soa& W, const Soa& Wn, const 
         if (D >= 2) u = uadd<false>(u, umul<false>(usub<false>(load_u(FY, m, false), load_u(FY, m + ce.s[1], false)), dt_dy));
         if (D == 3) u = uadd<false>(u, umul<false>(usub<false>(load_u(FZ, m, false), load_u(FZ, m + ce.s[2], false)), dt_dz));
     }
+    if (gate && stopped(gate)) return 0.0;
     if (D >= 2 && !finite<MHD>(u)) report(err, ST_APPLY_NAN, (unsigned long long)m, E_NAN);
     w = prim<MHD>(u, ph);
     if (MHD && D >= 2) {
@@ -1601,18 +1717,20 @@ __device__ __forceinline__ double apply_body(const Soa& W, const Soa& Wn, const 
 }
 template <int D, bool MHD>
 KB __global__ void k_apply(Soa W, Soa Wn, FSoa FX, FSoa FY, FSoa FZ, const double* Bnx, const double* Bny, const double* Bnz, Ext ce,
-                           Ext fe, double dt_dx, double dt_dy, double dt_dz, Phys ph, unsigned long long* err, double* cflpart,
+                           Ext fe, const StepDts* ts, Phys ph, unsigned long long* err, double* cflpart,
                            int cfl_mode, double cdx, double cdy, double cdz) {
-    const double v = apply_body<D, MHD>(W, Wn, FX, FY, FZ, Bnx, Bny, Bnz, ce, fe, dt_dx, dt_dy, dt_dz, ph, err, tid_xcd(), cflpart != nullptr,
-                                        cfl_mode, cdx, cdy, cdz);
-    if (cflpart) block_max_store(v, cflpart);  // uniform branch
+    const double v = apply_body<D, MHD>(W, Wn, FX, FY, FZ, Bnx, Bny, Bnz, ce, fe, dts(ts, 0), dts(ts, 1), dts(ts, 2), ph, err, tid_xcd(),
+                                        cflpart != nullptr, cfl_mode, cdx, cdy, cdz, ts);
+    if (cflpart && !stopped(ts)) block_max_store(v, cflpart);  // uniform branch; a stopped step leaves the committed state's maxima
 }
 
 // 1D Godunov::sweep update (Splitting.cpp:67-95): cells [-g+1, n+g-2] take
 // the flux difference; cell n+g-2 then takes the sweep's trailing zero
 // update (a prim->cons->prim round trip).  Ghosts are committed too.
 template <bool MHD>
-KB __global__ void k_apply1(Soa W, Soa Wn, FSoa F, Ext ce, double dt_dx, Phys ph, unsigned long long* err) {
+KB __global__ void k_apply1(Soa W, Soa Wn, FSoa F, Ext ce, const StepDts* ts, Phys ph, unsigned long long* err) {
+    if (stopped(ts)) return;
+    const double dt_dx = dts(ts, 0);
     const long m = tid();
     if (m >= ce.size) return;
     const int nf = MHD ? 8 : 5, g = ce.g, n = ce.n[0];
@@ -1755,39 +1873,51 @@ void launch_soa_to_aos(Soa soa, int nf, double* a, int stride, long n, hipStream
 }
 
 template <int D, bool MHD>
-static void cfl_t(const StepCtx& c, unsigned long long* out, hipStream_t s) {
+static void cfl_t(const StepCtx& c, unsigned long long* out, StepCtl* run, hipStream_t s) {
     const int n1 = c.ce.g < 1 ? c.ce.g : 1;
     Box b = make_box(D, -n1, c.ce.n[0] + n1, -n1, c.ce.n[1] + n1, -n1, c.ce.n[2] + n1);
     const unsigned nb = std::min(blocks(b.count()), 8192u);
-    hipLaunchKernelGGL((k_cfl<D, MHD>), dim3(nb), dim3(256), 0, s, c.W, c.ce, b, c.ph, c.cfl_mode, c.d[0], c.d[1], c.d[2], out);
+    hipLaunchKernelGGL((k_cfl<D, MHD>), dim3(nb), dim3(256), 0, s, c.W, c.ce, b, c.ph, c.cfl_mode, c.d[0], c.d[1], c.d[2], out,
+                       run, c.cfl_coeff);
 }
 template <int D, bool MHD>
-static void cfl_tail_t(const StepCtx& c, long nparts, unsigned long long* out, hipStream_t s) {
+static void cfl_tail_t(const StepCtx& c, long nparts, unsigned long long* out, StepCtl* run, hipStream_t s) {
     const long work = nparts + (long)c.ce.n[0] * c.ce.n[1] * c.ce.n[2];  // upper bound; the kernel is grid-stride
     const unsigned nb = std::min(blocks(work), 2048u);
     hipLaunchKernelGGL((k_cfl_tail<D, MHD>), dim3(nb), dim3(256), 0, s, c.W, c.ce, c.cflpart, nparts, c.ph, c.cfl_mode, c.d[0], c.d[1],
-                       c.d[2], out);
+                       c.d[2], out, run, c.cfl_coeff);
 }
-void launch_cfl_tail(const StepCtx& c, long nparts, unsigned long long* out, hipStream_t s) {
-    if (c.dim == 2) c.mhd ? cfl_tail_t<2, true>(c, nparts, out, s) : cfl_tail_t<2, false>(c, nparts, out, s);
-    else c.mhd ? cfl_tail_t<3, true>(c, nparts, out, s) : cfl_tail_t<3, false>(c, nparts, out, s);
+void launch_cfl_tail(const StepCtx& c, long nparts, unsigned long long* out, bool run, hipStream_t s) {
+    StepCtl* r = run ? c.ctl : nullptr;
+    if (c.dim == 2) c.mhd ? cfl_tail_t<2, true>(c, nparts, out, r, s) : cfl_tail_t<2, false>(c, nparts, out, r, s);
+    else c.mhd ? cfl_tail_t<3, true>(c, nparts, out, r, s) : cfl_tail_t<3, false>(c, nparts, out, r, s);
 }
-void launch_cfl(const StepCtx& c, unsigned long long* out, hipStream_t s) {
-    if (c.dim == 1) c.mhd ? cfl_t<1, true>(c, out, s) : cfl_t<1, false>(c, out, s);
-    else if (c.dim == 2) c.mhd ? cfl_t<2, true>(c, out, s) : cfl_t<2, false>(c, out, s);
-    else c.mhd ? cfl_t<3, true>(c, out, s) : cfl_t<3, false>(c, out, s);
+void launch_cfl(const StepCtx& c, unsigned long long* out, bool run, hipStream_t s) {
+    StepCtl* r = run ? c.ctl : nullptr;
+    if (c.dim == 1) c.mhd ? cfl_t<1, true>(c, out, r, s) : cfl_t<1, false>(c, out, r, s);
+    else if (c.dim == 2) c.mhd ? cfl_t<2, true>(c, out, r, s) : cfl_t<2, false>(c, out, r, s);
+    else c.mhd ? cfl_t<3, true>(c, out, r, s) : cfl_t<3, false>(c, out, r, s);
+}
+void launch_ctl_set(const StepCtx& c, double dt, hipStream_t s) {
+    hipLaunchKernelGGL(k_ctl_set, dim3(1), dim3(1), 0, s, c.ctl, dt, c.d[0], c.d[1], c.d[2]);
+}
+void launch_ctl_begin(const StepCtx& c, double left, double tol, hipStream_t s) {
+    hipLaunchKernelGGL(k_ctl_begin, dim3(1), dim3(1), 0, s, c.ctl, left, tol);
+}
+void launch_ctl_next(const StepCtx& c, hipStream_t s) {
+    hipLaunchKernelGGL(k_ctl_next, dim3(1), dim3(1), 0, s, c.ctl, c.d[0], c.d[1], c.d[2]);
 }
 
 template <int D, bool MHD, class R, int AX>
-static void flux_t(const StepCtx& c, const Soa& HL, const Soa& HR, const FSoa& F, Box b, double dt_d, int stage, hipStream_t s) {
+static void flux_t(const StepCtx& c, const Soa& HL, const Soa& HR, const FSoa& F, Box b, int stage, hipStream_t s) {
     if (b.count() <= 0) return;
-    hipLaunchKernelGGL((k_flux<D, MHD, R, AX>), dim3(blocks(b.count())), dim3(256), 0, s, HL, HR, F, c.ce, b, dt_d, c.ph, c.err, stage);
+    hipLaunchKernelGGL((k_flux<D, MHD, R, AX>), dim3(blocks(b.count())), dim3(256), 0, s, HL, HR, F, c.ce, b, &c.ctl->t, c.ph, c.err, stage);
 }
 template <int D, bool MHD, class R>
-static void flux_ax(const StepCtx& c, int ax, const Soa& HL, const Soa& HR, const FSoa& F, Box b, double dt_d, int stage, hipStream_t s) {
-    if (ax == 0) flux_t<D, MHD, R, 0>(c, HL, HR, F, b, dt_d, stage, s);
-    else if (ax == 1) { if constexpr (D >= 2) flux_t<D, MHD, R, 1>(c, HL, HR, F, b, dt_d, stage, s); }
-    else { if constexpr (D >= 3) flux_t<D, MHD, R, 2>(c, HL, HR, F, b, dt_d, stage, s); }
+static void flux_ax(const StepCtx& c, int ax, const Soa& HL, const Soa& HR, const FSoa& F, Box b, int stage, hipStream_t s) {
+    if (ax == 0) flux_t<D, MHD, R, 0>(c, HL, HR, F, b, stage, s);
+    else if (ax == 1) { if constexpr (D >= 2) flux_t<D, MHD, R, 1>(c, HL, HR, F, b, stage, s); }
+    else { if constexpr (D >= 3) flux_t<D, MHD, R, 2>(c, HL, HR, F, b, stage, s); }
 }
 
 // Face-range boxes of computeFlux_* for axis `ax`: [lo, hi] inclusive along
@@ -1825,9 +1955,9 @@ static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, 
     for (int q = 0; q < 3; q++) {
         a.B[q] = c.B[q]; a.Bh[q] = et(c.Bh[q]); a.E0[q] = et(c.E0[q]); a.Fp[q] = fs(c.Fp[q]);
         a.lo[q] = b.lo[q]; a.hi[q] = b.hi[q];
-        a.dt_d[q] = c.dt / c.d[q];
     }
     a.Fo = out; a.ce = c.ce; a.fe = c.fe; a.ph = c.ph; a.err = c.err; a.stage = stage;
+    a.ts = &c.ctl->t; a.half = c.half;
     if constexpr (eref_in_sweep<D, MHD, FINAL, AX>())
         if (stage == ST_PRED_X + AX)  // the CTU predictor (not the flux sweep of a step without CTU)
             for (int q = 0; q < 3; q++) a.eref[q] = et(c.Eh[q]);  // read by the predictor EMF before whalf overwrites it
@@ -1869,7 +1999,6 @@ static void sweep(const StepCtx& c, int ax, const Box& b, const FSoa& out, int s
 template <int D, bool MHD, class R>
 static void step_fused(const StepCtx& c, hipStream_t s) {
     const Ext& ce = c.ce;
-    const double dt_d[3] = {c.dt / c.d[0], c.dt / c.d[1], c.dt / c.d[2]};
     if (c.ctu) {
         for (int ax = 0; ax < D; ax++) {
             Box b = MHD ? face_box(D, ce, ax, -1, 1, -2, 2) : face_box(D, ce, ax, 0, 0, -1, 1);
@@ -1892,11 +2021,11 @@ static void step_fused(const StepCtx& c, hipStream_t s) {
             }
             mark(c, K_EMF_PRED);
             hipLaunchKernelGGL((k_faraday<D, ET>), dim3(blocks(c.fe.size)), dim3(256), 0, s, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]), c.B[0], c.B[1],
-                               c.B[2], et(c.Bh[0]), et(c.Bh[1]), et(c.Bh[2]), c.fe, 1, 0.5 * dt_d[0], 0.5 * dt_d[1], 0.5 * dt_d[2]);
+                               c.B[2], et(c.Bh[0]), et(c.Bh[1]), et(c.Bh[2]), c.fe, 1, &c.ctl->t);
             mark(c, K_FARADAY_HALF);
             Box cb = make_box(D, -1, ce.n[0] + 1, -1, ce.n[1] + 1, -1, ce.n[2] + 1);
             hipLaunchKernelGGL((k_whalf<D>), dim3(blocks(cb.count())), dim3(256), 0, s, c.W, fs(c.Fp[0]), fs(c.Fp[1]), fs(c.Fp[2]), et(c.Bh[0]),
-                               et(c.Bh[1]), et(c.Bh[2]), ce, c.fe, cb, 0.5 * dt_d[0], 0.5 * dt_d[1], 0.5 * dt_d[2], c.ph, et(c.Eh[0]), et(c.Eh[1]),
+                               et(c.Bh[1]), et(c.Bh[2]), ce, c.fe, cb, &c.ctl->t, c.ph, et(c.Eh[0]), et(c.Eh[1]),
                                et(c.Eh[2]), c.err);
             mark(c, K_WHALF);
         }
@@ -1917,11 +2046,11 @@ static void step_fused(const StepCtx& c, hipStream_t s) {
             emf3_tiled(fs(c.F[0]), fs(c.F[1]), fs(c.F[2]), eh, ce, c.fe, eb, c.ctu, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]), s);
         mark(c, K_EMF);
         hipLaunchKernelGGL((k_faraday<D, double>), dim3(blocks(c.fe.size)), dim3(256), 0, s, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]), c.B[0], c.B[1], c.B[2],
-                           c.Bn[0], c.Bn[1], c.Bn[2], c.fe, 0, dt_d[0], dt_d[1], dt_d[2]);
+                           c.Bn[0], c.Bn[1], c.Bn[2], c.fe, 0, &c.ctl->t);
         mark(c, K_FARADAY);
     }
     hipLaunchKernelGGL((k_apply<D, MHD>), dim3(blocks(ce.size)), dim3(256), 0, s, c.W, c.Wn, fs(c.F[0]), fs(c.F[1]), fs(c.F[2]), c.Bn[0], c.Bn[1],
-                       c.Bn[2], ce, c.fe, dt_d[0], dt_d[1], dt_d[2], c.ph, c.err, c.cflpart, c.cfl_mode, c.d[0], c.d[1], c.d[2]);
+                       c.Bn[2], ce, c.fe, &c.ctl->t, c.ph, c.err, c.cflpart, c.cfl_mode, c.d[0], c.d[1], c.d[2]);
     mark(c, K_APPLY);
 }
 
@@ -1934,21 +2063,20 @@ static void step_t(const StepCtx& c, hipStream_t s) {
         }
     }
     const Ext& ce = c.ce;
-    const double dt_d[3] = {c.dt / c.d[0], c.dt / c.d[1], c.dt / c.d[2]};
     const int g = ce.g;
     // half states
     {
         Box all = make_box(D, -g, ce.n[0] + g, -g, ce.n[1] + g, -g, ce.n[2] + g);
         hipLaunchKernelGGL((k_half<D, MHD, R>), dim3(blocks(all.count())), dim3(256), 0, s, c.W, c.B[0], c.B[1], c.B[2], ce, c.fe,
-                           c.HS[0], c.HS[1], c.HS[2], c.HS[3], c.HS[4], c.HS[5], dt_d[0], dt_d[1], dt_d[2], c.ph);
+                           c.HS[0], c.HS[1], c.HS[2], c.HS[3], c.HS[4], c.HS[5], &c.ctl->t, c.ph);
         mark(c, K_HALF);
     }
     if (D == 1) {
         Box fb = make_box(1, -g + 1, ce.n[0] + g, 0, 1, 0, 1);
-        flux_ax<D, MHD, R>(c, 0, c.HS[0], c.HS[1], fs(c.F[0]), fb, dt_d[0], ST_FLUX_X, s);
+        flux_ax<D, MHD, R>(c, 0, c.HS[0], c.HS[1], fs(c.F[0]), fb, ST_FLUX_X, s);
         mark(c, K_FLUX_X);
         if constexpr (D == 1)
-            hipLaunchKernelGGL((k_apply1<MHD>), dim3(blocks(ce.size)), dim3(256), 0, s, c.W, c.Wn, fs(c.F[0]), ce, dt_d[0], c.ph, c.err);
+            hipLaunchKernelGGL((k_apply1<MHD>), dim3(blocks(ce.size)), dim3(256), 0, s, c.W, c.Wn, fs(c.F[0]), ce, &c.ctl->t, c.ph, c.err);
         mark(c, K_APPLY);
         return;
     }
@@ -1956,7 +2084,7 @@ static void step_t(const StepCtx& c, hipStream_t s) {
         if constexpr (MHD) {
             // ctu_sweep_MHD predictor fluxes on [-1, n+1] x [-2, n+2)
             for (int ax = 0; ax < D; ax++) {
-                flux_ax<D, MHD, R>(c, ax, c.HS[2 * ax], c.HS[2 * ax + 1], fs(c.F[ax]), face_box(D, ce, ax, -1, 1, -2, 2), dt_d[ax],
+                flux_ax<D, MHD, R>(c, ax, c.HS[2 * ax], c.HS[2 * ax + 1], fs(c.F[ax]), face_box(D, ce, ax, -1, 1, -2, 2),
                                    ST_PRED_X + ax, s);
                 mark(c, K_PRED_X + ax);
             }
@@ -1970,30 +2098,30 @@ static void step_t(const StepCtx& c, hipStream_t s) {
                                    eb, 1, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]));
             mark(c, K_EMF_PRED);
             hipLaunchKernelGGL((k_faraday<D, ET>), dim3(blocks(c.fe.size)), dim3(256), 0, s, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]), c.B[0], c.B[1],
-                               c.B[2], et(c.Bh[0]), et(c.Bh[1]), et(c.Bh[2]), c.fe, 1, 0.5 * dt_d[0], 0.5 * dt_d[1], 0.5 * dt_d[2]);
+                               c.B[2], et(c.Bh[0]), et(c.Bh[1]), et(c.Bh[2]), c.fe, 1, &c.ctl->t);
             mark(c, K_FARADAY_HALF);
             Box cb = make_box(D, -1, ce.n[0] + 1, -1, ce.n[1] + 1, -1, ce.n[2] + 1);
             hipLaunchKernelGGL((k_whalf<D>), dim3(blocks(cb.count())), dim3(256), 0, s, c.W, fs(c.F[0]), fs(c.F[1]), fs(c.F[2]), et(c.Bh[0]), et(c.Bh[1]),
-                               et(c.Bh[2]), ce, c.fe, cb, 0.5 * dt_d[0], 0.5 * dt_d[1], 0.5 * dt_d[2], c.ph, et(c.Eh[0]), et(c.Eh[1]), et(c.Eh[2]),
+                               et(c.Bh[2]), ce, c.fe, cb, &c.ctl->t, c.ph, et(c.Eh[0]), et(c.Eh[1]), et(c.Eh[2]),
                                c.err);
             mark(c, K_WHALF);
             hipLaunchKernelGGL((k_ctu_mhd<D>), dim3(blocks(cb.count())), dim3(256), 0, s, c.W, c.B[0], c.B[1], c.B[2], et(c.Bh[0]), et(c.Bh[1]),
                                et(c.Bh[2]), et(c.E0[0]), et(c.E0[1]), et(c.E0[2]), fs(c.F[0]), fs(c.F[1]), fs(c.F[2]), c.HS[0], c.HS[1], c.HS[2], c.HS[3],
-                               c.HS[4], c.HS[5], ce, c.fe, cb, dt_d[0], dt_d[1], dt_d[2], c.ph);
+                               c.HS[4], c.HS[5], ce, c.fe, cb, &c.ctl->t, c.ph);
             mark(c, K_CTU);
         } else if constexpr (D == 2) {
             // ctu_sweep_hydro 2D (CTU.cpp:206-218)
-            flux_ax<D, MHD, R>(c, 0, c.HS[0], c.HS[1], fs(c.F[0]), face_box(D, ce, 0, 0, 0, -1, 1), dt_d[0], ST_PRED_X, s);
+            flux_ax<D, MHD, R>(c, 0, c.HS[0], c.HS[1], fs(c.F[0]), face_box(D, ce, 0, 0, 0, -1, 1), ST_PRED_X, s);
             mark(c, K_PRED_X);
-            flux_ax<D, MHD, R>(c, 1, c.HS[2], c.HS[3], fs(c.F[1]), face_box(D, ce, 1, 0, 0, -1, 1), dt_d[1], ST_PRED_Y, s);
+            flux_ax<D, MHD, R>(c, 1, c.HS[2], c.HS[3], fs(c.F[1]), face_box(D, ce, 1, 0, 0, -1, 1), ST_PRED_Y, s);
             mark(c, K_PRED_Y);
             Box bx = make_box(2, -1, ce.n[0] + 1, 0, ce.n[1]);
             hipLaunchKernelGGL((k_correct<D, R>), dim3(blocks(bx.count())), dim3(256), 0, s, c.HS[0], c.HS[1], fs(c.F[1]), ce, bx, 1,
-                               0.5 * dt_d[1], c.ph);
+                               &c.ctl->t, c.ph);
             mark(c, K_CTU);
             Box by = make_box(2, 0, ce.n[0], -1, ce.n[1] + 1);
             hipLaunchKernelGGL((k_correct<D, R>), dim3(blocks(by.count())), dim3(256), 0, s, c.HS[2], c.HS[3], fs(c.F[0]), ce, by, 0,
-                               0.5 * dt_d[0], c.ph);
+                               &c.ctl->t, c.ph);
             mark(c, K_CTU);
         } else {
             ctu_hydro3(c, s);
@@ -2003,13 +2131,13 @@ static void step_t(const StepCtx& c, hipStream_t s) {
     // final fluxes
     if (MHD) {
         for (int ax = 0; ax < D; ax++) {
-            flux_ax<D, MHD, R>(c, ax, c.HS[2 * ax], c.HS[2 * ax + 1], fs(c.F[ax]), face_box(D, ce, ax, 0, 0, -1, 1), dt_d[ax],
+            flux_ax<D, MHD, R>(c, ax, c.HS[2 * ax], c.HS[2 * ax + 1], fs(c.F[ax]), face_box(D, ce, ax, 0, 0, -1, 1),
                                ST_FLUX_X + ax, s);
             mark(c, K_FLUX_X + ax);
         }
     } else {
         for (int ax = 0; ax < D; ax++) {
-            flux_ax<D, MHD, R>(c, ax, c.HS[2 * ax], c.HS[2 * ax + 1], fs(c.F[ax]), face_box(D, ce, ax, 0, 0, 0, 0), dt_d[ax],
+            flux_ax<D, MHD, R>(c, ax, c.HS[2 * ax], c.HS[2 * ax + 1], fs(c.F[ax]), face_box(D, ce, ax, 0, 0, 0, 0),
                                ST_FLUX_X + ax, s);
             mark(c, K_FLUX_X + ax);
         }
@@ -2025,11 +2153,11 @@ static void step_t(const StepCtx& c, hipStream_t s) {
                                c.ctu, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]));
         mark(c, K_EMF);
         hipLaunchKernelGGL((k_faraday<D, double>), dim3(blocks(c.fe.size)), dim3(256), 0, s, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]), c.B[0], c.B[1], c.B[2],
-                           c.Bn[0], c.Bn[1], c.Bn[2], c.fe, 0, dt_d[0], dt_d[1], dt_d[2]);
+                           c.Bn[0], c.Bn[1], c.Bn[2], c.fe, 0, &c.ctl->t);
         mark(c, K_FARADAY);
     }
     hipLaunchKernelGGL((k_apply<D, MHD>), dim3(blocks(ce.size)), dim3(256), 0, s, c.W, c.Wn, fs(c.F[0]), fs(c.F[1]), fs(c.F[2]), c.Bn[0], c.Bn[1],
-                       c.Bn[2], ce, c.fe, dt_d[0], dt_d[1], dt_d[2], c.ph, c.err, c.cflpart, c.cfl_mode, c.d[0], c.d[1], c.d[2]);
+                       c.Bn[2], ce, c.fe, &c.ctl->t, c.ph, c.err, c.cflpart, c.cfl_mode, c.d[0], c.d[1], c.d[2]);
     mark(c, K_APPLY);
 }
 
@@ -2037,48 +2165,47 @@ static void step_t(const StepCtx& c, hipStream_t s) {
 // dt/3 transverse corrections, then the state corrections.
 void ctu_hydro3(const StepCtx& c, hipStream_t s) {
     const Ext& ce = c.ce;
-    const double dx = c.dt / c.d[0], dy = c.dt / c.d[1], dz = c.dt / c.d[2];
     const Soa &xL = c.HS[0], &xR = c.HS[1], &yL = c.HS[2], &yR = c.HS[3], &zL = c.HS[4], &zR = c.HS[5];
     const FSoa FX = fs(c.F[0]), FY = fs(c.F[1]), FZ = fs(c.F[2]);
     FSoa T[5];  // five scratch flux arrays
     for (int q = 0; q < 5; q++) T[q] = fs(c.T[q]);
     const int nx = ce.n[0], ny = ce.n[1], nz = ce.n[2];
-    flux_t<3, false, double, 0>(c, xL, xR, FX, make_box(3, 0, nx + 1, -1, ny + 1, -1, nz + 1), dx, ST_PRED_X, s);
-    flux_t<3, false, double, 1>(c, yL, yR, FY, make_box(3, -1, nx + 1, 0, ny + 1, -1, nz + 1), dy, ST_PRED_Y, s);
-    flux_t<3, false, double, 2>(c, zL, zR, FZ, make_box(3, -1, nx + 1, -1, ny + 1, 0, nz + 1), dz, ST_PRED_Z, s);
-    auto ctu = [&](int ax, const Soa& L, const Soa& Rr, const FSoa& Tr, int tax, const FSoa& out, double dd, double dtt, int stage) {
+    flux_t<3, false, double, 0>(c, xL, xR, FX, make_box(3, 0, nx + 1, -1, ny + 1, -1, nz + 1), ST_PRED_X, s);
+    flux_t<3, false, double, 1>(c, yL, yR, FY, make_box(3, -1, nx + 1, 0, ny + 1, -1, nz + 1), ST_PRED_Y, s);
+    flux_t<3, false, double, 2>(c, zL, zR, FZ, make_box(3, -1, nx + 1, -1, ny + 1, 0, nz + 1), ST_PRED_Z, s);
+    auto ctu = [&](int ax, const Soa& L, const Soa& Rr, const FSoa& Tr, int tax, const FSoa& out, int stage) {
         int isX = tax == 0, isY = tax == 1, isZ = tax == 2;
         Box b;
         if (ax == 0) b = make_box(3, 0, nx + 1, -1 + isY, ny + 1 - isY, -1 + isZ, nz + 1 - isZ);
         else if (ax == 1) b = make_box(3, -1 + isX, nx + 1 - isX, 0, ny + 1, -1 + isZ, nz + 1 - isZ);
         else b = make_box(3, -1 + isX, nx + 1 - isX, -1 + isY, ny + 1 - isY, 0, nz + 1);
         if (ax == 0)
-            hipLaunchKernelGGL((k_ctu_flux<double, 0>), dim3(blocks(b.count())), dim3(256), 0, s, L, Rr, Tr, out, ce, b, tax, dd, dtt, c.ph, c.err, stage);
+            hipLaunchKernelGGL((k_ctu_flux<double, 0>), dim3(blocks(b.count())), dim3(256), 0, s, L, Rr, Tr, out, ce, b, tax, &c.ctl->t, c.ph, c.err, stage);
         else if (ax == 1)
-            hipLaunchKernelGGL((k_ctu_flux<double, 1>), dim3(blocks(b.count())), dim3(256), 0, s, L, Rr, Tr, out, ce, b, tax, dd, dtt, c.ph, c.err, stage);
+            hipLaunchKernelGGL((k_ctu_flux<double, 1>), dim3(blocks(b.count())), dim3(256), 0, s, L, Rr, Tr, out, ce, b, tax, &c.ctl->t, c.ph, c.err, stage);
         else
-            hipLaunchKernelGGL((k_ctu_flux<double, 2>), dim3(blocks(b.count())), dim3(256), 0, s, L, Rr, Tr, out, ce, b, tax, dd, dtt, c.ph, c.err, stage);
+            hipLaunchKernelGGL((k_ctu_flux<double, 2>), dim3(blocks(b.count())), dim3(256), 0, s, L, Rr, Tr, out, ce, b, tax, &c.ctl->t, c.ph, c.err, stage);
     };
-    auto corr = [&](const Soa& L, const Soa& Rr, const FSoa& F, double dd, int sdim, int fdim) {
+    auto corr = [&](const Soa& L, const Soa& Rr, const FSoa& F, int sdim, int fdim) {
         int lo[3] = {0, 0, 0}, hi[3] = {nx, ny, nz};
         lo[sdim] = -1; hi[sdim] += 1;
         Box b = make_box(3, lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]);
-        hipLaunchKernelGGL((k_correct<3, double>), dim3(blocks(b.count())), dim3(256), 0, s, L, Rr, F, ce, b, fdim, dd, c.ph);
+        hipLaunchKernelGGL((k_correct<3, double>), dim3(blocks(b.count())), dim3(256), 0, s, L, Rr, F, ce, b, fdim, &c.ctl->t, c.ph);
     };
     const FSoa &FXz = T[0], &FYz = T[1], &FXy = T[2], &FZy = T[3], &FYx = T[4];
-    ctu(0, xL, xR, FZ, 2, FXz, dx, dz / 3.0, ST_CTU_F0 + 0);
-    ctu(1, yL, yR, FZ, 2, FYz, dy, dz / 3.0, ST_CTU_F0 + 1);
-    ctu(0, xL, xR, FY, 1, FXy, dx, dy / 3.0, ST_CTU_F0 + 2);
-    ctu(2, zL, zR, FY, 1, FZy, dz, dy / 3.0, ST_CTU_F0 + 3);
-    corr(xL, xR, FYz, 0.5 * dy, 0, 1);
-    corr(xL, xR, FZy, 0.5 * dz, 0, 2);
-    ctu(1, yL, yR, FX, 0, FYx, dy, dx / 3.0, ST_CTU_F0 + 4);
+    ctu(0, xL, xR, FZ, 2, FXz, ST_CTU_F0 + 0);
+    ctu(1, yL, yR, FZ, 2, FYz, ST_CTU_F0 + 1);
+    ctu(0, xL, xR, FY, 1, FXy, ST_CTU_F0 + 2);
+    ctu(2, zL, zR, FY, 1, FZy, ST_CTU_F0 + 3);
+    corr(xL, xR, FYz, 0, 1);
+    corr(xL, xR, FZy, 0, 2);
+    ctu(1, yL, yR, FX, 0, FYx, ST_CTU_F0 + 4);
     const FSoa& FZx = FZ;  // FZ is no longer needed
-    ctu(2, zL, zR, FX, 0, FZx, dz, dx / 3.0, ST_CTU_F0 + 5);
-    corr(yL, yR, FXz, 0.5 * dx, 1, 0);
-    corr(yL, yR, FZx, 0.5 * dz, 1, 2);
-    corr(zL, zR, FXy, 0.5 * dx, 2, 0);
-    corr(zL, zR, FYx, 0.5 * dy, 2, 1);
+    ctu(2, zL, zR, FX, 0, FZx, ST_CTU_F0 + 5);
+    corr(yL, yR, FXz, 1, 0);
+    corr(yL, yR, FZx, 1, 2);
+    corr(zL, zR, FXy, 2, 0);
+    corr(zL, zR, FYx, 2, 1);
 }
 
 // ===================================================== batched patches
@@ -2221,15 +2348,17 @@ KB __global__ void kb_dt(BatchArgs A) {
     double dt = A.cfl_coeff / m;
     for (int h = 0; h < A.halv[p]; h++) dt *= 0.5;
     A.dt[p] = dt;
+    const double q[3] = {dt / A.P[p].d[0], dt / A.P[p].d[1], dt / 1.0};
+    for (int k = 0; k < 3; k++) { A.ts[p].full[k] = q[k]; A.ts[p].half[k] = 0.5 * q[k]; }
 }
 template <int AX, bool FIN>
 __device__ __forceinline__ SweepArgs batch_sweep_args(const BatchArgs& A, const PatchView& v, int p) {
     SweepArgs s{};
-    const double dt = A.dt[p];
-    const double dt_d[3] = {dt / v.dx, dt / v.dy, dt / 1.0};
     s.W = v.W;
+    s.ts = A.ts + p;
+    s.half = 0;
     for (int q = 0; q < 3; q++) {
-        s.B[q] = v.B[q]; s.Bh[q] = v.Bh[q]; s.E0[q] = v.E0[q]; s.Fp[q] = v.Fp[q]; s.dt_d[q] = dt_d[q];
+        s.B[q] = v.B[q]; s.Bh[q] = v.Bh[q]; s.E0[q] = v.E0[q]; s.Fp[q] = v.Fp[q];
     }
     s.ce = v.ce; s.fe = v.fe; s.ph = A.ph; s.err = A.err + p;
     const int nx = v.ce.n[0], ny = v.ce.n[1];
@@ -2292,25 +2421,22 @@ template <bool HALF>
 KB __global__ void kb_faraday(BatchArgs A, BlockTable bt) {
     BATCH_ITEM(bt)
     const PatchView v = patch_view(A, p);
-    const double dt = A.dt[p], f = HALF ? 0.5 : 1.0;
-    const double dx = f * (dt / v.dx), dy = f * (dt / v.dy), dz = f * (dt / 1.0);
+    const double dx = dts(A.ts + p, 0, HALF), dy = dts(A.ts + p, 1, HALF), dz = dts(A.ts + p, 2, HALF);
     if (HALF) faraday_body<2, ET>(v.E0[0], v.E0[1], v.E0[2], v.B[0], v.B[1], v.B[2], v.Bh[0], v.Bh[1], v.Bh[2], v.fe, 1, dx, dy, dz, t);
     else faraday_body<2, double>(v.E0[0], v.E0[1], v.E0[2], v.B[0], v.B[1], v.B[2], v.Bn[0], v.Bn[1], v.Bn[2], v.fe, 0, dx, dy, dz, t);
 }
 KB __global__ void kb_whalf(BatchArgs A, BlockTable bt) {
     BATCH_ITEM(bt)
     const PatchView v = patch_view(A, p);
-    const double dt = A.dt[p];
     const Box cb = make_box(2, -1, v.ce.n[0] + 1, -1, v.ce.n[1] + 1);
-    whalf_body<2>(v.W, v.Fp[0], v.Fp[1], v.Fp[2], v.Bh[0], v.Bh[1], v.Bh[2], v.ce, v.fe, cb, 0.5 * (dt / v.dx), 0.5 * (dt / v.dy),
-                  0.5 * (dt / 1.0), A.ph, v.Eh[0], v.Eh[1], v.Eh[2], A.err + p, t);
+    whalf_body<2>(v.W, v.Fp[0], v.Fp[1], v.Fp[2], v.Bh[0], v.Bh[1], v.Bh[2], v.ce, v.fe, cb, dts(A.ts + p, 0, true),
+                  dts(A.ts + p, 1, true), dts(A.ts + p, 2, true), A.ph, v.Eh[0], v.Eh[1], v.Eh[2], A.err + p, t);
 }
 KB __global__ void kb_apply(BatchArgs A, BlockTable bt) {
     BATCH_ITEM(bt)
     const PatchView v = patch_view(A, p);
-    const double dt = A.dt[p];
-    double m = apply_body<2, true>(v.W, v.Wn, v.F[0], v.F[1], v.F[2], v.Bn[0], v.Bn[1], v.Bn[2], v.ce, v.fe, dt / v.dx, dt / v.dy,
-                                   dt / 1.0, A.ph, A.err + p, t, true, A.cfl_mode, v.dx, v.dy, 1.0);
+    double m = apply_body<2, true>(v.W, v.Wn, v.F[0], v.F[1], v.F[2], v.Bn[0], v.Bn[1], v.Bn[2], v.ce, v.fe, dts(A.ts + p, 0),
+                                   dts(A.ts + p, 1), dts(A.ts + p, 2), A.ph, A.err + p, t, true, A.cfl_mode, v.dx, v.dy, 1.0);
     // the new state's CFL maximum over the patch's interior, for the next
     // step if this one is committed (one atomic per workgroup)
     for (int off = 32; off > 0; off >>= 1) m = dmax(m, __shfl_xor(m, off));
@@ -2380,7 +2506,9 @@ void launch_batch_step(const BatchArgs& a, const BlockTable* bt, bool init_only,
 template <class T> __device__ __forceinline__ P<T> to_line(const P<T>& w, int ax) { return ax == 0 ? w : ax == 1 ? swapXY(w) : swapXZ(w); }
 template <class T> __device__ __forceinline__ U<T> to_line(const U<T>& u, int ax) { return ax == 0 ? u : ax == 1 ? swapXY(u) : swapXZ(u); }
 template <int D, int AX>
-KB __global__ void k_apply_axis(Soa W, Soa Wn, FSoa F, Ext ce, double dt_d, Phys ph) {
+KB __global__ void k_apply_axis(Soa W, Soa Wn, FSoa F, Ext ce, const StepDts* ts, int half, Phys ph) {
+    if (stopped(ts)) return;
+    const double dt_d = dts(ts, AX, half);
     const long m = tid();
     if (m >= ce.size) return;
     const int g = ce.g, n = ce.n[AX];
@@ -2419,7 +2547,7 @@ static void split_axis_t(const StepCtx& c, const Soa& in, const Soa& out, hipStr
         }
         const Box b = make_box(D, lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]);
         sweep<D, false, RT, false>(cs, AX, b, fs(c.F[AX]), ST_FLUX_X + AX, s);
-        hipLaunchKernelGGL((k_apply_axis<D, AX>), dim3(blocks(ce.size)), dim3(256), 0, s, in, out, fs(c.F[AX]), ce, c.dt / c.d[AX], c.ph);
+        hipLaunchKernelGGL((k_apply_axis<D, AX>), dim3(blocks(ce.size)), dim3(256), 0, s, in, out, fs(c.F[AX]), ce, &c.ctl->t, c.half, c.ph);
     }
 }
 void launch_split_axis(const StepCtx& c, int ax, Soa in, Soa out, hipStream_t s) {

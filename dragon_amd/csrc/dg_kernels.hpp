@@ -16,6 +16,28 @@ static const char* const kKernelNames[K_COUNT] = {
     "boundary", "cfl", "half_states", "pred_sweep_x", "pred_sweep_y", "pred_sweep_z", "emf_pred", "faraday_half",
     "whalf", "ctu_correct", "flux_sweep_x", "flux_sweep_y", "flux_sweep_z", "emf", "faraday", "apply"};
 
+// The step sizes of a step, in device memory: the CFL pass may have found
+// them on the device (launch_ctl_* / launch_cfl), so that the host need not
+// wait for one step to launch the next.
+struct StepDts {
+    double full[3], half[3];  // dt / dx, dt / dy, dt / dz and their halves
+    int stop, pad;            // set: every kernel of the step leaves at once
+};
+// Control of a run of steps launched without waiting (dg_advance).  The CFL
+// pass of a step commits the one before it: where that one failed, or no time
+// is left, it sets `stop` and every later launch of the run does nothing.
+constexpr int CTL_RING = 64;  // steps of a run
+enum { CTL_NO_SPEED = 1 };    // why: the maximum signal speed is zero
+struct StepCtl {
+    StepDts t;
+    double dt, left, left_next, tol;  // of the step begun last: its dt, the time left before and after it
+    unsigned long long err;           // its failure key
+    unsigned long long vmax;          // CFL maximum being gathered (FP64 bits)
+    int count, why;                   // steps begun; CTL_*
+    unsigned ticket, pad;             // workgroups of the CFL pass that have finished
+    double ring[CTL_RING];            // dt of each step begun
+};
+
 // Everything one unsplit step needs: geometry, physics switches, the current
 // and next state, and the scratch arrays of the stages.
 struct StepCtx {
@@ -28,7 +50,9 @@ struct StepCtx {
     Ext ce, fe;
     Phys ph;
     double d[3];
-    double dt;
+    StepCtl* ctl;         // step sizes, stop flag and failure word
+    int half;             // split sweeps: steps of dt / 2
+    double cfl_coeff;
     Soa W, Wn;            // current / next cell state
     double* B[3];         // current face B
     double* Bn[3];        // next face B
@@ -50,6 +74,7 @@ inline void mark(const StepCtx& c, int id) {
 
 // One boundary pass (cells or faces of one face/axis of one BC element).
 struct BCArgs {
+    const StepCtl* ctl;  // of a run of steps (its end is checked before the pass), or null
     Soa W;
     double* B[3];
     Ext ce, fe;
@@ -64,6 +89,7 @@ struct BCPass {
     double st[8];
 };
 struct BCListArgs {
+    const StepCtl* ctl;     // as BCArgs
     Soa W;
     double* B[3];
     Ext ce, fe;
@@ -123,6 +149,7 @@ struct BatchArgs {
     unsigned long long* vnext; // per patch: the apply pass's maximum over the interior of the state it wrote (FP64 bits)
     int* cfl_ok;               // per patch: vnext describes the current state (its last attempt was committed)
     double* dt;                // per patch dt of the current attempt
+    StepDts* ts;               // per patch dt / dx, dt / dy of the current attempt
     int* halv;                 // per patch halvings since the last accepted step
     int* active;               // per patch: steps in this launch sequence
     Phys ph;
@@ -146,8 +173,11 @@ struct BatchArgs {
     void launch_split_axis(const StepCtx& c, int ax, Soa in, Soa out, hipStream_t s);  /* one split sweep (hydro) */ \
     void launch_bc(const BCArgs& a, bool faces, hipStream_t s);                                                 \
     bool launch_bc_list(BCListArgs& a, hipStream_t s);                                                          \
-    void launch_cfl(const StepCtx& c, unsigned long long* out, hipStream_t s);                                  \
-    void launch_cfl_tail(const StepCtx& c, long nparts, unsigned long long* out, hipStream_t s);                \
+    void launch_cfl(const StepCtx& c, unsigned long long* out, bool run, hipStream_t s);                        \
+    void launch_cfl_tail(const StepCtx& c, long nparts, unsigned long long* out, bool run, hipStream_t s);      \
+    void launch_ctl_set(const StepCtx& c, double dt, hipStream_t s);        /* one step of size dt */             \
+    void launch_ctl_begin(const StepCtx& c, double left, double tol, hipStream_t s);  /* a run of steps */        \
+    void launch_ctl_next(const StepCtx& c, hipStream_t s);                  /* its next step, without CFL */      \
     void launch_init_B(int dim, Soa W, double* B, Ext ce, Ext fe, hipStream_t s);                               \
     void launch_divb(int dim, double* B, Ext ce, Ext fe, const double d[3], unsigned long long* out, hipStream_t s); \
     void launch_fill_u64(unsigned long long* p, unsigned long long v, int n, hipStream_t s);                    \
