@@ -161,7 +161,7 @@ static StepCtx make_ctx(dg_grid* g) {
     if (g->Fp)
         for (int q = 0; q < g->d.dim; q++) c.Fp[q] = soa(g->Fp + (long)q * g->nf * nc, nc);
     if (g->T)
-        for (int q = 0; q < 5; q++) c.T[q] = soa(g->T + (long)q * g->nf * nc, nc);
+        for (int q = 0; q < (g->fused ? 6 : 5); q++) c.T[q] = soa(g->T + (long)q * g->nf * nc, nc);
     c.err = &g->ctl->err;
     c.cflpart = g->cflpart;
     c.mark = g->timing ? tm_mark : nullptr;
@@ -210,9 +210,10 @@ int dg_create(const dg_desc* desc, dg_grid** out) {
     };
     bool ok = hipStreamCreateWithFlags(&g->s, hipStreamNonBlocking) == hipSuccess;
     ok = ok && alloc(&g->W, 8 * nc) && alloc(&g->Wn, 8 * nc);
-    // fused sweeps (MHD 2D/3D, hydro 2D) need predictor + corrector fluxes;
-    // 1D and 3D hydro keep the reference's half-state arrays
-    const bool fusable = (d.mhd && d.dim >= 2) || (!d.mhd && d.dim == 2);
+    // fused sweeps (2D, 3D) need predictor + corrector fluxes, 3D hydro six
+    // corner fluxes instead of the former; 1D keeps the reference's half-state
+    // arrays
+    const bool fusable = d.dim >= 2, hydro3 = !d.mhd && d.dim == 3;
     g->fused = fusable && getenv("DG_UNFUSED") == nullptr;
     // diagnostic: fixed faces per walker of the strided-axis sweeps (results do not depend on it)
     if (const char* mc = getenv("DG_MARCH_CHUNK")) g->march_chunk = atoi(mc);
@@ -220,9 +221,9 @@ int dg_create(const dg_desc* desc, dg_grid** out) {
     // uses, so the FP64 parity tests hold that form to the oracle bit for bit
     g->march_window = getenv("DG_MARCH_WINDOW_CHECK") != nullptr;
     ok = ok && alloc(&g->F, (long)d.dim * g->nf * nc);
-    if (g->fused) ok = ok && (!d.ctu || alloc(&g->Fp, (long)d.dim * g->nf * nc));
+    if (g->fused) ok = ok && (!d.ctu || hydro3 || alloc(&g->Fp, (long)d.dim * g->nf * nc));
     else ok = ok && alloc(&g->HS, 2L * d.dim * g->nf * nc);
-    if (!d.mhd && d.dim == 3 && d.ctu) ok = ok && alloc(&g->T, 5L * g->nf * nc);
+    if (hydro3 && d.ctu) ok = ok && alloc(&g->T, (g->fused ? 6L : 5L) * g->nf * nc);
     if (faces) ok = ok && alloc(&g->B, 3 * nfc) && alloc(&g->Bn, 3 * nfc) && alloc(&g->Bh, 3 * nfc) && alloc(&g->E0, 3 * nfc) &&
                     alloc(&g->Eh, 3 * nfc);
     if (d.dim >= 2) {
@@ -1062,15 +1063,16 @@ extern "C" int dg_step_noalloc(const dg_desc* desc, const double* w_in, const do
     g.ce = make_ext(d.dim, d.nx, d.ny, d.nz, gh);
     g.fe = make_ext(d.dim, d.nx + 1, d.ny + 1, d.nz + 1, gh);
     g.ph = make_phys(d);
-    g.fused = (d.mhd && d.dim >= 2) || (!d.mhd && d.dim == 2);
-    const NoallocLayout L = noalloc_layout(d, g.ce, g.fe, g.fused);
+    g.fused = d.dim >= 2;
+    const bool hydro3 = !d.mhd && d.dim == 3;
+    const NoallocLayout L = noalloc_layout(d, g.ce, g.fe, g.fused && !hydro3);
     g.W = const_cast<double*>(w_in);
     g.Wn = w_out;
     if (faces) { g.B = const_cast<double*>(B_in); g.Bn = B_out; }
     g.F = base + L.F;
     if (L.Fp >= 0) g.Fp = base + L.Fp;
     if (L.HS >= 0) g.HS = base + L.HS;
-    if (L.T >= 0) g.T = base + L.T;
+    if (hydro3) { g.T = g.HS; g.HS = nullptr; }  // the layout's half states hold the six corner fluxes
     if (L.Bh >= 0) { g.Bh = base + L.Bh; g.E0 = base + L.E0; g.Eh = base + L.Eh; }
     g.ctl = (StepCtl*)((unsigned char*)sp + NOALLOC_SCRATCH_BYTES);
     g.cflpart = nullptr;

@@ -753,8 +753,8 @@ struct SweepArgs {
     const double* B[3];
     const ET* Bh[3];       // half-step face B (ET storage)
     const ET* E0[3];
-    FSoa Fp[3];            // predictor fluxes (corrector pass input)
-    FSoa Fo;               // output fluxes of this axis
+    FSoa Fp[3];            // predictor fluxes (corrector pass input; 3D hydro: [0], [1] the corner fluxes of the corrections)
+    FSoa Fo, Fo2;          // output fluxes of this axis (Fo2: corner sweeps only)
     Ext ce, fe;
     int lo[3], hi[3];      // faces [lo, hi) per dim; face f of axis AX sits between cells f-1 and f
     const StepDts* ts;
@@ -830,7 +830,16 @@ __device__ __forceinline__ void ctu_correct(const SweepArgs& a, long m, long q, 
     const Ext& ce = a.ce;
     const Phys& ph = a.ph;
     auto fd = [&](int ax) { return usub<MHD>(load_u(a.Fp[ax], m, MHD), load_u(a.Fp[ax], m + ce.s[ax], MHD)); };
-    if constexpr (!MHD) {  // correctState (hydro 2D): minus the transverse flux difference
+    if constexpr (!MHD && D == 3) {  // correctState (hydro 3D, CTU.cpp:228-259): one transverse corner flux after the other
+        constexpr int T1 = AX == 0 ? 1 : 0, T2 = AX == 2 ? 1 : 2;
+        U<double> t = umul<false>(usub<false>(load_u(a.Fp[0], m + ce.s[T1], false), load_u(a.Fp[0], m, false)), dts(a.ts, T1, true));
+        L = prim<false>(usub<false>(cons<false>(L, ph), t), ph);
+        Rr = prim<false>(usub<false>(cons<false>(Rr, ph), t), ph);
+        t = umul<false>(usub<false>(load_u(a.Fp[1], m + ce.s[T2], false), load_u(a.Fp[1], m, false)), dts(a.ts, T2, true));
+        L = prim<false>(usub<false>(cons<false>(L, ph), t), ph);
+        Rr = prim<false>(usub<false>(cons<false>(Rr, ph), t), ph);
+        return;
+    } else if constexpr (!MHD) {  // correctState (hydro 2D): minus the transverse flux difference
         constexpr int T = AX == 0 ? 1 : 0;
         U<double> t = umul<false>(usub<false>(load_u(a.Fp[T], m + ce.s[T], false), load_u(a.Fp[T], m, false)), 0.5 * a.dt_d(T));
         L = prim_c<false>(usub<false>(cons_c<false>(L, ph), t), ph);
@@ -963,16 +972,19 @@ __device__ __forceinline__ void cell_states(const SweepArgs& a, int i, int j, in
     }
 }
 
-template <bool MHD, class R, int AX>
-__device__ __forceinline__ void face_flux(const SweepArgs& a, P<R> l, P<R> r, long m) {
+template <bool MHD, class R, int AX, class RS = R>
+__device__ __forceinline__ void face_flux(const SweepArgs& a, const P<R>& l0, const P<R>& r0, long m) {
+    P<RS> l, r;
+    if constexpr (sizeof(RS) == sizeof(R)) { l = l0; r = r0; }
+    else { l = p_wide(l0); r = p_wide(r0); }
     if (AX == 1) { l = swapXY(l); r = swapXY(r); }
     if (AX == 2) { l = swapXZ(l); r = swapXZ(r); }
     int fail = RF_OK;
-    U<R> f = riemann_x<MHD, R>(l, r, R(a.dt_d(AX)), a.ph, &fail);
+    U<RS> f = riemann_x<MHD, RS>(l, r, RS(a.dt_d(AX)), a.ph, &fail);
     if (fail) report(a.err, a.stage, (unsigned long long)m, fail == RF_BAD_INPUT ? E_RIEMANN_INPUT : E_RIEMANN_SOLUTION);
     if (AX == 1) f = swapXY(f);
     if (AX == 2) f = swapXZ(f);
-    store_u<R>(a.Fo, m, f, MHD);
+    store_u<RS>(a.Fo, m, f, MHD);
 }
 
 // Windowed walkers (stencil cells carried in registers) for the FP32 form;
@@ -991,7 +1003,8 @@ template <> struct Pair2<double> { using T = double2; };
 // windowed walker parks its carried state in LDS in the predictor too (the
 // batched walkers); without it, a must be the kernel's own argument (the
 // single-grid walkers).
-template <int D, bool MHD, class R, int AX, bool FINAL, bool WIN = march_window<R>(), bool PARKALL = false>
+// RS: the type the faces are solved in.
+template <int D, bool MHD, class R, int AX, bool FINAL, bool WIN = march_window<R>(), bool PARKALL = false, class RS = R>
 __device__ __forceinline__ void sweep_march_body(const SweepArgs& a, long t) {
     constexpr int T0 = AX == 0 ? 1 : 0;            // slower transverse dim (3D only)
     constexpr int T1 = D == 3 ? (AX == 2 ? 1 : 2) : (AX == 0 ? 1 : 0);  // fastest transverse dim
@@ -1074,10 +1087,10 @@ __device__ __forceinline__ void sweep_march_body(const SweepArgs& a, long t) {
                 put(2, Rc);
                 // Rc's only copy for the next face is the one in LDS
                 asm volatile("" ::: "memory");
-                if (f >= f0) face_flux<MHD, R, AX>(a, Rp, Lc, m);  // uniform per wavefront
+                if (f >= f0) face_flux<MHD, R, AX, RS>(a, Rp, Lc, m);  // uniform per wavefront
                 sl = 1 - sl;
             } else {
-                if (f >= f0) face_flux<MHD, R, AX>(a, Rp, Lc, m);
+                if (f >= f0) face_flux<MHD, R, AX, RS>(a, Rp, Lc, m);
                 Rp = Rc;
                 wl = wc;
                 wc = wr;
@@ -1102,7 +1115,7 @@ __device__ __forceinline__ void sweep_march_body(const SweepArgs& a, long t) {
             cell_states_from<D, MHD, R, AX, FINAL>(a, idx[0], idx[1], idx[2], p_cast<R>(ld(f - 1, m - s)), p_cast<R>(ld(f, m)),
                                                    p_cast<R>(nxt), Lc, Rc);
             nxt = ld(f + 2, m + 2 * s);
-            if (f >= f0) face_flux<MHD, R, AX>(a, Rp, Lc, m);
+            if (f >= f0) face_flux<MHD, R, AX, RS>(a, Rp, Lc, m);
             Rp = Rc;
             m += s;
         }
@@ -1111,13 +1124,13 @@ __device__ __forceinline__ void sweep_march_body(const SweepArgs& a, long t) {
 // Occupancy floor of the FP32 walkers: four waves per SIMD for the predictor
 // (133 registers, 8 bytes per lane spilled at four, 5-8% faster than three)
 // and the parked corrector (116-118 registers).  1 = the compiler's choice.
-template <int D, int AX, class R, bool FINAL> constexpr int march_min_waves() {
-    return DG_SWEEP_WAVES == 0 && sizeof(R) == 4 && (!FINAL || !(D == 3 && AX == 0)) ? 4 : 1;
+template <int D, int AX, class R, bool FINAL, class RS> constexpr int march_min_waves() {
+    return DG_SWEEP_WAVES == 0 && sizeof(R) == 4 && sizeof(RS) == 4 && (!FINAL || !(D == 3 && AX == 0)) ? 4 : 1;
 }
-template <int D, bool MHD, class R, int AX, bool FINAL>
-KS __attribute__((amdgpu_waves_per_eu(march_min_waves<D, AX, R, FINAL>()))) __global__ void k_sweep_march(SweepArgs a) {
+template <int D, bool MHD, class R, int AX, bool FINAL, class RS>
+KS __attribute__((amdgpu_waves_per_eu(march_min_waves<D, AX, R, FINAL, RS>()))) __global__ void k_sweep_march(SweepArgs a) {
     if (stopped(a.ts)) return;
-    sweep_march_body<D, MHD, R, AX, FINAL>(a, tid_xcd());
+    sweep_march_body<D, MHD, R, AX, FINAL, march_window<R>(), false, RS>(a, tid_xcd());
 }
 template <int D, bool MHD, class R, int AX, bool FINAL>
 KS __global__ void k_sweep_march_window(SweepArgs a) {
@@ -1135,7 +1148,7 @@ template <class R> __device__ __forceinline__ P<R> shfl_up1(const P<R>& w) {
 // c0-1+l and lanes 1..SW-1 take the left state from the lane below, so a
 // segment computes SW-1 faces.  With SW = 64 the segment is the wavefront
 // and its index is wave-uniform.
-template <int D, bool MHD, class R, int AX, bool FINAL, int SW = 64>
+template <int D, bool MHD, class R, int AX, bool FINAL, int SW = 64, class RS = R>
 __device__ __forceinline__ void sweep_wave_body(const SweepArgs& a, long seg_id, int lane) {
     constexpr int T0 = 0;                 // slowest transverse dim
     constexpr int T1 = D == 3 ? 1 : 0;    // faster transverse dim
@@ -1158,7 +1171,7 @@ __device__ __forceinline__ void sweep_wave_body(const SweepArgs& a, long seg_id,
     if (live) cell_states<D, MHD, R, AX, FINAL>(a, idx[0], idx[1], idx[2], L, Rr, &wc);
     if constexpr (eref_in_sweep<D, MHD, FINAL, AX>()) store_eref(a, live, idx, wc);
     const P<R> Rl = shfl_up1(Rr);  // lane 0 of a segment takes the lane below's value and leaves it unused
-    if (ll >= 1 && live) face_flux<MHD, R, AX>(a, Rl, L, a.ce.at(idx[0], idx[1], idx[2]));
+    if (ll >= 1 && live) face_flux<MHD, R, AX, RS>(a, Rl, L, a.ce.at(idx[0], idx[1], idx[2]));
 }
 // Contiguous axis, streamed: the cells to rebuild, lo-1 .. hi-1 of every
 // line (line after line, which is also their order in memory when the range
@@ -1169,7 +1182,7 @@ __device__ __forceinline__ void sweep_wave_body(const SweepArgs& a, long seg_id,
 // lanes form a face except at line starts, where fixed segments of 63 faces
 // per line (9 wavefronts for the 517 faces of a 512^3 predictor line) left a
 // tenth of the lanes idle.
-template <int D, bool MHD, class R, int AX, bool FINAL>
+template <int D, bool MHD, class R, int AX, bool FINAL, class RS = R>
 __device__ __forceinline__ void sweep_stream_body(const SweepArgs& a, int w, int lane) {
     static_assert(AX == D - 1, "contiguous axis");
     const int len = a.hi[AX] - a.lo[AX];
@@ -1187,18 +1200,123 @@ __device__ __forceinline__ void sweep_stream_body(const SweepArgs& a, int w, int
     if (live) cell_states<D, MHD, R, AX, FINAL>(a, idx[0], idx[1], idx[2], L, Rr, &wc);
     if constexpr (eref_in_sweep<D, MHD, FINAL, AX>()) store_eref(a, live, idx, wc);
     const P<R> Rl = shfl_up1(Rr);  // lane 0 takes the lane below's value and leaves it unused
-    if (lane >= 1 && live && c >= 1) face_flux<MHD, R, AX>(a, Rl, L, a.ce.at(idx[0], idx[1], idx[2]));
+    if (lane >= 1 && live && c >= 1) face_flux<MHD, R, AX, RS>(a, Rl, L, a.ce.at(idx[0], idx[1], idx[2]));
 }
 // Occupancy floor of the contiguous-axis sweeps: the FP64 ones need 176
 // registers, 8 short of three waves per SIMD; at three they spill 12 bytes
 // per lane.  1 = the compiler's choice.
 template <class R> constexpr int wave_min_waves() { return DG_SWEEP_WAVES == 0 && sizeof(R) == 8 ? 3 : 1; }
-template <int D, bool MHD, class R, int AX, bool FINAL>
+template <int D, bool MHD, class R, int AX, bool FINAL, class RS>
 KS __attribute__((amdgpu_waves_per_eu(wave_min_waves<R>()))) __global__ void k_sweep_wave(SweepArgs a) {
     if (stopped(a.ts)) return;
     // the wavefront index is uniform: keep it in a scalar register
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    sweep_stream_body<D, MHD, R, AX, FINAL>(a, (int)block_xcd() * (int)(blockDim.x >> 6) + w, threadIdx.x & 63);
+    sweep_stream_body<D, MHD, R, AX, FINAL, RS>(a, (int)block_xcd() * (int)(blockDim.x >> 6) + w, threadIdx.x & 63);
+}
+
+// ================================================== 3D hydro corner sweeps
+// computeCTUFlux_X/Y/Z (CTU.cpp:306-370) of one axis, both of its corner
+// fluxes at once: the fluxes along AX between half states corrected by a third
+// of the flux difference of one transverse axis T1 (into Fo) and of the other,
+// T2 (into Fo2).  The half states are rebuilt in registers from the cells, as
+// in the sweeps above, and corrected and solved in FP64 in both forms.  The
+// half states as arrays (six of them, written once, read by six corner passes
+// and rewritten by six correction passes) cost 420 field accesses a cell where
+// this takes 190: 150 x 128 x 170 FP64 2.5 -> @@ ms a step.
+template <class R, int AX>
+__device__ __forceinline__ void corner_states(const SweepArgs& a, const int* idx, const P<R>& wl, const P<R>& wc, const P<R>& wr,
+                                              P<double>& L1, P<double>& R1, P<double>& L2, P<double>& R2) {
+    constexpr int T1 = AX == 0 ? 1 : 0, T2 = AX == 2 ? 1 : 2;
+    const Ext& ce = a.ce;
+    P<R> L, Rr;
+    cell_states_from<3, false, R, AX, false>(a, idx[0], idx[1], idx[2], wl, wc, wr, L, Rr);
+    const P<double> l = p_wide(L), r = p_wide(Rr);
+    const U<double> ul = cons<false>(l, a.ph), ur = cons<false>(r, a.ph);
+    const long m = ce.at(idx[0], idx[1], idx[2]);
+    L1 = L2 = l;
+    R1 = R2 = r;
+    if (idx[T1] >= 0 && idx[T1] < ce.n[T1]) {
+        const U<double> t = umul<false>(usub<false>(load_u(a.Fp[T1], m + ce.s[T1], false), load_u(a.Fp[T1], m, false)), dts(a.ts, T1) / 3.0);
+        L1 = prim<false>(usub<false>(ul, t), a.ph);
+        R1 = prim<false>(usub<false>(ur, t), a.ph);
+    }
+    if (idx[T2] >= 0 && idx[T2] < ce.n[T2]) {
+        const U<double> t = umul<false>(usub<false>(load_u(a.Fp[T2], m + ce.s[T2], false), load_u(a.Fp[T2], m, false)), dts(a.ts, T2) / 3.0);
+        L2 = prim<false>(usub<false>(ul, t), a.ph);
+        R2 = prim<false>(usub<false>(ur, t), a.ph);
+    }
+}
+template <int AX>
+__device__ __forceinline__ void corner_flux(const SweepArgs& a, P<double> l, P<double> r, const int* idx, int t, const FSoa& out, int stage) {
+    if (idx[t] < 0 || idx[t] >= a.ce.n[t]) return;
+    if (AX == 1) { l = swapXY(l); r = swapXY(r); }
+    if (AX == 2) { l = swapXZ(l); r = swapXZ(r); }
+    int fail = RF_OK;
+    U<double> f = riemann_x<false, double>(l, r, a.dt_d(AX), a.ph, &fail);
+    if (fail) {
+        // the reference walks these loops with the flux axis innermost
+        const int g = a.ce.g;
+        constexpr int o0 = AX == 0 ? 1 : 0, o1 = AX == 2 ? 1 : 2;
+        unsigned long long seq = ((unsigned long long)(idx[o0] + g) * 65536ull + (unsigned long long)(idx[o1] + g)) * 65536ull +
+                                 (unsigned long long)(idx[AX] + g);
+        report(a.err, stage, seq, fail == RF_BAD_INPUT ? E_RIEMANN_INPUT : E_RIEMANN_SOLUTION);
+    }
+    if (AX == 1) f = swapXY(f);
+    if (AX == 2) f = swapXZ(f);
+    store_u<double>(out, a.ce.at(idx[0], idx[1], idx[2]), f, false);
+}
+template <int AX>
+__device__ __forceinline__ void corner_fluxes(const SweepArgs& a, const P<double>& l1, const P<double>& r1, const P<double>& l2,
+                                              const P<double>& r2, const int* idx) {
+    constexpr int T1 = AX == 0 ? 1 : 0, T2 = AX == 2 ? 1 : 2;
+    corner_flux<AX>(a, l1, r1, idx, T1, a.Fo, a.stage & 255);
+    corner_flux<AX>(a, l2, r2, idx, T2, a.Fo2, a.stage >> 8);
+}
+// Strided axes: a walker of a.chunk faces per thread (sweep_march_body).
+template <class R, int AX> KS __global__ void k_corner_march(SweepArgs a) {
+    if (stopped(a.ts)) return;
+    constexpr int T0 = AX == 0 ? 1 : 0;
+    const long t = tid_xcd(), n1 = a.hi[2] - a.lo[2], n0 = a.hi[T0] - a.lo[T0];
+    const int len = a.hi[AX] - a.lo[AX], nch = (len + a.chunk - 1) / a.chunk;
+    if (t >= (long)nch * n0 * n1) return;
+    int idx[3];
+    idx[2] = a.lo[2] + (int)(t % n1);
+    const long r = t / n1;
+    idx[T0] = a.lo[T0] + (int)(r % n0);
+    const int f0 = a.lo[AX] + (int)(r / n0) * a.chunk, f1 = min(a.hi[AX], f0 + a.chunk);
+    const long s = a.ce.s[AX];
+    idx[AX] = f0 - 1;
+    long m = a.ce.at(idx[0], idx[1], idx[2]);
+    P<double> p1 = pzero<double>(), p2 = pzero<double>();
+    // cells f0 - 2 .. f1 exist: faces [0, n], two ghosts
+    P<double> nxt = load_p<double>(a.W, m + s, false);
+    for (int f = f0 - 1; f < f1; f++) {
+        idx[AX] = f;
+        P<double> L1, R1, L2, R2;
+        corner_states<R, AX>(a, idx, load_p<R>(a.W, m - s, false), load_p<R>(a.W, m, false), p_cast<R>(nxt), L1, R1, L2, R2);
+        if (f + 1 < f1) nxt = load_p<double>(a.W, m + 2 * s, false);
+        if (f >= f0) corner_fluxes<AX>(a, p1, L1, p2, L2, idx);
+        p1 = R1;
+        p2 = R2;
+        m += s;
+    }
+}
+// Contiguous axis: the lines' cells streamed (sweep_stream_body).
+template <class R> KS __global__ void k_corner_wave(SweepArgs a) {
+    if (stopped(a.ts)) return;
+    const int w = (int)block_xcd() * (int)(blockDim.x >> 6) + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, cells = a.hi[2] - a.lo[2] + 1, n1 = a.hi[1] - a.lo[1], n0 = a.hi[0] - a.lo[0];
+    const unsigned g = 63u * (unsigned)w + (unsigned)lane;
+    const bool live = g < (unsigned)(n0 * n1 * cells);
+    const unsigned line = g / (unsigned)cells, c = g - line * (unsigned)cells;
+    const int idx[3] = {a.lo[0] + (int)(line / (unsigned)n1), a.lo[1] + (int)(line % (unsigned)n1), a.lo[2] - 1 + (int)c};
+    P<double> L1 = pzero<double>(), R1 = L1, L2 = L1, R2 = L1;
+    if (live) {
+        const long m = a.ce.at(idx[0], idx[1], idx[2]);
+        corner_states<R, 2>(a, idx, load_p<R>(a.W, m - 1, false), load_p<R>(a.W, m, false), load_p<R>(a.W, m + 1, false), L1, R1, L2, R2);
+    }
+    const P<double> l1 = shfl_up1(R1), l2 = shfl_up1(R2);
+    if (lane >= 1 && live && c >= 1) corner_fluxes<2>(a, l1, L1, l2, L2, idx);
 }
 
 // ===================================================== CTU hydro (2D/3D)
@@ -1948,7 +2066,7 @@ static long march_chunk(long faces, bool fp64) {
 }
 
 // One sweep launch for axis AX over the face box b.
-template <int D, bool MHD, class R, bool FINAL, int AX>
+template <int D, bool MHD, class R, bool FINAL, int AX, class RS>
 static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, hipStream_t s) {
     SweepArgs a{};
     a.W = c.W;
@@ -1970,7 +2088,7 @@ static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, 
         const long cells = ntrans * (len + 1);
         const long waves = cells > 1 ? (cells - 1 + 62) / 63 : 1;
         a.chunk = 63;
-        hipLaunchKernelGGL((k_sweep_wave<D, MHD, R, AX, FINAL>), dim3(blocks(waves * 64)), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_sweep_wave<D, MHD, R, AX, FINAL, RS>), dim3(blocks(waves * 64)), dim3(256), 0, s, a);
     } else {
         const long chunk0 = march_chunk(len * ntrans, sizeof(R) == 8);
         long chunk = c.march_chunk > 0 ? c.march_chunk : chunk0;
@@ -1983,23 +2101,70 @@ static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, 
                 return;
             }
         }
-        hipLaunchKernelGGL((k_sweep_march<D, MHD, R, AX, FINAL>), dim3(blocks(nch * ntrans)), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_sweep_march<D, MHD, R, AX, FINAL, RS>), dim3(blocks(nch * ntrans)), dim3(256), 0, s, a);
     }
 }
-template <int D, bool MHD, class R, bool FINAL>
+template <int D, bool MHD, class R, bool FINAL, class RS = R>
 static void sweep(const StepCtx& c, int ax, const Box& b, const FSoa& out, int stage, hipStream_t s) {
-    if (ax == 0) sweep_t<D, MHD, R, FINAL, 0>(c, b, out, stage, s);
-    else if (ax == 1) { if constexpr (D >= 2) sweep_t<D, MHD, R, FINAL, 1>(c, b, out, stage, s); }
-    else { if constexpr (D >= 3) sweep_t<D, MHD, R, FINAL, 2>(c, b, out, stage, s); }
+    if (ax == 0) sweep_t<D, MHD, R, FINAL, 0, RS>(c, b, out, stage, s);
+    else if (ax == 1) { if constexpr (D >= 2) sweep_t<D, MHD, R, FINAL, 1, RS>(c, b, out, stage, s); }
+    else { if constexpr (D >= 3) sweep_t<D, MHD, R, FINAL, 2, RS>(c, b, out, stage, s); }
 }
 
-// The step with fused sweeps (MHD 2D/3D, hydro 2D): predictor fluxes ->
+// 3D hydro CTU, 12 solves (CTU.cpp:222-261), half states rebuilt in each
+// sweep: three predictor sweeps, three corner sweeps of two fluxes each, three
+// corrector sweeps.  The corner flux along axis a corrected by axis t is
+// c.T[corner(a, t)].  Predictor and corner fluxes are solved in FP64 in both
+// forms; the corrector's replace the predictor's, which nothing reads then.
+static int corner(int a, int t) { return 2 * a + (t == (a == 2 ? 1 : 2)); }
+template <class R>
+static void hydro3_fluxes(const StepCtx& c, hipStream_t s) {
+    const Ext& ce = c.ce;
+    for (int ax = 0; ax < 3; ax++) {
+        sweep<3, false, R, false, double>(c, ax, face_box(3, ce, ax, 0, 0, -1, 1), fs(c.F[ax]), ST_PRED_X + ax, s);
+        mark(c, K_PRED_X + ax);
+    }
+    static const int order[3][3] = {{0, 2, 0}, {4, 0, 1}, {5, 3, 0}};  // the reference's position of the flux along a corrected by t
+    for (int ax = 0; ax < 3; ax++) {
+        const int t1 = ax == 0 ? 1 : 0, t2 = ax == 2 ? 1 : 2;
+        SweepArgs a{};
+        a.W = c.W;
+        const Box b = face_box(3, ce, ax, 0, 0, -1, 1);
+        for (int q = 0; q < 3; q++) { a.Fp[q] = fs(c.F[q]); a.lo[q] = b.lo[q]; a.hi[q] = b.hi[q]; }
+        a.Fo = fs(c.T[corner(ax, t1)]); a.Fo2 = fs(c.T[corner(ax, t2)]);
+        a.ce = ce; a.fe = c.fe; a.ph = c.ph; a.err = c.err; a.ts = &c.ctl->t; a.half = 0;
+        a.stage = (ST_CTU_F0 + order[ax][t1]) | (ST_CTU_F0 + order[ax][t2]) << 8;
+        const long len = b.hi[ax] - b.lo[ax], ntrans = b.count() / len;
+        if (ax == 2) {
+            const long waves = (ntrans * (len + 1) - 1 + 62) / 63;
+            hipLaunchKernelGGL((k_corner_wave<R>), dim3(blocks(waves * 64)), dim3(256), 0, s, a);
+        } else {
+            a.chunk = (int)std::min(len, c.march_chunk > 0 ? (long)c.march_chunk : march_chunk(len * ntrans, true));
+            const long nch = (len + a.chunk - 1) / a.chunk;
+            if (ax == 0) hipLaunchKernelGGL((k_corner_march<R, 0>), dim3(blocks(nch * ntrans)), dim3(256), 0, s, a);
+            else hipLaunchKernelGGL((k_corner_march<R, 1>), dim3(blocks(nch * ntrans)), dim3(256), 0, s, a);
+        }
+        mark(c, K_CTU);
+    }
+    for (int ax = 0; ax < 3; ax++) {
+        const int t1 = ax == 0 ? 1 : 0, t2 = ax == 2 ? 1 : 2;
+        StepCtx cc = c;
+        cc.Fp[0] = c.T[corner(t1, t2)];
+        cc.Fp[1] = c.T[corner(t2, t1)];
+        sweep<3, false, R, true>(cc, ax, face_box(3, ce, ax, 0, 0, 0, 0), fs(c.F[ax]), ST_FLUX_X + ax, s);
+        mark(c, K_FLUX_X + ax);
+    }
+}
+
+// The step with fused sweeps (2D, 3D): predictor fluxes ->
 // [MHD: corner EMF, half-step faces, half-step reference EMF] -> corrector
 // fluxes (CTU correction inside) -> [MHD: EMF, Faraday] -> apply.
 template <int D, bool MHD, class R>
 static void step_fused(const StepCtx& c, hipStream_t s) {
     const Ext& ce = c.ce;
-    if (c.ctu) {
+    if constexpr (D == 3 && !MHD) {
+        if (c.ctu) hydro3_fluxes<R>(c, s);
+    } else if (c.ctu) {
         for (int ax = 0; ax < D; ax++) {
             Box b = MHD ? face_box(D, ce, ax, -1, 1, -2, 2) : face_box(D, ce, ax, 0, 0, -1, 1);
             sweep<D, MHD, R, false>(c, ax, b, fs(c.Fp[ax]), ST_PRED_X + ax, s);
@@ -2030,7 +2195,7 @@ static void step_fused(const StepCtx& c, hipStream_t s) {
             mark(c, K_WHALF);
         }
     }
-    for (int ax = 0; ax < D; ax++) {
+    for (int ax = 0; ax < D && !(D == 3 && !MHD && c.ctu); ax++) {
         Box b = MHD ? face_box(D, ce, ax, 0, 0, -1, 1) : face_box(D, ce, ax, 0, 0, 0, 0);
         if (c.ctu) sweep<D, MHD, R, true>(c, ax, b, fs(c.F[ax]), ST_FLUX_X + ax, s);
         else sweep<D, MHD, R, false>(c, ax, b, fs(c.F[ax]), ST_FLUX_X + ax, s);
@@ -2056,7 +2221,7 @@ static void step_fused(const StepCtx& c, hipStream_t s) {
 
 template <int D, bool MHD, class R>
 static void step_t(const StepCtx& c, hipStream_t s) {
-    if constexpr ((MHD && D >= 2) || (!MHD && D == 2)) {
+    if constexpr (D >= 2) {
         if (c.fused) {
             step_fused<D, MHD, R>(c, s);
             return;

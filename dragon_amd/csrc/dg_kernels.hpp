@@ -60,7 +60,7 @@ struct StepCtx {
     Soa HS[6];            // xL, xR, yL, yR, zL, zR
     Soa F[3];             // corrector (final) fluxes; reference-structured path: both
     Soa Fp[3];            // predictor fluxes of the fused path
-    Soa T[5];             // 3D hydro corner fluxes
+    Soa T[6];             // 3D hydro corner fluxes (reference-structured path: five)
     double* E0[3];        // corner EMF (predictor, then final)
     double* Eh[3];        // half-step reference EMF
     unsigned long long* err;
