@@ -349,15 +349,15 @@ __host__ __device__ inline BCShell face_shell(const Ext& ce, int dim) {
     return BCShell{dim, {ce.n[0] - 1, ce.n[1] - 1, ce.n[2] - 1}, ce.g + 1, ce.g + 1};
 }
 // Fields [f0, f1) of the t-th ghost cell.
-__device__ __forceinline__ void bc_list_cell(const BCListArgs& a, const Ext& ce, unsigned t, int f0, int f1) {
+__device__ __forceinline__ void bc_list_cell(const BCPass* ps, int np, int dim, const Soa& W, const Ext& ce, unsigned t, int f0, int f1) {
     int i, j, k;
-    cell_shell(ce, a.dim).point(t, i, j, k);
+    cell_shell(ce, dim).point(t, i, j, k);
     const long dst = ce.at(i, j, k);
     unsigned neg = 0, in_lo = 0, in_hi = 0;  // per field: sign change, inflow through a low / high face dropped
     bool hit = false;
     int fixed = -1;  // the pass whose state the cell takes
-    for (int q = a.npass - 1; q >= 0 && fixed < 0; q--) {
-        const BCPass& p = a.p[q];
+    for (int q = np - 1; q >= 0 && fixed < 0; q--) {
+        const BCPass& p = ps[q];
         const int ax = p.axis, n = ax == 0 ? ce.n[0] : ax == 1 ? ce.n[1] : ce.n[2], x = ax == 0 ? i : ax == 1 ? j : k;
         if (p.side == 0 ? x >= 0 : x < n) continue;
         hit = true;
@@ -380,34 +380,35 @@ __device__ __forceinline__ void bc_list_cell(const BCListArgs& a, const Ext& ce,
     auto finish = [&](int f, double v) {
         if (neg >> f & 1) v *= -1;
         if ((in_lo >> f & 1 && v > 0) || (in_hi >> f & 1 && v < 0)) v = 0;
-        a.W(f, dst) = v;
+        W(f, dst) = v;
     };
     if (f1 - f0 == 1) {
-        finish(f0, fixed >= 0 ? a.p[fixed].st[f0] : a.W(f0, src));
+        finish(f0, fixed >= 0 ? ps[fixed].st[f0] : W(f0, src));
         return;
     }
     double v[8];  // read before any is written, so that the reads overlap
 #pragma unroll
     for (int f = 0; f < 8; f++)
-        if (f < f1) v[f] = fixed >= 0 ? a.p[fixed].st[f] : a.W(f, src);
+        if (f < f1) v[f] = fixed >= 0 ? ps[fixed].st[f] : W(f, src);
 #pragma unroll
     for (int f = 0; f < 8; f++)
         if (f < f1) finish(f, v[f]);
 }
-__device__ __forceinline__ void bc_list_face(const BCListArgs& a, const Ext& ce, const Ext& fe, unsigned t, int c) {
+__device__ __forceinline__ void bc_list_face(const BCPass* ps, int np, int dim, double* const Bc[3], const Ext& ce, const Ext& fe, unsigned t,
+                                             int c) {
     int i, j, k;
-    face_shell(ce, a.dim).point(t, i, j, k);
+    face_shell(ce, dim).point(t, i, j, k);
     i++;
-    if (a.dim >= 2) j++;
-    if (a.dim >= 3) k++;
-    double* const B = c == 0 ? a.B[0] : c == 1 ? a.B[1] : a.B[2];
+    if (dim >= 2) j++;
+    if (dim >= 3) k++;
+    double* const B = c == 0 ? Bc[0] : c == 1 ? Bc[1] : Bc[2];
     const long dst = fe.at(i, j, k);
     const int ng = ce.g;
     double v = 0, sgn = 1;
     int ext = 0, exg = 0;  // extrapolation of the normal component: side + 1, faces beyond the last one kept
     bool hit = false, fixed = false;
-    for (int q = a.npass - 1; q >= 0 && !fixed; q--) {
-        const BCPass& p = a.p[q];
+    for (int q = np - 1; q >= 0 && !fixed; q--) {
+        const BCPass& p = ps[q];
         const int ax = p.axis, n = ax == 0 ? ce.n[0] : ax == 1 ? ce.n[1] : ce.n[2], x = ax == 0 ? i : ax == 1 ? j : k;
         const bool normal = c == ax;
         int y = x;
@@ -465,17 +466,17 @@ __device__ __forceinline__ void bc_list_face(const BCListArgs& a, const Ext& ce,
 template <bool WHOLE>
 __device__ __forceinline__ void bc_list_body(const BCListArgs& a, const Ext& ce, const Ext& fe, unsigned t) {
     if (WHOLE) {
-        if (t < a.ncell) bc_list_cell(a, ce, t, 0, a.nf);
+        if (t < a.ncell) bc_list_cell(a.p, a.npass, a.dim, a.W, ce, t, 0, a.nf);
         else if (t - a.ncell < a.nface)
-            for (int c = 0; c < 3; c++) bc_list_face(a, ce, fe, t - a.ncell, c);
+            for (int c = 0; c < 3; c++) bc_list_face(a.p, a.npass, a.dim, a.B, ce, fe, t - a.ncell, c);
         return;
     }
     const unsigned cells = a.ncell * (unsigned)a.nf;
     if (t < cells) {
         const int f = (int)(t / a.ncell);
-        bc_list_cell(a, ce, t % a.ncell, f, f + 1);
+        bc_list_cell(a.p, a.npass, a.dim, a.W, ce, t % a.ncell, f, f + 1);
     } else if (t - cells < 3 * a.nface) {
-        bc_list_face(a, ce, fe, (t - cells) % a.nface, (int)((t - cells) / a.nface));
+        bc_list_face(a.p, a.npass, a.dim, a.B, ce, fe, (t - cells) % a.nface, (int)((t - cells) / a.nface));
     }
 }
 template <bool WHOLE>
@@ -2427,9 +2428,7 @@ __device__ __forceinline__ PatchView patch_view(const BatchArgs& A, int p) {
     if (!A.active[p]) return;                   \
     const long t = (long)bt.first[bx] + threadIdx.x;
 
-KB __global__ void kb_begin(BatchArgs A) {
-    const int p = (int)tid();
-    if (p >= A.npatch) return;
+__device__ __forceinline__ void batch_begin(const BatchArgs& A, int p) {
     const bool on = A.status[p] == 0 && (A.cls_filter < 0 || A.P[p].cls == A.cls_filter);
     A.active[p] = on ? 1 : 0;
     if (on) {
@@ -2441,36 +2440,20 @@ KB __global__ void kb_begin(BatchArgs A) {
         A.err[p] = ~0ull;
     }
 }
-// Boundary pass of every patch: both sides of one axis in one launch (they
-// touch disjoint ghost slabs for sides of 4 cells or more), in the pass
-// order of a list element's apply.
-template <bool FACES, int AX>
-KB __global__ void kb_bc(BatchArgs A, BlockTable bt) {
+KB __global__ void kb_begin(BatchArgs A) {
+    const int p = (int)tid();
+    if (p < A.npatch) batch_begin(A, p);
+}
+// The boundary pass of every patch in one launch (bc_list_cell / _face, a
+// thread per ghost cell and field or boundary face and component): the two
+// sides of x, then of y, outflow or periodic.  (Four launches of one pass
+// each took 43 us of the 1.05 ms step of 96 patches.)
+KB __global__ void kb_bc(BatchArgs A, BlockTable bt, BCPasses bc) {
     BATCH_ITEM(bt)
     const PatchView v = patch_view(A, p);
-    constexpr int G = 3;
-    const long cnt = v.ce.n[AX == 0 ? 1 : 0] + 2 * G + (FACES ? 1 : 0);
-    const bool periodic = A.bc_kind == 1;
-    if (t >= (!FACES && AX == 1 ? 2 * G : periodic ? 1 : 2) * cnt) return;
-    BCArgs b{};
-    b.W = v.W;
-    for (int c = 0; c < 3; c++) b.B[c] = v.B[c];
-    b.ce = v.ce; b.fe = v.fe; b.dim = 2; b.nf = 8; b.kind = A.bc_kind; b.corners = 1; b.gated = 0;
-    b.axis = AX;
-    b.lo[0] = -G; b.hi[0] = (int)(-G + cnt);
-    b.lo[1] = 0; b.hi[1] = 1;
-    if constexpr (!FACES && AX == 1) {
-        // The cell pass along y (the contiguous axis), one item per ghost
-        // cell, both sides: patches hold at least 4 cells along y, so every
-        // cell a ghost reads is interior and the g loop has no order to keep.
-        const int side = (int)(t / (cnt * G));
-        const long r = t % (cnt * G);
-        bc_cell(b, b.lo[0] + (int)(r / G), 0, (int)(r % G) + 1, side);
-        return;
-    }
-    b.side = periodic ? 2 : (int)(t / cnt);
-    if (FACES) bc_faces_body(b, t % cnt);
-    else bc_cells_body(b, t % cnt);
+    const unsigned nc = cell_shell(v.ce, 2).count(), nf = face_shell(v.ce, 2).count(), u = (unsigned)t;
+    if (u < 8 * nc) bc_list_cell(bc.p, 4, 2, v.W, v.ce, u % nc, (int)(u / nc), (int)(u / nc) + 1);
+    else if (u - 8 * nc < 3 * nf) bc_list_face(bc.p, 4, 2, v.B, v.ce, v.fe, (u - 8 * nc) % nf, (int)((u - 8 * nc) / nf));
 }
 KB __global__ void kb_init_B(BatchArgs A, BlockTable bt) {
     BATCH_ITEM(bt)
@@ -2485,12 +2468,18 @@ KB __global__ void kb_init_B(BatchArgs A, BlockTable bt) {
 KB __global__ void kb_cfl(BatchArgs A, BlockTable bt) {
     BATCH_ITEM(bt)
     const PatchView v = patch_view(A, p);
-    const long ny2 = v.ce.n[1] + 2;
     double m = 0;
-    const int i = (int)(t / ny2) - 1, j = (int)(t % ny2) - 1;
-    const bool interior = i >= 0 && i < v.ce.n[0] && j >= 0 && j < v.ce.n[1];
-    if (t < (long)(v.ce.n[0] + 2) * ny2 && !(interior && A.cfl_ok[p]))
+    int i, j, k;
+    if (A.cfl_ok[p]) {  // the interior's maximum is known: the one-cell shell, densely, and most workgroups have nothing
+        const BCShell sh{2, {v.ce.n[0], v.ce.n[1], 1}, 1, 1};
+        if (t - threadIdx.x >= sh.count()) return;  // the whole workgroup
+        if (t < sh.count()) {
+            sh.point((unsigned)t, i, j, k);
+            m = dmax(m, cfl_speed_at<2, true>(v.W, v.ce, i, j, 0, A.ph, A.cfl_mode, v.dx, v.dy, 1.0));
+        }
+    } else if (make_box(2, -1, v.ce.n[0] + 1, -1, v.ce.n[1] + 1).point(t, i, j, k)) {
         m = dmax(m, cfl_speed_at<2, true>(v.W, v.ce, i, j, 0, A.ph, A.cfl_mode, v.dx, v.dy, 1.0));
+    }
     for (int off = 32; off > 0; off >>= 1) m = dmax(m, __shfl_xor(m, off));
     __shared__ double wmax[BATCH_THREADS / 64];
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
@@ -2614,9 +2603,8 @@ KB __global__ void kb_apply(BatchArgs A, BlockTable bt) {
         if (b > 0) atomicMax(A.vnext + p, (unsigned long long)__double_as_longlong(b));
     }
 }
-KB __global__ void kb_commit(BatchArgs A) {
-    const int p = (int)tid();
-    if (p >= A.npatch || !A.active[p]) return;
+__device__ __forceinline__ void batch_commit(const BatchArgs& A, int p) {
+    if (!A.active[p]) return;
     // vnext describes the state only when the attempt was committed
     A.cfl_ok[p] = A.commit && A.err[p] == ~0ull ? 1 : 0;
     if (!A.commit) return;
@@ -2631,16 +2619,21 @@ KB __global__ void kb_commit(BatchArgs A) {
         if (0.5 * A.dt[p] < A.tol) A.status[p] = BATCH_ERR_DT;  // "Timestep has fallen below minimum"
     }
 }
+// The end of a step and, inside a sequence of steps, the beginning of the next.
+KB __global__ void kb_commit(BatchArgs A, int next) {
+    const int p = (int)tid();
+    if (p >= A.npatch) return;
+    batch_commit(A, p);
+    if (next) batch_begin(A, p);
+}
 
-void launch_batch_step(const BatchArgs& a, const BlockTable* bt, bool init_only, hipStream_t s) {
+// first / last: of a sequence of steps (the commit between two of them begins the next).
+void launch_batch_step(const BatchArgs& a, const BlockTable* bt, bool init_only, bool first, bool last, hipStream_t s) {
     const dim3 T(BATCH_THREADS);
     const unsigned pb = blocks(a.npatch);
     auto grid = [&](int k) { return dim3(bt[k].nblocks); };
-    hipLaunchKernelGGL(kb_begin, dim3(pb), T, 0, s, a);
-    hipLaunchKernelGGL((kb_bc<false, 0>), grid(BK_BCC_X), T, 0, s, a, bt[BK_BCC_X]);
-    hipLaunchKernelGGL((kb_bc<false, 1>), grid(BK_BCC_Y), T, 0, s, a, bt[BK_BCC_Y]);
-    hipLaunchKernelGGL((kb_bc<true, 0>), grid(BK_BCF_X), T, 0, s, a, bt[BK_BCF_X]);
-    hipLaunchKernelGGL((kb_bc<true, 1>), grid(BK_BCF_Y), T, 0, s, a, bt[BK_BCF_Y]);
+    if (first) hipLaunchKernelGGL(kb_begin, dim3(pb), T, 0, s, a);
+    hipLaunchKernelGGL(kb_bc, grid(BK_BC), T, 0, s, a, bt[BK_BC], a.bc);
     if (init_only) {
         hipLaunchKernelGGL(kb_init_B, grid(BK_CELLS), T, 0, s, a, bt[BK_CELLS]);
         return;
@@ -2657,7 +2650,7 @@ void launch_batch_step(const BatchArgs& a, const BlockTable* bt, bool init_only,
     hipLaunchKernelGGL((kb_emf<false>), grid(BK_EDGES), T, 0, s, a, bt[BK_EDGES]);
     hipLaunchKernelGGL((kb_faraday<false>), grid(BK_FACES), T, 0, s, a, bt[BK_FACES]);
     hipLaunchKernelGGL(kb_apply, grid(BK_CELLS), T, 0, s, a, bt[BK_CELLS]);
-    hipLaunchKernelGGL(kb_commit, dim3(pb), T, 0, s, a);
+    hipLaunchKernelGGL(kb_commit, dim3(pb), T, 0, s, a, last ? 0 : 1);
 }
 
 // ====================================================== Strang split step

@@ -114,7 +114,7 @@ enum { BATCH_CLASSES = 4, BATCH_THREADS = 256 };
 enum { BATCH_ERR_CFL = 5, BATCH_ERR_DT = 6 };
 // work kinds of a batched step (items per patch in dg_api.hip: batch_items)
 enum BatchKind {
-    BK_BCC_X, BK_BCC_Y, BK_BCF_X, BK_BCF_Y,  // boundary passes: cells / faces, x then y, both sides
+    BK_BC,                                   // boundary: ghost cells x 8 fields, then boundary faces x 3 components
     BK_CELLS1,                               // cells [-1, n+1)^2: CFL, half-step state
     BK_PRED_X, BK_PRED_Y,                    // predictor sweeps (x: faces-per-thread chunks; y: 63 faces per wavefront)
     BK_EDGES_P,                              // edges [-1, n+2)^2: predictor EMF
@@ -128,6 +128,9 @@ struct BlockTable {
     const int* patch;   // per workgroup: patch
     const int* first;   // per workgroup: first work item (a multiple of BATCH_THREADS)
     unsigned nblocks;
+};
+struct BCPasses {
+    BCPass p[4];
 };
 struct BatchArgs {
     const PatchDesc* P;
@@ -154,7 +157,8 @@ struct BatchArgs {
     int* active;               // per patch: steps in this launch sequence
     Phys ph;
     double cfl_coeff, tol;
-    int cfl_mode, bc_kind;     // bc_kind: 0 outflow, 1 periodic (all faces, corner ghosts)
+    int cfl_mode;
+    BCPasses bc;               // outflow or periodic on every face, corner ghosts
     int chunk[BATCH_CLASSES];  // x-sweep faces per thread, per size class
     int ysw[BATCH_CLASSES];    // y-sweep segment width in lanes (64, 32, 16: 63, 31, 15 faces), per size class
     int commit;                // 0: run the step, keep every patch's state and counters (tuning)
@@ -168,7 +172,7 @@ struct BatchArgs {
 // pressure recovery and CT).  Separate namespaces keep every kernel symbol of
 // one build out of the other.
 #define DG_LAUNCH_INTERFACE                                                                                     \
-    void launch_batch_step(const BatchArgs& a, const BlockTable* bt, bool init_only, hipStream_t s);           \
+    void launch_batch_step(const BatchArgs& a, const BlockTable* bt, bool init_only, bool first, bool last, hipStream_t s); \
     void launch_step(const StepCtx& c, hipStream_t s);                                                          \
     void launch_split_axis(const StepCtx& c, int ax, Soa in, Soa out, hipStream_t s);  /* one split sweep (hydro) */ \
     void launch_bc(const BCArgs& a, bool faces, hipStream_t s);                                                 \
