@@ -41,7 +41,7 @@ struct dg_grid {
     int sweep_step = 0;         // split step: rotation of the sweep order (Grid.hpp:93, 135)
     double *E0 = nullptr, *Eh = nullptr;
     double* cflpart = nullptr;  // per-block CFL maxima of the committed state, written by the apply pass
-    long ncflpart = 0;
+    long ncflpart = 0;          // maxima the last step left
     bool cfl_cached = false;    // cflpart describes the current W (set by a committed step)
     unsigned long long* dev_words = nullptr;   // [1] CFL max bits, [2..3] diagnostics
     unsigned long long* host_words = nullptr;  // pinned mirror
@@ -227,8 +227,9 @@ int dg_create(const dg_desc* desc, dg_grid** out) {
     if (faces) ok = ok && alloc(&g->B, 3 * nfc) && alloc(&g->Bn, 3 * nfc) && alloc(&g->Bh, 3 * nfc) && alloc(&g->E0, 3 * nfc) &&
                     alloc(&g->Eh, 3 * nfc);
     if (d.dim >= 2) {
-        g->ncflpart = ((long)nc + 255) / 256;
-        ok = ok && alloc(&g->cflpart, g->ncflpart);
+        // one per workgroup of the pass that writes the next state
+        const long parts = d.dim == 2 ? ct_tiles(d.nx + 1 + 2 * gh, d.ny + 1 + 2 * gh) : 0;
+        ok = ok && alloc(&g->cflpart, std::max(parts, (nc + 255) / 256));
     }
     ok = ok && hipMalloc((void**)&g->dev_words, 4 * sizeof(unsigned long long)) == hipSuccess;
     ok = ok && hipHostMalloc((void**)&g->host_words, 4 * sizeof(unsigned long long), hipHostMallocDefault) == hipSuccess;
@@ -540,8 +541,7 @@ int dg_step(dg_grid* g, double dt, dg_status* st) {
     launch_ctl_set(c, dt, g->s);
     if (g->timing) HIPCHK(hipEventRecord(g->ev0, g->s));
     tm_record(g, -1);
-    if (c.mixed) p32::launch_step(c, g->s);
-    else p64::launch_step(c, g->s);
+    g->ncflpart = c.mixed ? p32::launch_step(c, g->s) : p64::launch_step(c, g->s);
     HIPCHK(hipGetLastError());
     if (g->timing) HIPCHK(hipEventRecord(g->ev1, g->s));
     HIPCHK(hipMemcpyAsync(&g->host_ctl->err, &g->ctl->err, sizeof(unsigned long long), hipMemcpyDeviceToHost, g->s));
@@ -660,8 +660,7 @@ static int advance_run(dg_grid* g, double left, int check_cfl, int n, int* done,
         if (!check_cfl) launch_ctl_next(c, g->s);
         else if (cached) launch_cfl_tail(c, g->ncflpart, nullptr, true, g->s);
         else launch_cfl(c, nullptr, true, g->s);
-        if (c.mixed) p32::launch_step(c, g->s);
-        else p64::launch_step(c, g->s);
+        g->ncflpart = c.mixed ? p32::launch_step(c, g->s) : p64::launch_step(c, g->s);
         cached = g->cflpart != nullptr;
         std::swap(g->W, g->Wn);
         if (g->B) std::swap(g->B, g->Bn);
@@ -1189,11 +1188,10 @@ static long batch_items(const dg_batch* b, const PatchDesc& q, int kind) {
         case BK_CELLS1: return (nx + 2) * (ny + 2);
         case BK_PRED_X: return chunked(nx + 3, ny + 4);
         case BK_PRED_Y: return segments(ny + 3, nx + 4);
-        case BK_EDGES_P: return (nx + 3) * (ny + 3);
-        case BK_FACES: return q.nfc;
+        case BK_EDGES: return 256 * ct_tiles(nx + 3, ny + 3);
+        case BK_FACES: return 256 * ct_tiles(nx + 7, ny + 7);
         case BK_FLUX_X: return chunked(nx + 1, ny + 2);
         case BK_FLUX_Y: return segments(ny + 1, nx + 2);
-        case BK_EDGES: return (nx + 1) * (ny + 1);
         default: return q.nc;  // BK_CELLS
     }
 }

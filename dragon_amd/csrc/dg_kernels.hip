@@ -767,13 +767,12 @@ struct SweepArgs {
 };
 // The MHD predictor sweep along the contiguous axis also writes each rebuilt
 // cell's reference EMF, cross(B, v) of the state it holds: its cells cover
-// the predictor EMF's ([-2, n+1] in every dimension). In the FP32 form the
-// EMF then reads 12 bytes per cell instead of B and v in FP64 (48 bytes), and
-// in 2D forms each cell's once instead of once per corner. The FP64 form does
-// this in 3D only (the EMF reads 24 bytes instead of 48); its cross product is
-// the one the EMF would form from the same W, so results are unchanged.
+// the predictor EMF's ([-2, n+1] in every dimension).  The EMF then reads 12
+// (FP32 form) or 24 bytes per cell instead of B and v in FP64 (48 bytes), and
+// in 2D forms each cell's once instead of once per corner.  The cross product
+// is the one the EMF would form from the same W, so results are unchanged.
 template <int D, bool MHD, bool FINAL, int AX> constexpr bool eref_in_sweep() {
-    return D >= 2 && AX == D - 1 && MHD && !FINAL && (sizeof(FT) == 4 || D == 3);
+    return D >= 2 && AX == D - 1 && MHD && !FINAL;
 }
 // From the cell state the sweep already holds in FP32.  A cell rebuilt by
 // two lanes (segment or wavefront overlaps) is written twice, with the same
@@ -1699,10 +1698,9 @@ __device__ __forceinline__ void whalf_body(const Soa& W, const FSoa& FX, const F
     if (D == 3) u = uadd<true>(u, umul<true>(usub<true>(load_u_nb<2>(FZ, m), load_u_nb<2>(FZ, m + ce.s[2])), hz));
     if (gate && stopped(gate)) return;
     if (!finite<true>(u)) report(err, ST_WHALF_NAN, (unsigned long long)m, E_NAN);
-    w = prim<true>(u, ph);
     double cbx, cby, cbz;
     cell_B(Bhx, Bhy, Bhz, fe, D, i, j, k, cbx, cby, cbz);
-    w = body_field(w, cbx, cby, cbz, ph);
+    w = body_field(prim<true>(u, ph), cbx, cby, cbz, ph);
     double ex, ey, ez;
     cross(w.Bx, w.By, w.Bz, w.vx, w.vy, w.vz, ex, ey, ez);
     const long e = fe.at(i, j, k);
@@ -1786,6 +1784,35 @@ KB __global__ void k_ctu_mhd(Soa W, const double* Bx, const double* By, const do
 }
 
 // ========================================================= apply + commit
+// A cell's conserved state plus its flux differences (applyFluxes).
+template <int D, bool MHD>
+__device__ __forceinline__ U<double> flux_update(const Soa& W, const FSoa& FX, const FSoa& FY, const FSoa& FZ, const Ext& ce, double dt_dx,
+                                                 double dt_dy, double dt_dz, const Phys& ph, long m) {
+    U<double> u = cons<MHD>(load_p<double>(W, m, MHD), ph);
+    if constexpr (MHD) {
+        u = uadd<true>(u, umul<true>(usub<true>(load_u_nb<0>(FX, m), load_u_nb<0>(FX, m + ce.s[0])), dt_dx));
+        if (D >= 2) u = uadd<true>(u, umul<true>(usub<true>(load_u_nb<1>(FY, m), load_u_nb<1>(FY, m + ce.s[1])), dt_dy));
+        if (D == 3) u = uadd<true>(u, umul<true>(usub<true>(load_u_nb<2>(FZ, m), load_u_nb<2>(FZ, m + ce.s[2])), dt_dz));
+    } else {
+        u = uadd<false>(u, umul<false>(usub<false>(load_u(FX, m, false), load_u(FX, m + ce.s[0], false)), dt_dx));
+        if (D >= 2) u = uadd<false>(u, umul<false>(usub<false>(load_u(FY, m, false), load_u(FY, m + ce.s[1], false)), dt_dy));
+        if (D == 3) u = uadd<false>(u, umul<false>(usub<false>(load_u(FZ, m, false), load_u(FZ, m + ce.s[2], false)), dt_dz));
+    }
+    return u;
+}
+// The end of a cell's update: conserved state u and cell B of the new faces to
+// the next primitive state, with the checks.  Returns the signal speed where
+// `cfl` is set.
+template <int D, bool MHD>
+__device__ __forceinline__ double apply_finish(const U<double>& u, const Soa& Wn, double cbx, double cby, double cbz, const Phys& ph,
+                                               unsigned long long* err, long m, bool cfl, int cfl_mode, double cdx, double cdy, double cdz) {
+    if (D >= 2 && !finite<MHD>(u)) report(err, ST_APPLY_NAN, (unsigned long long)m, E_NAN);
+    P<double> w = prim<MHD>(u, ph);
+    if (MHD && D >= 2) w = body_field(w, cbx, cby, cbz, ph);
+    if (!physical<MHD>(w)) report(err, ST_UNPHYSICAL, (unsigned long long)m, E_UNPHYSICAL);
+    store_p_nt(Wn, m, w, MHD);
+    return cfl ? dmax(0.0, cfl_speed_w<D, MHD>(w, ph, cfl_mode, cdx, cdy, cdz)) : 0.0;  // NaN never wins
+}
 // applyFluxes (Unsplit.cpp:256-288) + computeBodyFields with the new faces +
 // the physicality check (Unsplit.cpp:94-99, 188-195), writing the complete
 // next state: interior cells updated, ghost cells copied (the reference
@@ -1811,28 +1838,11 @@ __device__ __forceinline__ double apply_body(const Soa& W, const Soa& Wn, const 
         for (int f = 0; f < nf; f++) st_nt(Wn, f, m, W(f, m));
         return 0.0;
     }
-    P<double> w = load_p<double>(W, m, MHD);
-    U<double> u = cons<MHD>(w, ph);
-    if constexpr (MHD) {
-        u = uadd<true>(u, umul<true>(usub<true>(load_u_nb<0>(FX, m), load_u_nb<0>(FX, m + ce.s[0])), dt_dx));
-        if (D >= 2) u = uadd<true>(u, umul<true>(usub<true>(load_u_nb<1>(FY, m), load_u_nb<1>(FY, m + ce.s[1])), dt_dy));
-        if (D == 3) u = uadd<true>(u, umul<true>(usub<true>(load_u_nb<2>(FZ, m), load_u_nb<2>(FZ, m + ce.s[2])), dt_dz));
-    } else {
-        u = uadd<false>(u, umul<false>(usub<false>(load_u(FX, m, false), load_u(FX, m + ce.s[0], false)), dt_dx));
-        if (D >= 2) u = uadd<false>(u, umul<false>(usub<false>(load_u(FY, m, false), load_u(FY, m + ce.s[1], false)), dt_dy));
-        if (D == 3) u = uadd<false>(u, umul<false>(usub<false>(load_u(FZ, m, false), load_u(FZ, m + ce.s[2], false)), dt_dz));
-    }
+    const U<double> u = flux_update<D, MHD>(W, FX, FY, FZ, ce, dt_dx, dt_dy, dt_dz, ph, m);
     if (gate && stopped(gate)) return 0.0;
-    if (D >= 2 && !finite<MHD>(u)) report(err, ST_APPLY_NAN, (unsigned long long)m, E_NAN);
-    w = prim<MHD>(u, ph);
-    if (MHD && D >= 2) {
-        double cbx, cby, cbz;
-        cell_B(Bnx, Bny, Bnz, fe, D, i, j, k, cbx, cby, cbz);
-        w = body_field(w, cbx, cby, cbz, ph);
-    }
-    if (!physical<MHD>(w)) report(err, ST_UNPHYSICAL, (unsigned long long)m, E_UNPHYSICAL);
-    store_p_nt(Wn, m, w, MHD);
-    return cfl ? dmax(0.0, cfl_speed_w<D, MHD>(w, ph, cfl_mode, cdx, cdy, cdz)) : 0.0;  // NaN never wins
+    double cbx = 0, cby = 0, cbz = 0;
+    if (MHD && D >= 2) cell_B(Bnx, Bny, Bnz, fe, D, i, j, k, cbx, cby, cbz);
+    return apply_finish<D, MHD>(u, Wn, cbx, cby, cbz, ph, err, m, cfl, cfl_mode, cdx, cdy, cdz);
 }
 template <int D, bool MHD>
 KB __global__ void k_apply(Soa W, Soa Wn, FSoa FX, FSoa FY, FSoa FZ, const double* Bnx, const double* Bny, const double* Bnz, Ext ce,
@@ -1841,6 +1851,174 @@ KB __global__ void k_apply(Soa W, Soa Wn, FSoa FX, FSoa FY, FSoa FZ, const doubl
     const double v = apply_body<D, MHD>(W, Wn, FX, FY, FZ, Bnx, Bny, Bnz, ce, fe, dts(ts, 0), dts(ts, 1), dts(ts, 2), ph, err, tid_xcd(),
                                         cflpart != nullptr, cfl_mode, cdx, cdy, cdz, ts);
     if (cflpart && !stopped(ts)) block_max_store(v, cflpart);  // uniform branch; a stopped step leaves the committed state's maxima
+}
+
+// ======================================================= 2D CT in one pass
+// The constrained-transport stages around the 2D corrector, each half as one
+// pass over tiles of 8 x 32 points, a thread each: the tile's corner EMFs and
+// those of its high borders (9 x 33) are evaluated into LDS, and each thread
+// goes on to its faces and its cell with them.  Every value is formed by the
+// expressions of the separate stages (corner EMF, Faraday, half-step state /
+// apply), so results are theirs bit for bit.  The cell's flux sums are formed
+// before the EMFs, so their loads are in flight during them.  Bound by memory
+// (2048^2 mixed: 4.2-4.5 TB/s of the 4.8 a copy reaches) and, on small grids, by
+// latency.  Half step / final, against EMF + Faraday + whalf / apply: 2048^2
+// mixed 229 -> 216 / 307 -> 295 us, 771 x 530 FP64 43 -> 28 / 49 -> 32, 128^2 21
+// -> 10 / 23 -> 14; 96 patches FP64 0.88 -> 0.83 ms a step.  (Each thread
+// evaluating its four corners itself, without LDS: 252 / 334 us at 2048^2.)
+struct PtrsCt {  // arguments of the single grid's passes
+    Soa W, Wn;
+    FSoa FX, FY;
+    ERef ref;
+    double *B[3], *Bn[3];
+    ET *E0[3], *Bh[3], *Eh[3];
+    Ext ce, fe;
+    const StepDts* ts;
+    Phys ph;
+    unsigned long long* err;
+    double* cflpart;
+    int upwind, cfl_mode;
+    double cd[2];
+};
+constexpr int CT_TI = 8, CT_TJ = 32;  // tile (ct_tiles): rows long enough to be read in whole lines, 16% more EMFs than points
+static_assert(CT_TI * CT_TJ == 256, "a thread per point of a tile");
+struct CtTile {
+    ET x[CT_TI + 1][CT_TJ + 1], y[CT_TI + 1][CT_TJ + 1], z[CT_TI + 1][CT_TJ + 1];
+};
+struct Emf2 {
+    double x, y, z;
+};
+// Corner EMF of edge (i, j).
+__device__ __forceinline__ Emf2 emf2_at(const FSoa& FX, const FSoa& FY, const ERef& ref, const Ext& ce, const Ext& fe, int i, int j, int upwind) {
+    auto f = [&](const FSoa& F, int fld, int a, int b) { return double(F(fld, ce.at(a, b, 0))); };
+    auto r = [&](const ET* c, int a, int b) { return ed(c, fe.at(a, b, 0)); };
+    Emf2 e{0, 0, 0};
+    {
+        const double fy = f(FY, U_BZ, i, j), fx = f(FX, U_BZ, i, j);
+        e.x = -fy;
+        e.y = fx;
+        if (upwind) {
+            e.x += 0.25 * (-2 * fy - r(ref.x, i, j) - r(ref.x, i, j - 1));
+            e.y += 0.25 * (2 * fx - r(ref.y, i, j) - r(ref.y, i - 1, j));
+        }
+    }
+    {
+        const double yl = f(FY, U_BX, i - 1, j), yh = f(FY, U_BX, i, j), xl = f(FX, U_BY, i, j - 1), xh = f(FX, U_BY, i, j);
+        e.z = (yl - xl + yh - xh) * 0.25;
+        if (upwind) {
+            const double r00 = r(ref.z, i - 1, j - 1), r01 = r(ref.z, i - 1, j), r10 = r(ref.z, i, j - 1), r11 = r(ref.z, i, j);
+            e.z += upwind_corr(f(FX, U_RHO, i, j), yl, yh, r01, r11);
+            e.z += upwind_corr(f(FX, U_RHO, i, j - 1), yl, yh, r00, r10);
+            e.z += upwind_corr(f(FY, U_RHO, i, j), -xl, -xh, r10, r11);
+            e.z += upwind_corr(f(FY, U_RHO, i - 1, j), -xl, -xh, r00, r01);
+        }
+    }
+    return e;
+}
+// EMFs of the tile's points (i0 + a, j0 + b), a <= CT_TI, b <= CT_TJ, that lie
+// in [lo, hi0] x [lo, hi1].
+__device__ __forceinline__ void ct_edges(CtTile& S, const FSoa& FX, const FSoa& FY, const ERef& ref, const Ext& ce, const Ext& fe, int i0, int j0,
+                                         int lo, int hi0, int hi1, int upwind) {
+    for (int e = threadIdx.x; e < (CT_TI + 1) * (CT_TJ + 1); e += 256) {
+        const int a = e / (CT_TJ + 1), b = e % (CT_TJ + 1), i = i0 + a, j = j0 + b;
+        if (i < lo || i > hi0 || j < lo || j > hi1) continue;
+        const Emf2 v = emf2_at(FX, FY, ref, ce, fe, i, j, upwind);
+        S.x[a][b] = v.x; S.y[a][b] = v.y; S.z[a][b] = v.z;
+    }
+}
+// The half-step stages of the predictor: EMF -> half-step faces -> half-step
+// state -> its reference EMF, over the edges of [-1, n+2)^2.  `ref` is the
+// cells' reference EMF and Eh the half-step one: different arrays, for threads
+// read neighbours' `ref`.  Writes the x and y EMF and the x and y half-step
+// faces, which the corrector reads, and Eh.
+__device__ __forceinline__ void ct_half2_body(CtTile& S, const Soa& W, const FSoa& FX, const FSoa& FY, const ERef& ref, double* const B[3],
+                                              const Ext& ce, const Ext& fe, double hx, double hy, const Phys& ph, ET* const E0[3],
+                                              ET* const Bh[3], ET* const Eh[3], unsigned long long* err, unsigned tile,
+                                              const StepDts* gate = nullptr) {
+    const int nx = ce.n[0], ny = ce.n[1];
+    const unsigned ntj = (unsigned)(ny + 3 + CT_TJ - 1) / CT_TJ;
+    const int i0 = (int)(tile / ntj) * CT_TI - 1, j0 = (int)(tile % ntj) * CT_TJ - 1;
+    const int a = threadIdx.x / CT_TJ, b = threadIdx.x % CT_TJ, i = i0 + a, j = j0 + b;
+    const bool in = i <= nx + 1 && j <= ny + 1, xc = i <= nx, yc = j <= ny, cell = in && xc && yc;  // the last edges bound no cell
+    const long q = fe.at(i, j, 0), m = ce.at(i, j, 0);
+    U<double> u = uzero<double>();
+    if (cell) u = flux_update<2, true>(W, FX, FY, FY, ce, hx, hy, 0.0, ph, m);
+    ct_edges(S, FX, FY, ref, ce, fe, i0, j0, -1, nx + 1, ny + 1, 1);
+    __syncthreads();
+    if (!in) return;
+    E0[0][q] = S.x[a][b]; E0[1][q] = S.y[a][b];
+    const double z00 = S.z[a][b];
+    // the half-step faces are ET, as they are stored
+    double bx0 = 0, by0 = 0;
+    if (yc) {
+        const ET v = ET(ld32(B[0], q) - (double(S.z[a][b + 1]) - z00) * hy);
+        Bh[0][q] = v;
+        bx0 = v;
+    }
+    if (xc) {
+        const ET v = ET(ld32(B[1], q) - -(double(S.z[a + 1][b]) - z00) * hx);
+        Bh[1][q] = v;
+        by0 = v;
+    }
+    if (!cell || (gate && stopped(gate))) return;
+    const double z11 = S.z[a + 1][b + 1];
+    const double bx1 = ET(ld32(B[0], q + fe.s[0]) - (z11 - double(S.z[a + 1][b])) * hy);
+    const double by1 = ET(ld32(B[1], q + fe.s[1]) - -(z11 - double(S.z[a][b + 1])) * hx);
+    const double bz = ET(ld32(B[2], q) - ((double(S.y[a + 1][b]) - double(S.y[a][b])) * hx - (double(S.x[a][b + 1]) - double(S.x[a][b])) * hy));
+    if (!finite<true>(u)) report(err, ST_WHALF_NAN, (unsigned long long)m, E_NAN);
+    const P<double> w = body_field(prim<true>(u, ph), (bx0 + bx1) * 0.5, (by0 + by1) * 0.5, bz, ph);
+    double ex, ey, ez;
+    cross(w.Bx, w.By, w.Bz, w.vx, w.vy, w.vz, ex, ey, ez);
+    Eh[0][q] = ex; Eh[1][q] = ey; Eh[2][q] = ez;
+}
+KB __global__ void k_ct_half2(PtrsCt c) {
+    __shared__ CtTile S;
+    ct_half2_body(S, c.W, c.FX, c.FY, c.ref, c.B, c.ce, c.fe, dts(c.ts, 0, true), dts(c.ts, 1, true), c.ph, c.E0, c.Bh, c.Eh, c.err, block_xcd(),
+                  c.ts);
+}
+// The final stages: EMF -> faces -> next state, over the face index space: a
+// thread writes its point's three faces and, where its cell is an interior
+// one, the cell from the four faces around it (its own two and the next ones,
+// formed again); ghosts are copied.
+__device__ __forceinline__ double ct_final2_body(CtTile& S, const Soa& W, const Soa& Wn, const FSoa& FX, const FSoa& FY, const ERef& ref,
+                                                 double* const B[3], double* const Bn[3], const Ext& ce, const Ext& fe, double dt_dx,
+                                                 double dt_dy, int upwind, const Phys& ph, unsigned long long* err, unsigned tile, bool cfl,
+                                                 int cfl_mode, double cdx, double cdy, const StepDts* gate = nullptr) {
+    const int nx = ce.n[0], ny = ce.n[1], g = ce.g;
+    const unsigned ntj = (unsigned)(ny + 1 + 2 * g + CT_TJ - 1) / CT_TJ;
+    const int i0 = (int)(tile / ntj) * CT_TI - g, j0 = (int)(tile % ntj) * CT_TJ - g;
+    const int a = threadIdx.x / CT_TJ, b = threadIdx.x % CT_TJ, i = i0 + a, j = j0 + b;
+    const bool in = i <= nx + g && j <= ny + g;
+    const bool face = in && i >= 0 && i <= nx && j >= 0 && j <= ny, inner = face && i < nx && j < ny;
+    const long q = fe.at(i, j, 0), m = ce.at(i, j, 0);
+    U<double> u = uzero<double>();
+    if (inner) u = flux_update<2, true>(W, FX, FY, FY, ce, dt_dx, dt_dy, 0.0, ph, m);
+    ct_edges(S, FX, FY, ref, ce, fe, i0, j0, 0, nx, ny, upwind);
+    __syncthreads();
+    if (!in || (gate && stopped(gate))) return 0.0;
+    double b0 = ld32(B[0], q), b1 = ld32(B[1], q), b2 = ld32(B[2], q);
+    if (face) {
+        const double z00 = S.z[a][b];
+        if (j < ny) b0 -= (double(S.z[a][b + 1]) - z00) * dt_dy;
+        if (i < nx) b1 -= -(double(S.z[a + 1][b]) - z00) * dt_dx;
+        if (inner) b2 -= (double(S.y[a + 1][b]) - double(S.y[a][b])) * dt_dx - (double(S.x[a][b + 1]) - double(S.x[a][b])) * dt_dy;
+    }
+    Bn[0][q] = b0; Bn[1][q] = b1; Bn[2][q] = b2;
+    if (!inner) {
+        if (i < nx + g && j < ny + g)
+            for (int f = 0; f < 8; f++) st_nt(Wn, f, m, W(f, m));
+        return 0.0;
+    }
+    const double z11 = S.z[a + 1][b + 1];
+    const double bx1 = ld32(B[0], q + fe.s[0]) - (z11 - double(S.z[a + 1][b])) * dt_dy;
+    const double by1 = ld32(B[1], q + fe.s[1]) - -(z11 - double(S.z[a][b + 1])) * dt_dx;
+    return apply_finish<2, true>(u, Wn, (b0 + bx1) * 0.5, (b1 + by1) * 0.5, b2, ph, err, m, cfl, cfl_mode, cdx, cdy, 1.0);
+}
+KB __global__ void k_ct_final2(PtrsCt c) {
+    __shared__ CtTile S;
+    const double v = ct_final2_body(S, c.W, c.Wn, c.FX, c.FY, c.ref, c.B, c.Bn, c.ce, c.fe, dts(c.ts, 0), dts(c.ts, 1), c.upwind, c.ph, c.err,
+                                    block_xcd(), c.cflpart != nullptr, c.cfl_mode, c.cd[0], c.cd[1], c.ts);
+    if (c.cflpart && !stopped(c.ts)) block_max_store(v, c.cflpart);
 }
 
 // 1D Godunov::sweep update (Splitting.cpp:67-95): cells [-g+1, n+g-2] take
@@ -2079,7 +2257,8 @@ static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, 
     a.ts = &c.ctl->t; a.half = c.half;
     if constexpr (eref_in_sweep<D, MHD, FINAL, AX>())
         if (stage == ST_PRED_X + AX)  // the CTU predictor (not the flux sweep of a step without CTU)
-            for (int q = 0; q < 3; q++) a.eref[q] = et(c.Eh[q]);  // read by the predictor EMF before whalf overwrites it
+            // read by the predictor EMF; in 2D in the same launch that writes Eh, so the next faces' arrays hold it until the step writes them
+            for (int q = 0; q < 3; q++) a.eref[q] = et(D == 2 ? c.Bn[q] : c.Eh[q]);
     const long len = b.hi[AX] - b.lo[AX];
     long ntrans = 1;
     for (int d = 0; d < D; d++)
@@ -2160,8 +2339,16 @@ static void hydro3_fluxes(const StepCtx& c, hipStream_t s) {
 // The step with fused sweeps (2D, 3D): predictor fluxes ->
 // [MHD: corner EMF, half-step faces, half-step reference EMF] -> corrector
 // fluxes (CTU correction inside) -> [MHD: EMF, Faraday] -> apply.
+static PtrsCt ct_args(const StepCtx& c, const Soa F[3], const ERef& ref, int upwind) {
+    PtrsCt a{};
+    a.W = c.W; a.Wn = c.Wn; a.FX = fs(F[0]); a.FY = fs(F[1]); a.ref = ref;
+    for (int q = 0; q < 3; q++) { a.B[q] = c.B[q]; a.Bn[q] = c.Bn[q]; a.E0[q] = et(c.E0[q]); a.Bh[q] = et(c.Bh[q]); a.Eh[q] = et(c.Eh[q]); }
+    a.ce = c.ce; a.fe = c.fe; a.ts = &c.ctl->t; a.ph = c.ph; a.err = c.err; a.cflpart = c.cflpart;
+    a.upwind = upwind; a.cfl_mode = c.cfl_mode; a.cd[0] = c.d[0]; a.cd[1] = c.d[1];
+    return a;
+}
 template <int D, bool MHD, class R>
-static void step_fused(const StepCtx& c, hipStream_t s) {
+static long step_fused(const StepCtx& c, hipStream_t s) {
     const Ext& ce = c.ce;
     if constexpr (D == 3 && !MHD) {
         if (c.ctu) hydro3_fluxes<R>(c, s);
@@ -2171,20 +2358,15 @@ static void step_fused(const StepCtx& c, hipStream_t s) {
             sweep<D, MHD, R, false>(c, ax, b, fs(c.Fp[ax]), ST_PRED_X + ax, s);
             mark(c, K_PRED_X + ax);
         }
-        if constexpr (MHD) {
-            ERef none{nullptr, nullptr, nullptr};
+        if constexpr (MHD && D == 2) {
+            hipLaunchKernelGGL(k_ct_half2, dim3((unsigned)ct_tiles(ce.n[0] + 3, ce.n[1] + 3)), dim3(256), 0, s,
+                               ct_args(c, c.Fp, ERef{et(c.Bn[0]), et(c.Bn[1]), et(c.Bn[2])}, 1));
+            mark(c, K_WHALF);
+        } else if constexpr (MHD) {
             Box eb = make_box(D, -1, ce.n[0] + 2, -1, ce.n[1] + 2, -1, ce.n[2] + 2);
-            if constexpr (D == 2 && eref_in_sweep<D, MHD, false, D - 1>())  // the reference EMF from the y sweep
-                hipLaunchKernelGGL((k_emf2<false>), dim3(blocks(eb.count())), dim3(256), 0, s, fs(c.Fp[0]), fs(c.Fp[1]), c.W,
-                                   ERef{et(c.Eh[0]), et(c.Eh[1]), et(c.Eh[2])}, ce, c.fe, eb, 1, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]));
-            else if constexpr (D == 2)
-                hipLaunchKernelGGL((k_emf2<true>), dim3(blocks(eb.count())), dim3(256), 0, s, fs(c.Fp[0]), fs(c.Fp[1]), c.W, none, ce, c.fe, eb, 1,
-                                   et(c.E0[0]), et(c.E0[1]), et(c.E0[2]));
-            else {  // the reference EMF from the z sweep
-                static_assert(eref_in_sweep<D, MHD, false, D - 1>(), "the 3D predictor sweep stores the reference EMF");
-                emf3_tiled(fs(c.Fp[0]), fs(c.Fp[1]), fs(c.Fp[2]), ERef{et(c.Eh[0]), et(c.Eh[1]), et(c.Eh[2])}, ce, c.fe, eb, 1, et(c.E0[0]),
+            // the reference EMF from the z sweep
+            emf3_tiled(fs(c.Fp[0]), fs(c.Fp[1]), fs(c.Fp[2]), ERef{et(c.Eh[0]), et(c.Eh[1]), et(c.Eh[2])}, ce, c.fe, eb, 1, et(c.E0[0]),
                            et(c.E0[1]), et(c.E0[2]), s);
-            }
             mark(c, K_EMF_PRED);
             hipLaunchKernelGGL((k_faraday<D, ET>), dim3(blocks(c.fe.size)), dim3(256), 0, s, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]), c.B[0], c.B[1],
                                c.B[2], et(c.Bh[0]), et(c.Bh[1]), et(c.Bh[2]), c.fe, 1, &c.ctl->t);
@@ -2202,14 +2384,16 @@ static void step_fused(const StepCtx& c, hipStream_t s) {
         else sweep<D, MHD, R, false>(c, ax, b, fs(c.F[ax]), ST_FLUX_X + ax, s);
         mark(c, K_FLUX_X + ax);
     }
-    if constexpr (MHD) {
+    if constexpr (MHD && D == 2) {
+        const long tiles = ct_tiles(ce.n[0] + 1 + 2 * ce.g, ce.n[1] + 1 + 2 * ce.g);
+        hipLaunchKernelGGL(k_ct_final2, dim3((unsigned)tiles), dim3(256), 0, s,
+                           ct_args(c, c.F, ERef{et(c.Eh[0]), et(c.Eh[1]), et(c.Eh[2])}, c.ctu));
+        mark(c, K_APPLY);
+        return tiles;
+    } else if constexpr (MHD) {
         Box eb = make_box(D, 0, ce.n[0] + 1, 0, ce.n[1] + 1, 0, ce.n[2] + 1);
         ERef eh{et(c.Eh[0]), et(c.Eh[1]), et(c.Eh[2])};
-        if constexpr (D == 2)
-            hipLaunchKernelGGL((k_emf2<false>), dim3(blocks(eb.count())), dim3(256), 0, s, fs(c.F[0]), fs(c.F[1]), c.W, eh, ce, c.fe, eb, c.ctu,
-                               et(c.E0[0]), et(c.E0[1]), et(c.E0[2]));
-        else
-            emf3_tiled(fs(c.F[0]), fs(c.F[1]), fs(c.F[2]), eh, ce, c.fe, eb, c.ctu, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]), s);
+        emf3_tiled(fs(c.F[0]), fs(c.F[1]), fs(c.F[2]), eh, ce, c.fe, eb, c.ctu, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]), s);
         mark(c, K_EMF);
         hipLaunchKernelGGL((k_faraday<D, double>), dim3(blocks(c.fe.size)), dim3(256), 0, s, et(c.E0[0]), et(c.E0[1]), et(c.E0[2]), c.B[0], c.B[1], c.B[2],
                            c.Bn[0], c.Bn[1], c.Bn[2], c.fe, 0, &c.ctl->t);
@@ -2218,15 +2402,13 @@ static void step_fused(const StepCtx& c, hipStream_t s) {
     hipLaunchKernelGGL((k_apply<D, MHD>), dim3(blocks(ce.size)), dim3(256), 0, s, c.W, c.Wn, fs(c.F[0]), fs(c.F[1]), fs(c.F[2]), c.Bn[0], c.Bn[1],
                        c.Bn[2], ce, c.fe, &c.ctl->t, c.ph, c.err, c.cflpart, c.cfl_mode, c.d[0], c.d[1], c.d[2]);
     mark(c, K_APPLY);
+    return blocks(ce.size);
 }
 
 template <int D, bool MHD, class R>
-static void step_t(const StepCtx& c, hipStream_t s) {
+static long step_t(const StepCtx& c, hipStream_t s) {
     if constexpr (D >= 2) {
-        if (c.fused) {
-            step_fused<D, MHD, R>(c, s);
-            return;
-        }
+        if (c.fused) return step_fused<D, MHD, R>(c, s);
     }
     const Ext& ce = c.ce;
     const int g = ce.g;
@@ -2244,7 +2426,7 @@ static void step_t(const StepCtx& c, hipStream_t s) {
         if constexpr (D == 1)
             hipLaunchKernelGGL((k_apply1<MHD>), dim3(blocks(ce.size)), dim3(256), 0, s, c.W, c.Wn, fs(c.F[0]), ce, &c.ctl->t, c.ph, c.err);
         mark(c, K_APPLY);
-        return;
+        return 0;
     }
     if (c.ctu) {
         if constexpr (MHD) {
@@ -2325,6 +2507,7 @@ static void step_t(const StepCtx& c, hipStream_t s) {
     hipLaunchKernelGGL((k_apply<D, MHD>), dim3(blocks(ce.size)), dim3(256), 0, s, c.W, c.Wn, fs(c.F[0]), fs(c.F[1]), fs(c.F[2]), c.Bn[0], c.Bn[1],
                        c.Bn[2], ce, c.fe, &c.ctl->t, c.ph, c.err, c.cflpart, c.cfl_mode, c.d[0], c.d[1], c.d[2]);
     mark(c, K_APPLY);
+    return blocks(ce.size);
 }
 
 // 3D hydro CTU, 12 solves (CTU.cpp:222-261): six corner-flux passes with
@@ -2526,7 +2709,7 @@ __device__ __forceinline__ SweepArgs batch_sweep_args(const BatchArgs& A, const 
     s.Fo = FIN ? v.F[AX] : v.Fp[AX];
     s.stage = (FIN ? ST_FLUX_X : ST_PRED_X) + AX;
     if constexpr (eref_in_sweep<2, true, FIN, AX>())
-        for (int q = 0; q < 3; q++) s.eref[q] = v.Eh[q];  // the predictor EMF's reference, before whalf overwrites it
+        for (int q = 0; q < 3; q++) s.eref[q] = et(v.Bn[q]);  // the predictor EMF's reference, until the step writes the next faces
     return s;
 }
 template <bool FIN>
@@ -2552,45 +2735,19 @@ KS __attribute__((amdgpu_waves_per_eu(wave_min_waves<RT>()))) __global__ void kb
         default: s.chunk = 63; sweep_wave_body<2, true, RT, 1, FIN, 64>(s, w, lane); break;
     }
 }
-template <bool PRED>
-KB __global__ void kb_emf(BatchArgs A, BlockTable bt) {
+KB __global__ void kb_ct_half(BatchArgs A, BlockTable bt) {
     BATCH_ITEM(bt)
-    const PatchView v = patch_view(A, p);
-    const int lo = PRED ? -1 : 0, ex = PRED ? 2 : 1;
-    const Box eb = make_box(2, lo, v.ce.n[0] + ex, lo, v.ce.n[1] + ex);
-    if (PRED) {
-        if constexpr (eref_in_sweep<2, true, false, 1>()) {  // the reference EMF from the y sweep
-            const ERef eh{v.Eh[0], v.Eh[1], v.Eh[2]};
-            emf2_body<false>(v.Fp[0], v.Fp[1], v.W, eh, v.ce, v.fe, eb, 1, v.E0[0], v.E0[1], v.E0[2], t);
-        } else {
-            const ERef none{nullptr, nullptr, nullptr};
-            emf2_body<true>(v.Fp[0], v.Fp[1], v.W, none, v.ce, v.fe, eb, 1, v.E0[0], v.E0[1], v.E0[2], t);
-        }
-    } else {
-        const ERef eh{v.Eh[0], v.Eh[1], v.Eh[2]};
-        emf2_body<false>(v.F[0], v.F[1], v.W, eh, v.ce, v.fe, eb, 1, v.E0[0], v.E0[1], v.E0[2], t);
-    }
+    PatchView v = patch_view(A, p);
+    __shared__ CtTile S;
+    ct_half2_body(S, v.W, v.Fp[0], v.Fp[1], ERef{et(v.Bn[0]), et(v.Bn[1]), et(v.Bn[2])}, v.B, v.ce, v.fe, dts(A.ts + p, 0, true),
+                  dts(A.ts + p, 1, true), A.ph, v.E0, v.Bh, v.Eh, A.err + p, (unsigned)bt.first[bx] / 256u);
 }
-template <bool HALF>
-KB __global__ void kb_faraday(BatchArgs A, BlockTable bt) {
+KB __global__ void kb_ct_final(BatchArgs A, BlockTable bt) {
     BATCH_ITEM(bt)
-    const PatchView v = patch_view(A, p);
-    const double dx = dts(A.ts + p, 0, HALF), dy = dts(A.ts + p, 1, HALF), dz = dts(A.ts + p, 2, HALF);
-    if (HALF) faraday_body<2, ET>(v.E0[0], v.E0[1], v.E0[2], v.B[0], v.B[1], v.B[2], v.Bh[0], v.Bh[1], v.Bh[2], v.fe, 1, dx, dy, dz, t);
-    else faraday_body<2, double>(v.E0[0], v.E0[1], v.E0[2], v.B[0], v.B[1], v.B[2], v.Bn[0], v.Bn[1], v.Bn[2], v.fe, 0, dx, dy, dz, t);
-}
-KB __global__ void kb_whalf(BatchArgs A, BlockTable bt) {
-    BATCH_ITEM(bt)
-    const PatchView v = patch_view(A, p);
-    const Box cb = make_box(2, -1, v.ce.n[0] + 1, -1, v.ce.n[1] + 1);
-    whalf_body<2>(v.W, v.Fp[0], v.Fp[1], v.Fp[2], v.Bh[0], v.Bh[1], v.Bh[2], v.ce, v.fe, cb, dts(A.ts + p, 0, true),
-                  dts(A.ts + p, 1, true), dts(A.ts + p, 2, true), A.ph, v.Eh[0], v.Eh[1], v.Eh[2], A.err + p, t);
-}
-KB __global__ void kb_apply(BatchArgs A, BlockTable bt) {
-    BATCH_ITEM(bt)
-    const PatchView v = patch_view(A, p);
-    double m = apply_body<2, true>(v.W, v.Wn, v.F[0], v.F[1], v.F[2], v.Bn[0], v.Bn[1], v.Bn[2], v.ce, v.fe, dts(A.ts + p, 0),
-                                   dts(A.ts + p, 1), dts(A.ts + p, 2), A.ph, A.err + p, t, true, A.cfl_mode, v.dx, v.dy, 1.0);
+    PatchView v = patch_view(A, p);
+    __shared__ CtTile S;
+    double m = ct_final2_body(S, v.W, v.Wn, v.F[0], v.F[1], ERef{v.Eh[0], v.Eh[1], v.Eh[2]}, v.B, v.Bn, v.ce, v.fe, dts(A.ts + p, 0),
+                              dts(A.ts + p, 1), 1, A.ph, A.err + p, (unsigned)bt.first[bx] / 256u, true, A.cfl_mode, v.dx, v.dy);
     // the new state's CFL maximum over the patch's interior, for the next
     // step if this one is committed (one atomic per workgroup)
     for (int off = 32; off > 0; off >>= 1) m = dmax(m, __shfl_xor(m, off));
@@ -2642,14 +2799,10 @@ void launch_batch_step(const BatchArgs& a, const BlockTable* bt, bool init_only,
     hipLaunchKernelGGL(kb_dt, dim3(pb), T, 0, s, a);
     hipLaunchKernelGGL((kb_sweep_x<false>), grid(BK_PRED_X), T, 0, s, a, bt[BK_PRED_X]);
     hipLaunchKernelGGL((kb_sweep_y<false>), grid(BK_PRED_Y), T, 0, s, a, bt[BK_PRED_Y]);
-    hipLaunchKernelGGL((kb_emf<true>), grid(BK_EDGES_P), T, 0, s, a, bt[BK_EDGES_P]);
-    hipLaunchKernelGGL((kb_faraday<true>), grid(BK_FACES), T, 0, s, a, bt[BK_FACES]);
-    hipLaunchKernelGGL(kb_whalf, grid(BK_CELLS1), T, 0, s, a, bt[BK_CELLS1]);
+    hipLaunchKernelGGL(kb_ct_half, grid(BK_EDGES), T, 0, s, a, bt[BK_EDGES]);
     hipLaunchKernelGGL((kb_sweep_x<true>), grid(BK_FLUX_X), T, 0, s, a, bt[BK_FLUX_X]);
     hipLaunchKernelGGL((kb_sweep_y<true>), grid(BK_FLUX_Y), T, 0, s, a, bt[BK_FLUX_Y]);
-    hipLaunchKernelGGL((kb_emf<false>), grid(BK_EDGES), T, 0, s, a, bt[BK_EDGES]);
-    hipLaunchKernelGGL((kb_faraday<false>), grid(BK_FACES), T, 0, s, a, bt[BK_FACES]);
-    hipLaunchKernelGGL(kb_apply, grid(BK_CELLS), T, 0, s, a, bt[BK_CELLS]);
+    hipLaunchKernelGGL(kb_ct_final, grid(BK_FACES), T, 0, s, a, bt[BK_FACES]);
     hipLaunchKernelGGL(kb_commit, dim3(pb), T, 0, s, a, last ? 0 : 1);
 }
 
@@ -2719,10 +2872,10 @@ void launch_split_axis(const StepCtx& c, int ax, Soa in, Soa out, hipStream_t s)
     }
 }
 
-void launch_step(const StepCtx& c, hipStream_t s) {
-    if (c.dim == 1) c.mhd ? step_t<1, true, RT>(c, s) : step_t<1, false, RT>(c, s);
-    else if (c.dim == 2) c.mhd ? step_t<2, true, RT>(c, s) : step_t<2, false, RT>(c, s);
-    else c.mhd ? step_t<3, true, RT>(c, s) : step_t<3, false, RT>(c, s);
+long launch_step(const StepCtx& c, hipStream_t s) {
+    if (c.dim == 1) return c.mhd ? step_t<1, true, RT>(c, s) : step_t<1, false, RT>(c, s);
+    if (c.dim == 2) return c.mhd ? step_t<2, true, RT>(c, s) : step_t<2, false, RT>(c, s);
+    return c.mhd ? step_t<3, true, RT>(c, s) : step_t<3, false, RT>(c, s);
 }
 
 }  // namespace DG_NS

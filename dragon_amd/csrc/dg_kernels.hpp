@@ -115,13 +115,12 @@ enum { BATCH_ERR_CFL = 5, BATCH_ERR_DT = 6 };
 // work kinds of a batched step (items per patch in dg_api.hip: batch_items)
 enum BatchKind {
     BK_BC,                                   // boundary: ghost cells x 8 fields, then boundary faces x 3 components
-    BK_CELLS1,                               // cells [-1, n+1)^2: CFL, half-step state
+    BK_CELLS1,                               // cells [-1, n+1)^2: CFL
     BK_PRED_X, BK_PRED_Y,                    // predictor sweeps (x: faces-per-thread chunks; y: 63 faces per wavefront)
-    BK_EDGES_P,                              // edges [-1, n+2)^2: predictor EMF
-    BK_FACES,                                // every face: Faraday
+    BK_EDGES,                                // edges [-1, n+2)^2 in tiles: the half-step stages
     BK_FLUX_X, BK_FLUX_Y,                    // corrector sweeps
-    BK_EDGES,                                // edges [0, n+1)^2: EMF
-    BK_CELLS,                                // every cell: apply, initialize_B_fields
+    BK_FACES,                                // every face (and cell) in tiles: the final stages
+    BK_CELLS,                                // every cell: initialize_B_fields
     BK_COUNT
 };
 struct BlockTable {
@@ -173,7 +172,7 @@ struct BatchArgs {
 // one build out of the other.
 #define DG_LAUNCH_INTERFACE                                                                                     \
     void launch_batch_step(const BatchArgs& a, const BlockTable* bt, bool init_only, bool first, bool last, hipStream_t s); \
-    void launch_step(const StepCtx& c, hipStream_t s);                                                          \
+    long launch_step(const StepCtx& c, hipStream_t s);  /* returns the CFL maxima left in cflpart */              \
     void launch_split_axis(const StepCtx& c, int ax, Soa in, Soa out, hipStream_t s);  /* one split sweep (hydro) */ \
     void launch_bc(const BCArgs& a, bool faces, hipStream_t s);                                                 \
     bool launch_bc_list(BCListArgs& a, hipStream_t s);                                                          \
@@ -187,6 +186,8 @@ struct BatchArgs {
     void launch_fill_u64(unsigned long long* p, unsigned long long v, int n, hipStream_t s);                    \
     void launch_aos_to_soa(const double* a, int stride, int nf, Soa soa, long n, hipStream_t s);                \
     void launch_soa_to_aos(Soa soa, int nf, double* a, int stride, long n, hipStream_t s);
+// tiles of 8 x 32 points of the 2D constrained-transport passes
+inline long ct_tiles(long ni, long nj) { return ((ni + 7) / 8) * ((nj + 31) / 32); }
 namespace p64 { DG_LAUNCH_INTERFACE }
 namespace p32 { DG_LAUNCH_INTERFACE }
 
