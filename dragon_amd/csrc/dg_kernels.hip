@@ -1319,6 +1319,29 @@ template <class R> KS __global__ void k_corner_wave(SweepArgs a) {
     if (lane >= 1 && live && c >= 1) corner_fluxes<2>(a, l1, L1, l2, L2, idx);
 }
 
+// The sweeps of every axis in one launch, for grids whose single sweeps do not
+// fill the chip for long: they do not depend on each other, and side by side
+// one's last round of workgroups overlaps the next one's first.  Workgroups
+// [0, n0) sweep x, [n0, n0 + n1) y, the rest z.  (All run at the occupancy of
+// the largest, so large grids keep a launch per axis.)
+template <int D, bool MHD, class R, bool FINAL, class RS>
+KS __global__ void k_sweeps(SweepArgs ax, SweepArgs ay, SweepArgs az, unsigned n0, unsigned n1) {
+    if (stopped(ax.ts)) return;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    unsigned b = blockIdx.x;
+    if (b < n0) {
+        sweep_march_body<D, MHD, R, 0, FINAL, march_window<R>(), true, RS>(ax, (long)b * 256 + threadIdx.x);
+        return;
+    }
+    b -= n0;
+    if constexpr (D == 2) {
+        sweep_stream_body<D, MHD, R, 1, FINAL, RS>(ay, (int)b * 4 + wv, lane);
+    } else {
+        if (b < n1) sweep_march_body<D, MHD, R, 1, FINAL, march_window<R>(), true, RS>(ay, (long)b * 256 + threadIdx.x);
+        else sweep_stream_body<D, MHD, R, 2, FINAL, RS>(az, (int)(b - n1) * 4 + wv, lane);
+    }
+}
+
 // ===================================================== CTU hydro (2D/3D)
 // correctState (CTU.cpp:264-301): states along SAX corrected by the flux
 // difference of FAX.
@@ -2244,10 +2267,11 @@ static long march_chunk(long faces, bool fp64) {
     return std::max(1L, (long)(std::sqrt(2.0 * (double)faces / resident) + 0.5));
 }
 
-// One sweep launch for axis AX over the face box b.
-template <int D, bool MHD, class R, bool FINAL, int AX, class RS>
-static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, hipStream_t s) {
-    SweepArgs a{};
+// Arguments of the sweep of axis AX over the face box b; the workgroups it
+// takes (0: no faces).
+template <int D, bool MHD, bool FP64, bool FINAL, int AX>
+static unsigned sweep_args(const StepCtx& c, const Box& b, const FSoa& out, int stage, SweepArgs& a) {
+    a = SweepArgs{};
     a.W = c.W;
     for (int q = 0; q < 3; q++) {
         a.B[q] = c.B[q]; a.Bh[q] = et(c.Bh[q]); a.E0[q] = et(c.E0[q]); a.Fp[q] = fs(c.Fp[q]);
@@ -2263,25 +2287,34 @@ static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, 
     long ntrans = 1;
     for (int d = 0; d < D; d++)
         if (d != AX) ntrans *= b.hi[d] - b.lo[d];
-    if (len <= 0 || ntrans <= 0) return;
+    if (len <= 0 || ntrans <= 0) return 0;
     if constexpr (AX == D - 1) {
         const long cells = ntrans * (len + 1);
         const long waves = cells > 1 ? (cells - 1 + 62) / 63 : 1;
         a.chunk = 63;
-        hipLaunchKernelGGL((k_sweep_wave<D, MHD, R, AX, FINAL, RS>), dim3(blocks(waves * 64)), dim3(256), 0, s, a);
+        return blocks(waves * 64);
     } else {
-        const long chunk0 = march_chunk(len * ntrans, sizeof(R) == 8);
-        long chunk = c.march_chunk > 0 ? c.march_chunk : chunk0;
-        if (chunk > len) chunk = len;
-        const long nch = (len + chunk - 1) / chunk;
+        const long chunk = std::min(len, c.march_chunk > 0 ? (long)c.march_chunk : march_chunk(len * ntrans, FP64));
         a.chunk = (int)chunk;
+        return blocks((len + chunk - 1) / chunk * ntrans);
+    }
+}
+// One sweep launch for axis AX over the face box b.
+template <int D, bool MHD, class R, bool FINAL, int AX, class RS>
+static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, hipStream_t s) {
+    SweepArgs a;
+    const unsigned n = sweep_args<D, MHD, sizeof(R) == 8, FINAL, AX>(c, b, out, stage, a);
+    if (!n) return;
+    if constexpr (AX == D - 1) {
+        hipLaunchKernelGGL((k_sweep_wave<D, MHD, R, AX, FINAL, RS>), dim3(n), dim3(256), 0, s, a);
+    } else {
         if constexpr (!march_window<R>()) {
             if (c.march_window) {
-                hipLaunchKernelGGL((k_sweep_march_window<D, MHD, R, AX, FINAL>), dim3(blocks(nch * ntrans)), dim3(256), 0, s, a);
+                hipLaunchKernelGGL((k_sweep_march_window<D, MHD, R, AX, FINAL>), dim3(n), dim3(256), 0, s, a);
                 return;
             }
         }
-        hipLaunchKernelGGL((k_sweep_march<D, MHD, R, AX, FINAL, RS>), dim3(blocks(nch * ntrans)), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_sweep_march<D, MHD, R, AX, FINAL, RS>), dim3(n), dim3(256), 0, s, a);
     }
 }
 template <int D, bool MHD, class R, bool FINAL, class RS = R>
@@ -2289,6 +2322,30 @@ static void sweep(const StepCtx& c, int ax, const Box& b, const FSoa& out, int s
     if (ax == 0) sweep_t<D, MHD, R, FINAL, 0, RS>(c, b, out, stage, s);
     else if (ax == 1) { if constexpr (D >= 2) sweep_t<D, MHD, R, FINAL, 1, RS>(c, b, out, stage, s); }
     else { if constexpr (D >= 3) sweep_t<D, MHD, R, FINAL, 2, RS>(c, b, out, stage, s); }
+}
+// The sweeps of all axes: in one launch up to this many workgroups (about 4
+// million cells).  Per step, apart -> together: 3D MHD 24^3 FP64 146 -> 95 us,
+// 64 x 32 x 32 164 -> 136, 128^3 1772 -> 1743, but 160^3 (22 thousand) 3166 ->
+// 3171 and 240 x 200 x 261 8776 -> 9124; 2D MHD 128^2 81 -> 65, 1024^2 557 ->
+// 528, 2048^2 (19 thousand) 1887 -> 1911; 2D hydro 1800^2 762 -> 741; 3D hydro
+// 150 x 128 x 170 (17 thousand) 2054 -> 2010.
+constexpr unsigned MERGE_WORKGROUPS = 18000;
+template <int D, bool MHD, class R, bool FINAL, class RS = R>
+static void sweeps(const StepCtx& c, const Box b[3], const Soa out[3], int stage, int kernel_id, hipStream_t s) {
+    SweepArgs a[3];
+    unsigned n[3] = {0, 0, 0};
+    n[0] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 0>(c, b[0], fs(out[0]), stage, a[0]);
+    n[1] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 1>(c, b[1], fs(out[1]), stage + 1, a[1]);
+    if constexpr (D == 3) n[2] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 2>(c, b[2], fs(out[2]), stage + 2, a[2]);
+    if (n[0] + n[1] + n[2] <= MERGE_WORKGROUPS && !c.march_window) {
+        hipLaunchKernelGGL((k_sweeps<D, MHD, R, FINAL, RS>), dim3(n[0] + n[1] + n[2]), dim3(256), 0, s, a[0], a[1], a[D == 3 ? 2 : 1], n[0], n[1]);
+        mark(c, kernel_id);
+        return;
+    }
+    for (int ax = 0; ax < D; ax++) {
+        sweep<D, MHD, R, FINAL, RS>(c, ax, b[ax], fs(out[ax]), stage + ax, s);
+        mark(c, kernel_id + ax);
+    }
 }
 
 // 3D hydro CTU, 12 solves (CTU.cpp:222-261), half states rebuilt in each
@@ -2300,10 +2357,9 @@ static int corner(int a, int t) { return 2 * a + (t == (a == 2 ? 1 : 2)); }
 template <class R>
 static void hydro3_fluxes(const StepCtx& c, hipStream_t s) {
     const Ext& ce = c.ce;
-    for (int ax = 0; ax < 3; ax++) {
-        sweep<3, false, R, false, double>(c, ax, face_box(3, ce, ax, 0, 0, -1, 1), fs(c.F[ax]), ST_PRED_X + ax, s);
-        mark(c, K_PRED_X + ax);
-    }
+    Box pb[3];
+    for (int ax = 0; ax < 3; ax++) pb[ax] = face_box(3, ce, ax, 0, 0, -1, 1);
+    sweeps<3, false, R, false, double>(c, pb, c.F, ST_PRED_X, K_PRED_X, s);
     static const int order[3][3] = {{0, 2, 0}, {4, 0, 1}, {5, 3, 0}};  // the reference's position of the flux along a corrected by t
     for (int ax = 0; ax < 3; ax++) {
         const int t1 = ax == 0 ? 1 : 0, t2 = ax == 2 ? 1 : 2;
@@ -2353,11 +2409,9 @@ static long step_fused(const StepCtx& c, hipStream_t s) {
     if constexpr (D == 3 && !MHD) {
         if (c.ctu) hydro3_fluxes<R>(c, s);
     } else if (c.ctu) {
-        for (int ax = 0; ax < D; ax++) {
-            Box b = MHD ? face_box(D, ce, ax, -1, 1, -2, 2) : face_box(D, ce, ax, 0, 0, -1, 1);
-            sweep<D, MHD, R, false>(c, ax, b, fs(c.Fp[ax]), ST_PRED_X + ax, s);
-            mark(c, K_PRED_X + ax);
-        }
+        Box pb[3];
+        for (int ax = 0; ax < D; ax++) pb[ax] = MHD ? face_box(D, ce, ax, -1, 1, -2, 2) : face_box(D, ce, ax, 0, 0, -1, 1);
+        sweeps<D, MHD, R, false>(c, pb, c.Fp, ST_PRED_X, K_PRED_X, s);
         if constexpr (MHD && D == 2) {
             hipLaunchKernelGGL(k_ct_half2, dim3((unsigned)ct_tiles(ce.n[0] + 3, ce.n[1] + 3)), dim3(256), 0, s,
                                ct_args(c, c.Fp, ERef{et(c.Bn[0]), et(c.Bn[1]), et(c.Bn[2])}, 1));
@@ -2378,11 +2432,11 @@ static long step_fused(const StepCtx& c, hipStream_t s) {
             mark(c, K_WHALF);
         }
     }
-    for (int ax = 0; ax < D && !(D == 3 && !MHD && c.ctu); ax++) {
-        Box b = MHD ? face_box(D, ce, ax, 0, 0, -1, 1) : face_box(D, ce, ax, 0, 0, 0, 0);
-        if (c.ctu) sweep<D, MHD, R, true>(c, ax, b, fs(c.F[ax]), ST_FLUX_X + ax, s);
-        else sweep<D, MHD, R, false>(c, ax, b, fs(c.F[ax]), ST_FLUX_X + ax, s);
-        mark(c, K_FLUX_X + ax);
+    if (!(D == 3 && !MHD && c.ctu)) {
+        Box fb[3];
+        for (int ax = 0; ax < D; ax++) fb[ax] = MHD ? face_box(D, ce, ax, 0, 0, -1, 1) : face_box(D, ce, ax, 0, 0, 0, 0);
+        if (c.ctu) sweeps<D, MHD, R, true>(c, fb, c.F, ST_FLUX_X, K_FLUX_X, s);
+        else sweeps<D, MHD, R, false>(c, fb, c.F, ST_FLUX_X, K_FLUX_X, s);
     }
     if constexpr (MHD && D == 2) {
         const long tiles = ct_tiles(ce.n[0] + 1 + 2 * ce.g, ce.n[1] + 1 + 2 * ce.g);
