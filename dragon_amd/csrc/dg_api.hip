@@ -229,7 +229,7 @@ int dg_create(const dg_desc* desc, dg_grid** out) {
     if (d.dim >= 2) {
         // one per workgroup of the pass that writes the next state
         const long parts = d.dim == 2 ? ct_tiles(d.nx + 1 + 2 * gh, d.ny + 1 + 2 * gh) : 0;
-        ok = ok && alloc(&g->cflpart, std::max(parts, (nc + 255) / 256));
+        ok = ok && alloc(&g->cflpart, std::max(parts, nc / 248 + 2));
     }
     ok = ok && hipMalloc((void**)&g->dev_words, 4 * sizeof(unsigned long long)) == hipSuccess;
     ok = ok && hipHostMalloc((void**)&g->host_words, 4 * sizeof(unsigned long long), hipHostMallocDefault) == hipSuccess;
@@ -571,7 +571,10 @@ int dg_step(dg_grid* g, double dt, dg_status* st) {
 // the sweep order rotating with sweep_step (2 orders in 2D, 6 in 3D).  The
 // sweeps run W -> Wn -> Ws -> Wn [-> Ws -> Wn], each after the boundary pass
 // on its input; W is kept, so a failed step commits nothing.
-int dg_split_step(dg_grid* g, double dt, dg_status* st) {
+static int split_step(dg_grid* g, double dt, dg_status* st, bool filled);
+int dg_split_step(dg_grid* g, double dt, dg_status* st) { return split_step(g, dt, st, false); }
+// filled: the grid's boundary has just been applied (and W not changed since).
+static int split_step(dg_grid* g, double dt, dg_status* st, bool filled) {
     if (!g) return DG_ERR_ARG;
     const int D = g->d.dim;
     if (D == 1) return dg_step(g, dt, st);  // Grid1D::split_step is unsplit_step (Splitting.cpp:98)
@@ -603,15 +606,18 @@ int dg_split_step(dg_grid* g, double dt, dg_status* st) {
     double* const W0 = g->W;
     for (int q = 0; q < n; q++) {
         double* out = q % 2 == 0 ? g->Wn : g->Ws;
-        g->W = in;  // the boundary pass runs on this sweep's input
-        int rc = dg_apply_boundary(g);
-        g->W = W0;
-        if (rc) return rc;
+        if (q > 0 || !filled) {
+            g->W = in;  // the boundary pass runs on this sweep's input
+            int rc = dg_apply_boundary(g);
+            g->W = W0;
+            if (rc) return rc;
+        }
         StepCtx c = make_ctx(g);
         c.half = half[q];
+        if (q < n - 1) c.cflpart = nullptr;  // the last sweep's maxima are the next state's
         tm_record(g, -1);
-        if (c.mixed) p32::launch_split_axis(c, ax[q], soa(in, g->ce.size), soa(out, g->ce.size), g->s);
-        else p64::launch_split_axis(c, ax[q], soa(in, g->ce.size), soa(out, g->ce.size), g->s);
+        g->ncflpart = c.mixed ? p32::launch_split_axis(c, ax[q], soa(in, g->ce.size), soa(out, g->ce.size), g->s)
+                              : p64::launch_split_axis(c, ax[q], soa(in, g->ce.size), soa(out, g->ce.size), g->s);
         tm_record(g, K_FLUX_X + ax[q]);
         in = out;
     }
@@ -635,6 +641,7 @@ int dg_split_step(dg_grid* g, double dt, dg_status* st) {
     }
     std::swap(g->W, g->Wn);  // the last sweep wrote Wn (an odd number of sweeps)
     g->sweep_step++;
+    g->cfl_cached = g->cflpart != nullptr && !g->bc_cb;
     set_status(st, DG_OK, 0, 0, 0, "");
     return DG_OK;
 }
@@ -745,7 +752,7 @@ static int advance_loop(dg_grid* g, double dt, int check_cfl, long max_steps, dg
         }
         while (true) {
             if (!attempted) {
-                rc = split ? dg_split_step(g, t1, st) : dg_step(g, t1, st);
+                rc = split ? split_step(g, t1, st, !g->bc_cb) : dg_step(g, t1, st);
                 if (rc == DG_OK) break;
                 if (rc == DG_ERR_HIP || rc == DG_ERR_ARG || rc == DG_ERR_UNSUPPORTED) return rc;
             }

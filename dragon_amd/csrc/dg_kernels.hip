@@ -973,7 +973,7 @@ __device__ __forceinline__ void cell_states(const SweepArgs& a, int i, int j, in
 }
 
 template <bool MHD, class R, int AX, class RS = R>
-__device__ __forceinline__ void face_flux(const SweepArgs& a, const P<R>& l0, const P<R>& r0, long m) {
+__device__ __forceinline__ U<RS> face_flux_u(const SweepArgs& a, const P<R>& l0, const P<R>& r0, long m) {
     P<RS> l, r;
     if constexpr (sizeof(RS) == sizeof(R)) { l = l0; r = r0; }
     else { l = p_wide(l0); r = p_wide(r0); }
@@ -984,7 +984,11 @@ __device__ __forceinline__ void face_flux(const SweepArgs& a, const P<R>& l0, co
     if (fail) report(a.err, a.stage, (unsigned long long)m, fail == RF_BAD_INPUT ? E_RIEMANN_INPUT : E_RIEMANN_SOLUTION);
     if (AX == 1) f = swapXY(f);
     if (AX == 2) f = swapXZ(f);
-    store_u<RS>(a.Fo, m, f, MHD);
+    return f;
+}
+template <bool MHD, class R, int AX, class RS = R>
+__device__ __forceinline__ void face_flux(const SweepArgs& a, const P<R>& l, const P<R>& r, long m) {
+    store_u<RS>(a.Fo, m, face_flux_u<MHD, R, AX, RS>(a, l, r, m), MHD);
 }
 
 // Windowed walkers (stencil cells carried in registers) for the FP32 form;
@@ -2870,36 +2874,99 @@ void launch_batch_step(const BatchArgs& a, const BlockTable* bt, bool init_only,
 // cell n+g-2 takes the sweep's trailing zero update.  Hydro only.
 template <class T> __device__ __forceinline__ P<T> to_line(const P<T>& w, int ax) { return ax == 0 ? w : ax == 1 ? swapXY(w) : swapXZ(w); }
 template <class T> __device__ __forceinline__ U<T> to_line(const U<T>& u, int ax) { return ax == 0 ? u : ax == 1 ? swapXY(u) : swapXZ(u); }
+//
+// The last sweep of a step also leaves the workgroups' CFL maxima over the
+// interior (cfl.part), as the unsplit step's apply pass does: the next step's
+// CFL pass reduces those and the ghost shell (1000 x 611: 34 -> 8 us a step).
+struct SplitCfl {
+    double* part;  // or null
+    int mode;
+    double d[3];
+};
+// Update of cell (idx) from the fluxes fl, fr (in its line's frame) below and
+// above it along AX; cells the sweep does not update are copied.  Returns the
+// signal speed of an interior cell if asked for.
 template <int D, int AX>
-KB __global__ void k_apply_axis(Soa W, Soa Wn, FSoa F, Ext ce, const StepDts* ts, int half, Phys ph) {
-    if (stopped(ts)) return;
-    const double dt_d = dts(ts, AX, half);
-    const long m = tid();
-    if (m >= ce.size) return;
-    const int g = ce.g, n = ce.n[AX];
-    unsigned r = (unsigned)m;
-    int idx[3] = {0, 0, 0};
-    const unsigned Ny = D >= 2 ? ce.n[1] + 2 * g : 1, Nz = D >= 3 ? ce.n[2] + 2 * g : 1;
-    if (D == 3) { idx[2] = (int)(r % Nz) - g; r /= Nz; }
-    if (D >= 2) { idx[1] = (int)(r % Ny) - g; r /= Ny; }
-    idx[0] = (int)r - g;
-    const int a = idx[AX];
+__device__ __forceinline__ double split_update(const Soa& W, const Soa& Wn, const U<double>& fl, const U<double>& fr, const Ext& ce,
+                                               const int* idx, long m, double dt_d, const Phys& ph, const SplitCfl& cfl) {
+    const int g = ce.g, n = ce.n[AX], a = idx[AX];
     if (a < -g + 1 || a > n + g - 2) {
         for (int f = 0; f < 5; f++) Wn(f, m) = W(f, m);
-        return;
+        return 0.0;
     }
     P<double> w = to_line(load_p<double>(W, m, false), AX);
-    const U<double> fl = to_line(load_u(F, m, false), AX), fr = to_line(load_u(F, m + ce.s[AX], false), AX);
     U<double> u = uadd<false>(cons<false>(w, ph), umul<false>(usub<false>(fl, fr), dt_d));
     w = prim<false>(u, ph);
     if (a == n + g - 2) {  // the sweep's last update: the same flux on both sides
         u = uadd<false>(cons<false>(w, ph), umul<false>(usub<false>(fr, fr), dt_d));
         w = prim<false>(u, ph);
     }
-    store_p<double>(Wn, m, to_line(w, AX), false);
+    w = to_line(w, AX);
+    store_p<double>(Wn, m, w, false);
+    bool interior = cfl.part != nullptr;
+    for (int d = 0; d < D; d++) interior = interior && idx[d] >= 0 && idx[d] < ce.n[d];
+    return interior ? dmax(0.0, cfl_speed_w<D, false>(w, ph, cfl.mode, cfl.d[0], cfl.d[1], cfl.d[2])) : 0.0;  // NaN never wins
+}
+// The update pass of a strided axis.
+template <int D, int AX>
+KB __global__ void k_apply_axis(Soa W, Soa Wn, FSoa F, Ext ce, const StepDts* ts, int half, Phys ph, SplitCfl cfl) {
+    if (stopped(ts)) return;
+    const long m = tid();
+    double v = 0;
+    if (m < ce.size) {
+        const int g = ce.g;
+        unsigned r = (unsigned)m;
+        int idx[3] = {0, 0, 0};
+        const unsigned Ny = D >= 2 ? ce.n[1] + 2 * g : 1, Nz = D >= 3 ? ce.n[2] + 2 * g : 1;
+        if (D == 3) { idx[2] = (int)(r % Nz) - g; r /= Nz; }
+        if (D >= 2) { idx[1] = (int)(r % Ny) - g; r /= Ny; }
+        idx[0] = (int)r - g;
+        U<double> fl = uzero<double>(), fr = fl;
+        if (idx[AX] >= -g + 1 && idx[AX] <= ce.n[AX] + g - 2) {
+            fl = to_line(load_u(F, m, false), AX);
+            fr = to_line(load_u(F, m + ce.s[AX], false), AX);
+        }
+        v = split_update<D, AX>(W, Wn, fl, fr, ce, idx, m, dts(ts, AX, half), ph, cfl);
+    }
+    if (cfl.part) block_max_store(v, cfl.part);  // uniform branch
+}
+// Sweep and update of the contiguous axis in one pass: the lines' cells
+// streamed through wavefronts (sweep_stream_body), 62 of 64 lanes updating
+// their cell from the face below it and the next lane's, so the fluxes stay in
+// registers (1000 x 611 FP64: 44 -> 33 us with the gap between the launches).  Along the strided axes a
+// walker would solve a face more than it has cells: at the lengths that fill
+// the chip (3 to 8) that costs what the flux array does.
+template <int D, class R>
+KS __global__ void k_split_wave(SweepArgs a, Soa Wn, SplitCfl cfl) {
+    constexpr int AX = D - 1;
+    if (stopped(a.ts)) return;
+    const Ext& ce = a.ce;
+    const int g = ce.g, L = ce.n[AX] + 2 * g, n1 = D == 3 ? ce.n[1] + 2 * g : 1, n0 = ce.n[0] + 2 * g;
+    const long wave = (long)block_xcd() * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const long p = 62 * wave - 1 + lane;  // < 2^31: the host sizes grids far below
+    const bool live = p >= 0 && p < (long)n0 * n1 * L;
+    const unsigned q = live ? (unsigned)p : 0u, line = q / (unsigned)L, c = q - line * (unsigned)L;
+    int idx[3] = {0, 0, 0};
+    if (D == 3) { idx[0] = (int)(line / (unsigned)n1) - g; idx[1] = (int)(line % (unsigned)n1) - g; }
+    else idx[0] = (int)line - g;
+    idx[AX] = (int)c - g;
+    const long m = ce.at(idx[0], idx[1], idx[2]);
+    P<R> lo = pzero<R>(), hi = lo;
+    if (live) cell_states<D, false, R, AX, false>(a, idx[0], idx[1], idx[2], lo, hi);
+    const P<R> below = shfl_up1(hi);
+    U<R> f = uzero<R>();
+    if (live && lane >= 1 && c >= 1) f = face_flux_u<false, R, AX>(a, below, lo, m);
+    const U<double> fl{double(f.rho), double(f.E), double(f.mx), double(f.my), double(f.mz), 0, 0, 0};
+    const U<double> fr{double(__shfl_down(f.rho, 1)), double(__shfl_down(f.E, 1)), double(__shfl_down(f.mx, 1)), double(__shfl_down(f.my, 1)),
+                       double(__shfl_down(f.mz, 1)), 0, 0, 0};
+    double v = 0;
+    if (live && lane >= 1 && lane <= 62)
+        v = split_update<D, AX>(a.W, Wn, to_line(fl, AX), to_line(fr, AX), ce, idx, m, a.dt_d(AX), a.ph, cfl);
+    if (cfl.part) block_max_store(v, cfl.part);  // uniform branch
 }
 template <int D, int AX>
-static void split_axis_t(const StepCtx& c, const Soa& in, const Soa& out, hipStream_t s) {
+static long split_axis_t(const StepCtx& c, const Soa& in, const Soa& out, hipStream_t s) {
     if constexpr (AX < D) {
         StepCtx cs = c;
         cs.W = in;
@@ -2911,19 +2978,25 @@ static void split_axis_t(const StepCtx& c, const Soa& in, const Soa& out, hipStr
             hi[d] = ce.n[d] + g;
         }
         const Box b = make_box(D, lo[0], hi[0], lo[1], hi[1], lo[2], hi[2]);
-        sweep<D, false, RT, false>(cs, AX, b, fs(c.F[AX]), ST_FLUX_X + AX, s);
-        hipLaunchKernelGGL((k_apply_axis<D, AX>), dim3(blocks(ce.size)), dim3(256), 0, s, in, out, fs(c.F[AX]), ce, &c.ctl->t, c.half, c.ph);
+        const SplitCfl cfl{c.cflpart, c.cfl_mode, {c.d[0], c.d[1], c.d[2]}};
+        if constexpr (AX == D - 1) {
+            SweepArgs a;
+            if (!sweep_args<D, false, sizeof(RT) == 8, false, AX>(cs, b, fs(c.F[AX]), ST_FLUX_X + AX, a)) return 0;
+            const unsigned n = blocks((ce.size + 61) / 62 * 64);
+            hipLaunchKernelGGL((k_split_wave<D, RT>), dim3(n), dim3(256), 0, s, a, out, cfl);
+            return n;
+        } else {
+            sweep<D, false, RT, false>(cs, AX, b, fs(c.F[AX]), ST_FLUX_X + AX, s);
+            hipLaunchKernelGGL((k_apply_axis<D, AX>), dim3(blocks(ce.size)), dim3(256), 0, s, in, out, fs(c.F[AX]), ce, &c.ctl->t, c.half, c.ph, cfl);
+            return blocks(ce.size);
+        }
     }
+    return 0;
 }
-void launch_split_axis(const StepCtx& c, int ax, Soa in, Soa out, hipStream_t s) {
-    if (c.dim == 2) {
-        if (ax == 0) split_axis_t<2, 0>(c, in, out, s);
-        else split_axis_t<2, 1>(c, in, out, s);
-    } else if (c.dim == 3) {
-        if (ax == 0) split_axis_t<3, 0>(c, in, out, s);
-        else if (ax == 1) split_axis_t<3, 1>(c, in, out, s);
-        else split_axis_t<3, 2>(c, in, out, s);
-    }
+// Returns the CFL maxima left in c.cflpart, where it is set.
+long launch_split_axis(const StepCtx& c, int ax, Soa in, Soa out, hipStream_t s) {
+    if (c.dim == 2) return ax == 0 ? split_axis_t<2, 0>(c, in, out, s) : split_axis_t<2, 1>(c, in, out, s);
+    return ax == 0 ? split_axis_t<3, 0>(c, in, out, s) : ax == 1 ? split_axis_t<3, 1>(c, in, out, s) : split_axis_t<3, 2>(c, in, out, s);
 }
 
 long launch_step(const StepCtx& c, hipStream_t s) {

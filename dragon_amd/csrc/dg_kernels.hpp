@@ -173,7 +173,7 @@ struct BatchArgs {
 #define DG_LAUNCH_INTERFACE                                                                                     \
     void launch_batch_step(const BatchArgs& a, const BlockTable* bt, bool init_only, bool first, bool last, hipStream_t s); \
     long launch_step(const StepCtx& c, hipStream_t s);  /* returns the CFL maxima left in cflpart */              \
-    void launch_split_axis(const StepCtx& c, int ax, Soa in, Soa out, hipStream_t s);  /* one split sweep (hydro) */ \
+    long launch_split_axis(const StepCtx& c, int ax, Soa in, Soa out, hipStream_t s);  /* one split sweep (hydro) */ \
     void launch_bc(const BCArgs& a, bool faces, hipStream_t s);                                                 \
     bool launch_bc_list(BCListArgs& a, hipStream_t s);                                                          \
     void launch_cfl(const StepCtx& c, unsigned long long* out, bool run, hipStream_t s);                        \
