@@ -1128,11 +1128,16 @@ __device__ __forceinline__ void sweep_march_body(const SweepArgs& a, long t) {
 // Occupancy floor of the FP32 walkers: four waves per SIMD for the predictor
 // (133 registers, 8 bytes per lane spilled at four, 5-8% faster than three)
 // and the parked corrector (116-118 registers).  1 = the compiler's choice.
-template <int D, int AX, class R, bool FINAL, class RS> constexpr int march_min_waves() {
+// The FP64 2D hydro corrector is eight registers over three waves: held there
+// it spills 12 bytes per lane.  Hydro 1024^2: 262 -> 250 us per step.  (The 3D
+// hydro one spills 44 to 84: 150 x 128 x 170 2% slower.)
+template <int D, bool MHD, class R, bool FINAL> constexpr bool corrector_2d_hydro() { return D == 2 && !MHD && FINAL && sizeof(R) == 8; }
+template <int D, bool MHD, int AX, class R, bool FINAL, class RS> constexpr int march_min_waves() {
+    if (corrector_2d_hydro<D, MHD, R, FINAL>()) return 3;
     return DG_SWEEP_WAVES == 0 && sizeof(R) == 4 && sizeof(RS) == 4 && (!FINAL || !(D == 3 && AX == 0)) ? 4 : 1;
 }
 template <int D, bool MHD, class R, int AX, bool FINAL, class RS>
-KS __attribute__((amdgpu_waves_per_eu(march_min_waves<D, AX, R, FINAL, RS>()))) __global__ void k_sweep_march(SweepArgs a) {
+KS __attribute__((amdgpu_waves_per_eu(march_min_waves<D, MHD, AX, R, FINAL, RS>()))) __global__ void k_sweep_march(SweepArgs a) {
     if (stopped(a.ts)) return;
     sweep_march_body<D, MHD, R, AX, FINAL, march_window<R>(), false, RS>(a, tid_xcd());
 }
@@ -1329,7 +1334,7 @@ template <class R> KS __global__ void k_corner_wave(SweepArgs a) {
 // [0, n0) sweep x, [n0, n0 + n1) y, the rest z.  (All run at the occupancy of
 // the largest, so large grids keep a launch per axis.)
 template <int D, bool MHD, class R, bool FINAL, class RS>
-KS __global__ void k_sweeps(SweepArgs ax, SweepArgs ay, SweepArgs az, unsigned n0, unsigned n1) {
+KS __attribute__((amdgpu_waves_per_eu(corrector_2d_hydro<D, MHD, R, FINAL>() ? 3 : 1))) __global__ void k_sweeps(SweepArgs ax, SweepArgs ay, SweepArgs az, unsigned n0, unsigned n1) {
     if (stopped(ax.ts)) return;
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     unsigned b = blockIdx.x;
