@@ -2201,18 +2201,26 @@ void launch_soa_to_aos(Soa soa, int nf, double* a, int stride, long n, hipStream
     hipLaunchKernelGGL(k_soa_to_aos, dim3(blocks(n)), dim3(256), 0, s, soa, nf, a, stride, n);
 }
 
+// The CFL passes are bound by their bytes and, where their workgroups are
+// many, by the atomics each adds to one word (about 10 ns each): workgroups
+// enough to keep the loads in flight, no more.  With up to 8192 of them, and
+// the tail's counted from the grid's cells instead of the shell's, k_cfl of
+// 1024^2 hydro took 99 us and each step's tail 28 us.  Frames of steps, before
+// and now: 1024^2 2D hydro 1529 -> 1372 us, 771 x 530 2D MHD 1148 -> 1073,
+// 2048^2 mixed 5205 -> 5023, 150 x 128 x 170 hydro 6231 -> 6019.
 template <int D, bool MHD>
 static void cfl_t(const StepCtx& c, unsigned long long* out, StepCtl* run, hipStream_t s) {
     const int n1 = c.ce.g < 1 ? c.ce.g : 1;
     Box b = make_box(D, -n1, c.ce.n[0] + n1, -n1, c.ce.n[1] + n1, -n1, c.ce.n[2] + n1);
-    const unsigned nb = std::min(blocks(b.count()), 8192u);
+    const unsigned nb = std::min(blocks(b.count()), 1024u);
     hipLaunchKernelGGL((k_cfl<D, MHD>), dim3(nb), dim3(256), 0, s, c.W, c.ce, b, c.ph, c.cfl_mode, c.d[0], c.d[1], c.d[2], out,
                        run, c.cfl_coeff);
 }
 template <int D, bool MHD>
 static void cfl_tail_t(const StepCtx& c, long nparts, unsigned long long* out, StepCtl* run, hipStream_t s) {
-    const long work = nparts + (long)c.ce.n[0] * c.ce.n[1] * c.ce.n[2];  // upper bound; the kernel is grid-stride
-    const unsigned nb = std::min(blocks(work), 2048u);
+    const long n0 = c.ce.n[0] + 2, n1 = c.ce.n[1] + 2, n2 = c.ce.n[2] + 2;
+    const long work = nparts + 2 * (D == 2 ? n0 + n1 : n0 * n1 + n1 * n2 + n2 * n0);  // the maxima and the ghost shell; grid-stride
+    const unsigned nb = std::min(blocks(work), 512u);
     hipLaunchKernelGGL((k_cfl_tail<D, MHD>), dim3(nb), dim3(256), 0, s, c.W, c.ce, c.cflpart, nparts, c.ph, c.cfl_mode, c.d[0], c.d[1],
                        c.d[2], out, run, c.cfl_coeff);
 }
