@@ -119,6 +119,16 @@ template <class R, class T> __device__ __forceinline__ void store_u(const SoaT<T
     a(0, m) = T(u.rho); a(1, m) = T(u.E); a(2, m) = T(u.mx); a(3, m) = T(u.my); a(4, m) = T(u.mz);
     if (mhd) { a(5, m) = T(u.Bx); a(6, m) = T(u.By); a(7, m) = T(u.Bz); }
 }
+// An MHD flux along AX without its normal-B component, always +0 and read by
+// no pass after the sweeps (load_u_nb; the EMFs and CTU corrections take the
+// transverse ones): one field in eight not written.  Frames of steps, before
+// and now: 384^3 mixed 48.7 -> 48.1 ms, 2048^2 mixed 5023 -> 4937 us.
+template <int AX, class R, class T> __device__ __forceinline__ void store_u_nb(const SoaT<T>& a, long m, const U<R>& u) {
+    a(0, m) = T(u.rho); a(1, m) = T(u.E); a(2, m) = T(u.mx); a(3, m) = T(u.my); a(4, m) = T(u.mz);
+    if constexpr (AX != 0) a(5, m) = T(u.Bx);
+    if constexpr (AX != 1) a(6, m) = T(u.By);
+    if constexpr (AX != 2) a(7, m) = T(u.Bz);
+}
 __device__ __forceinline__ void cross(double ux, double uy, double uz, double vx, double vy, double vz, double& wx, double& wy, double& wz) {
     wx = uy * vz - uz * vy;  // Arithmetic.cpp:359-365
     wy = uz * vx - ux * vz;
@@ -988,7 +998,9 @@ __device__ __forceinline__ U<RS> face_flux_u(const SweepArgs& a, const P<R>& l0,
 }
 template <bool MHD, class R, int AX, class RS = R>
 __device__ __forceinline__ void face_flux(const SweepArgs& a, const P<R>& l, const P<R>& r, long m) {
-    store_u<RS>(a.Fo, m, face_flux_u<MHD, R, AX, RS>(a, l, r, m), MHD);
+    const U<RS> f = face_flux_u<MHD, R, AX, RS>(a, l, r, m);
+    if constexpr (MHD) store_u_nb<AX, RS>(a.Fo, m, f);
+    else store_u<RS>(a.Fo, m, f, false);
 }
 
 // Windowed walkers (stencil cells carried in registers) for the FP32 form;
