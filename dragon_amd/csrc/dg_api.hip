@@ -211,22 +211,21 @@ int dg_create(const dg_desc* desc, dg_grid** out) {
     bool ok = hipStreamCreateWithFlags(&g->s, hipStreamNonBlocking) == hipSuccess;
     ok = ok && alloc(&g->W, 8 * nc) && alloc(&g->Wn, 8 * nc);
     // fused sweeps (2D, 3D) need predictor + corrector fluxes, 3D hydro six
-    // corner fluxes instead of the former; 1D keeps the reference's half-state
-    // arrays
-    const bool fusable = d.dim >= 2, hydro3 = !d.mhd && d.dim == 3;
-    g->fused = fusable && getenv("DG_UNFUSED") == nullptr;
+    // corner fluxes instead of the former; the 1D step none
+    const bool hydro3 = !d.mhd && d.dim == 3;
+    g->fused = getenv("DG_UNFUSED") == nullptr;
     // diagnostic: fixed faces per walker of the strided-axis sweeps (results do not depend on it)
     if (const char* mc = getenv("DG_MARCH_CHUNK")) g->march_chunk = atoi(mc);
     // check: the FP64 walkers take the register-window form the FP32 build
     // uses, so the FP64 parity tests hold that form to the oracle bit for bit
     g->march_window = getenv("DG_MARCH_WINDOW_CHECK") != nullptr;
-    ok = ok && alloc(&g->F, (long)d.dim * g->nf * nc);
-    if (g->fused) ok = ok && (!d.ctu || hydro3 || alloc(&g->Fp, (long)d.dim * g->nf * nc));
+    if (!g->fused || d.dim >= 2) ok = ok && alloc(&g->F, (long)d.dim * g->nf * nc);
+    if (g->fused) ok = ok && (!d.ctu || hydro3 || d.dim == 1 || alloc(&g->Fp, (long)d.dim * g->nf * nc));
     else ok = ok && alloc(&g->HS, 2L * d.dim * g->nf * nc);
     if (hydro3 && d.ctu) ok = ok && alloc(&g->T, (g->fused ? 6L : 5L) * g->nf * nc);
     if (faces) ok = ok && alloc(&g->B, 3 * nfc) && alloc(&g->Bn, 3 * nfc) && alloc(&g->Bh, 3 * nfc) && alloc(&g->E0, 3 * nfc) &&
                     alloc(&g->Eh, 3 * nfc);
-    if (d.dim >= 2) {
+    if (d.dim >= 2 || g->fused) {
         // one per workgroup of the pass that writes the next state
         const long parts = d.dim == 2 ? ct_tiles(d.nx + 1 + 2 * gh, d.ny + 1 + 2 * gh) : 0;
         ok = ok && alloc(&g->cflpart, std::max(parts, nc / 248 + 2));
@@ -410,9 +409,10 @@ static void apply_one(dg_grid* g, const dg_bc& b) {
     }
 }
 
-// The implicit Outflow `imp` and then the list in one launch; false (nothing
-// done) where its passes do not fit one (launch_bc_list).
-static bool apply_list(dg_grid* g, const dg_bc& imp) {
+// The implicit Outflow `imp` and then the list in one launch, with the CFL
+// tail of the run's step `tail` where given; false (nothing done) where its
+// passes do not fit one (launch_bc_list, launch_bc_tail).
+static bool apply_list(dg_grid* g, const dg_bc& imp, const StepCtx* tail) {
     const int D = g->d.dim;
     const bool faces = g->d.mhd && D >= 2;
     BCListArgs a{};
@@ -436,7 +436,7 @@ static bool apply_list(dg_grid* g, const dg_bc& imp) {
     if (!add(imp)) return false;
     for (auto& b : g->bcs)
         if (!add(b)) return false;
-    return launch_bc_list(a, g->s);
+    return tail ? launch_bc_tail(a, *tail, g->ncflpart, g->s) : launch_bc_list(a, g->s);
 }
 
 // One element applied alone, without the list's implicit Outflow: the step
@@ -460,7 +460,10 @@ int dg_set_boundary_callback(dg_grid* g, int (*cb)(void* user), void* user) {
     return DG_OK;
 }
 
-int dg_apply_boundary(dg_grid* g) {
+static int apply_boundary(dg_grid* g, const StepCtx* tail, bool* tailed);
+int dg_apply_boundary(dg_grid* g) { return apply_boundary(g, nullptr, nullptr); }
+// tail: the step of a run whose CFL tail may go with the boundary (*tailed).
+static int apply_boundary(dg_grid* g, const StepCtx* tail, bool* tailed) {
     if (!g) return DG_ERR_ARG;
     if (g->bc_cb) {  // the caller applies the list itself (host-evaluated elements)
         g->cfl_cached = false;
@@ -472,7 +475,8 @@ int dg_apply_boundary(dg_grid* g) {
     dg_bc imp{};
     imp.kind = DG_BC_OUTFLOW; imp.faces = uncovered; imp.corners = 1; imp.gated = 0;
     tm_record(g, -1);
-    if (!apply_list(g, imp)) {
+    if (tail) *tailed = apply_list(g, imp, tail);
+    if (!(tail && *tailed) && !apply_list(g, imp, nullptr)) {
         apply_one(g, imp);
         for (auto& b : g->bcs) apply_one(g, b);
     }
@@ -662,9 +666,11 @@ static int advance_run(dg_grid* g, double left, int check_cfl, int n, int* done,
     int rc = DG_OK;
     bool cached = g->cfl_cached;
     for (int k = 0; k < n && rc == DG_OK; k++) {
-        rc = dg_apply_boundary(g);
         StepCtx c = make_ctx(g);
-        if (!check_cfl) launch_ctl_next(c, g->s);
+        bool begun = false;
+        rc = apply_boundary(g, check_cfl && cached ? &c : nullptr, &begun);
+        if (begun) {}
+        else if (!check_cfl) launch_ctl_next(c, g->s);
         else if (cached) launch_cfl_tail(c, g->ncflpart, nullptr, true, g->s);
         else launch_cfl(c, nullptr, true, g->s);
         g->ncflpart = c.mixed ? p32::launch_step(c, g->s) : p64::launch_step(c, g->s);
@@ -1069,9 +1075,9 @@ extern "C" int dg_step_noalloc(const dg_desc* desc, const double* w_in, const do
     g.ce = make_ext(d.dim, d.nx, d.ny, d.nz, gh);
     g.fe = make_ext(d.dim, d.nx + 1, d.ny + 1, d.nz + 1, gh);
     g.ph = make_phys(d);
-    g.fused = d.dim >= 2;
+    g.fused = true;
     const bool hydro3 = !d.mhd && d.dim == 3;
-    const NoallocLayout L = noalloc_layout(d, g.ce, g.fe, g.fused && !hydro3);
+    const NoallocLayout L = noalloc_layout(d, g.ce, g.fe, d.dim >= 2 && !hydro3);
     g.W = const_cast<double*>(w_in);
     g.Wn = w_out;
     if (faces) { g.B = const_cast<double*>(B_in); g.Bn = B_out; }

@@ -358,8 +358,10 @@ __host__ __device__ inline BCShell cell_shell(const Ext& ce, int dim) { return B
 __host__ __device__ inline BCShell face_shell(const Ext& ce, int dim) {
     return BCShell{dim, {ce.n[0] - 1, ce.n[1] - 1, ce.n[2] - 1}, ce.g + 1, ce.g + 1};
 }
-// Fields [f0, f1) of the t-th ghost cell.
-__device__ __forceinline__ void bc_list_cell(const BCPass* ps, int np, int dim, const Soa& W, const Ext& ce, unsigned t, int f0, int f1) {
+// Fields [f0, f1) of the t-th ghost cell.  out: the cell's fields after the
+// list, whether a pass writes it or not (f0 = 0).
+__device__ __forceinline__ void bc_list_cell(const BCPass* ps, int np, int dim, const Soa& W, const Ext& ce, unsigned t, int f0, int f1,
+                                             double* out = nullptr) {
     int i, j, k;
     cell_shell(ce, dim).point(t, i, j, k);
     const long dst = ce.at(i, j, k);
@@ -385,12 +387,13 @@ __device__ __forceinline__ void bc_list_cell(const BCPass* ps, int np, int dim, 
         }
         if (ax == 0) i = y; else if (ax == 1) j = y; else k = y;
     }
-    if (!hit) return;
+    if (!hit && !out) return;
     const long src = ce.at(i, j, k);
     auto finish = [&](int f, double v) {
         if (neg >> f & 1) v *= -1;
         if ((in_lo >> f & 1 && v > 0) || (in_hi >> f & 1 && v < 0)) v = 0;
-        W(f, dst) = v;
+        if (hit) W(f, dst) = v;
+        if (out) out[f] = v;
     };
     if (f1 - f0 == 1) {
         finish(f0, fixed >= 0 ? ps[fixed].st[f0] : W(f0, src));
@@ -528,18 +531,22 @@ __device__ __forceinline__ double cfl_speed_at(const Soa& W, const Ext& ce, int 
                                                double dy, double dz) {
     return cfl_speed_w<D, MHD>(load_p<double>(W, ce.at(i, j, k), MHD), ph, mode, dx, dy, dz);
 }
-// Block max of per-thread values into part[blockIdx.x] (plain store, no atomics).
-__device__ __forceinline__ void block_max_store(double m, double* part) {
+// Block max of per-thread values, in thread 0.
+__device__ __forceinline__ double block_max(double m) {
     for (int off = 32; off > 0; off >>= 1) m = dmax(m, __shfl_xor(m, off));
     __shared__ double wmax[4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane == 0) wmax[wave] = m;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double b = wmax[0];
+    double b = wmax[0];
+    if (threadIdx.x == 0)
         for (int q = 1; q < (int)(blockDim.x >> 6); q++) b = dmax(b, wmax[q]);
-        part[blockIdx.x] = b;
-    }
+    return b;
+}
+// The same into part[blockIdx.x] (plain store, no atomics).
+__device__ __forceinline__ void block_max_store(double m, double* part) {
+    const double b = block_max(m);
+    if (threadIdx.x == 0) part[blockIdx.x] = b;
 }
 // Begins the next step of a run: dt = min(time left, cfl) from the gathered
 // maximum (D: dimension, 0: no CFL), and the words of the step cleared.  One
@@ -633,7 +640,7 @@ KB __global__ void k_cfl_tail(Soa W, Ext ce, const double* part, long nparts, Ph
         } else if (r < 2 * (sx + sy)) {
             r -= 2 * sx;
             j = r < sy ? -1 : (int)n1;
-            r %= sy;
+            r %= (sy > 0 ? sy : 1);  // as sz: no y faces in 1D
             if (D == 3) { i = (int)(r / (n2 + 2)); k = (int)(r % (n2 + 2)) - 1; }
             else i = (int)r;
         } else {
@@ -644,16 +651,38 @@ KB __global__ void k_cfl_tail(Soa W, Ext ce, const double* part, long nparts, Ph
         }
         m = dmax(m, cfl_speed_at<D, MHD>(W, ce, i, j, k, ph, mode, dx, dy, dz));
     }
-    for (int off = 32; off > 0; off >>= 1) m = dmax(m, __shfl_xor(m, off));
-    __shared__ double wmax[4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) wmax[wave] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double b = wmax[0];
-        for (int q = 1; q < (int)(blockDim.x >> 6); q++) b = dmax(b, wmax[q]);
-        cfl_finish(b, out, run, D, coeff, dx, dy, dz);
+    const double b = block_max(m);
+    if (threadIdx.x == 0) cfl_finish(b, out, run, D, coeff, dx, dy, dz);
+}
+// The boundary list and the tail in one launch, in a run: a thread takes a
+// ghost cell whole, and its signal speed too where it lies in the shell, a
+// boundary face's component or one of the maxima.  At small sizes each of the
+// two launches is 4 to 6 us, next to nothing of it work.  Frames of steps,
+// apart and together: 1024^2 2D hydro 1372 -> 1296 us, 771 x 530 2D MHD 1073 ->
+// 1049, 128^2 530 -> 507, 64 x 32 x 32 3D MHD 791 -> 774.
+template <int D, bool MHD>
+KB __global__ void k_bc_tail(BCListArgs a, const double* part, unsigned nparts, Phys ph, int mode, double dx, double dy, double dz,
+                             StepCtl* run, double coeff) {
+    if (cfl_run_over(run)) return;
+    const unsigned faces = a.ncell + 3 * a.nface, all = faces + nparts, stride = gridDim.x * 256;
+    double m = 0;
+    for (unsigned t = (unsigned)tid(); t < all; t += stride) {
+        if (t >= faces) {
+            m = dmax(m, part[t - faces]);
+        } else if (t >= a.ncell) {
+            bc_list_face(a.p, a.npass, D, a.B, a.ce, a.fe, (t - a.ncell) % a.nface, (int)((t - a.ncell) / a.nface));
+        } else {
+            int i, j, k;
+            cell_shell(a.ce, D).point(t, i, j, k);
+            double u[8] = {};
+            bc_list_cell(a.p, a.npass, D, a.W, a.ce, t, 0, MHD ? 8 : 5, u);
+            if (i < -1 || i > a.ce.n[0] || (D >= 2 && (j < -1 || j > a.ce.n[1])) || (D >= 3 && (k < -1 || k > a.ce.n[2]))) continue;
+            const P<double> w{u[F_RHO], u[F_P], u[F_VX], u[F_VY], u[F_VZ], u[F_BX], u[F_BY], u[F_BZ]};
+            m = dmax(m, cfl_speed_w<D, MHD>(w, ph, mode, dx, dy, dz));
+        }
     }
+    const double b = block_max(m);
+    if (threadIdx.x == 0) cfl_finish(b, nullptr, run, D, coeff, dx, dy, dz);
 }
 template <int D, bool MHD>
 KB __global__ void k_cfl(Soa W, Ext ce, Box box, Phys ph, int mode, double dx, double dy, double dz, unsigned long long* out,
@@ -664,16 +693,8 @@ KB __global__ void k_cfl(Soa W, Ext ce, Box box, Phys ph, int mode, double dx, d
     const long cnt = box.count(), stride = (long)gridDim.x * blockDim.x;
     for (long t = tid(); t < cnt; t += stride)  // grid-stride: few blocks, few atomics
         if (box.point(t, i, j, k)) m = dmax(m, cfl_speed_at<D, MHD>(W, ce, i, j, k, ph, mode, dx, dy, dz));  // NaN never wins
-    for (int off = 32; off > 0; off >>= 1) m = dmax(m, __shfl_xor(m, off));
-    __shared__ double part[4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) part[wave] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double b = part[0];
-        for (int q = 1; q < (int)(blockDim.x >> 6); q++) b = dmax(b, part[q]);
-        cfl_finish(b, out, run, D, coeff, dx, dy, dz);
-    }
+    const double b = block_max(m);
+    if (threadIdx.x == 0) cfl_finish(b, out, run, D, coeff, dx, dy, dz);
 }
 
 // ============================================================ half states
@@ -2092,6 +2113,63 @@ KB __global__ void k_apply1(Soa W, Soa Wn, FSoa F, Ext ce, const StepDts* ts, Ph
     store_p<double>(Wn, m, w, MHD);
 }
 
+// The whole 1D step in one pass: half states, fluxes and the update, handed
+// from lane to lane of a wavefront, and the CFL maximum of the next state.
+// Lane l rebuilds cell 62 w + l - 1 and solves the face below it; lanes 1 ..
+// 62 update their cells (2 lanes in 64 repeat a neighbour's work, with the same
+// bits).  Bound by latency on the grids 1D problems have: the three separate
+// passes cost 12 us of launches, arrays written and read back, and a CFL scan
+// of every cell.  1024 cells, a frame of 20 steps, with the boundary and the
+// CFL in one launch too: 495 -> 329 us.
+constexpr int STEP1_CELLS = 4 * 62;  // per workgroup of four wavefronts
+template <class R> __device__ __forceinline__ U<double> flux_down1(const U<R>& f) {
+    return U<double>{__shfl_down(f.rho, 1), __shfl_down(f.E, 1), __shfl_down(f.mx, 1), __shfl_down(f.my, 1),
+                     __shfl_down(f.mz, 1), __shfl_down(f.Bx, 1), __shfl_down(f.By, 1), __shfl_down(f.Bz, 1)};
+}
+template <bool MHD, class R>
+KS __global__ void k_step1(Soa W, Soa Wn, Ext ce, const StepDts* ts, Phys ph, unsigned long long* err, double* cflpart) {
+    if (stopped(ts)) return;
+    const double dt_dx = dts(ts, 0);
+    const int lane = threadIdx.x & 63, g = ce.g, n = ce.n[0];
+    const long m = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * 62 + lane - 1;
+    const int i = (int)m - g;
+    const bool live = m >= 0 && m < ce.size;
+    P<double> w{};
+    P<R> L = pzero<R>(), Rr = pzero<R>();
+    if (live) {
+        w = load_p<double>(W, m, MHD);
+        const P<R> wc = p_cast<R>(w);
+        if (i >= -g + 1 && i < n + g - 1)
+            muscl<MHD, R>(load_p<R>(W, m - 1, MHD), L, wc, Rr, load_p<R>(W, m + 1, MHD), R(dt_dx), R(0), R(0), R(0), ph);
+        else
+            L = Rr = wc;
+    }
+    const P<R> l = shfl_up1(Rr);
+    U<R> f = uzero<R>();
+    if (live && lane >= 1 && i >= -g + 1) {
+        int fail = RF_OK;
+        f = riemann_x<MHD, R>(l, L, R(dt_dx), ph, &fail);
+        if (fail) report(err, ST_FLUX_X, (unsigned long long)m, fail == RF_BAD_INPUT ? E_RIEMANN_INPUT : E_RIEMANN_SOLUTION);
+    }
+    const U<double> fr = flux_down1(f);
+    double speed = 0;
+    if (live && lane >= 1 && lane <= 62) {
+        if (i < -g + 1 || i > n + g - 2) {
+            store_p<double>(Wn, m, w, MHD);
+        } else {
+            const U<double> fl{double(f.rho), double(f.E), double(f.mx), double(f.my), double(f.mz), double(f.Bx), double(f.By), double(f.Bz)};
+            w = prim<MHD>(uadd<MHD>(cons<MHD>(w, ph), umul<MHD>(usub<MHD>(fl, fr), dt_dx)), ph);
+            if (i == n + g - 2) w = prim<MHD>(uadd<MHD>(cons<MHD>(w, ph), umul<MHD>(usub<MHD>(fr, fr), dt_dx)), ph);
+            if (i >= 0 && i < n) {
+                if (!physical<MHD>(w)) report(err, ST_UNPHYSICAL, (unsigned long long)m, E_UNPHYSICAL);
+                speed = dmax(0.0, cfl_speed_w<1, MHD>(w, ph, 0, 1.0, 1.0, 1.0));  // NaN never wins
+            }
+            store_p<double>(Wn, m, w, MHD);
+        }
+    }
+    if (cflpart) block_max_store(speed, cflpart);
+}
+
 // AoS <-> SoA staging for upload/download in the reference's record layout.
 KB __global__ void k_aos_to_soa(const double* a, int stride, int nf, Soa s, long n) {
     const long m = tid();
@@ -2176,8 +2254,8 @@ constexpr unsigned BC_WHOLE = 65536;  // ghost cells from which a thread copies 
 // False where the list does not fit k_bc_list: an axis with a pass and fewer
 // than ng + 2 cells, two passes on one face, a periodic axis with another
 // pass, or more threads than 32 bits count.
-bool launch_bc_list(BCListArgs& a, hipStream_t s) {
-    if (a.npass == 0) return true;
+// Whether the list's passes fit one launch; counts its points.
+static bool bc_list_fits(BCListArgs& a) {
     int on[3] = {0, 0, 0}, periodic[3] = {0, 0, 0};
     for (int q = 0; q < a.npass; q++) {
         const BCPass& p = a.p[q];
@@ -2198,6 +2276,11 @@ bool launch_bc_list(BCListArgs& a, hipStream_t s) {
     if (cells * a.nf + fcs * 3 > 2e9) return false;
     a.ncell = cell_shell(a.ce, a.dim).count();
     a.nface = faces ? face_shell(a.ce, a.dim).count() : 0;
+    return true;
+}
+bool launch_bc_list(BCListArgs& a, hipStream_t s) {
+    if (a.npass == 0) return true;
+    if (!bc_list_fits(a)) return false;
     if (a.ncell >= BC_WHOLE) hipLaunchKernelGGL(k_bc_list<true>, dim3(blocks((long)a.ncell + a.nface)), dim3(256), 0, s, a);
     else hipLaunchKernelGGL(k_bc_list<false>, dim3(blocks((long)a.ncell * a.nf + 3L * a.nface)), dim3(256), 0, s, a);
     return true;
@@ -2231,15 +2314,33 @@ static void cfl_t(const StepCtx& c, unsigned long long* out, StepCtl* run, hipSt
 template <int D, bool MHD>
 static void cfl_tail_t(const StepCtx& c, long nparts, unsigned long long* out, StepCtl* run, hipStream_t s) {
     const long n0 = c.ce.n[0] + 2, n1 = c.ce.n[1] + 2, n2 = c.ce.n[2] + 2;
-    const long work = nparts + 2 * (D == 2 ? n0 + n1 : n0 * n1 + n1 * n2 + n2 * n0);  // the maxima and the ghost shell; grid-stride
+    const long work = nparts + 2 * (D == 1 ? 1 : D == 2 ? n0 + n1 : n0 * n1 + n1 * n2 + n2 * n0);  // the maxima and the ghost shell; grid-stride
     const unsigned nb = std::min(blocks(work), 512u);
     hipLaunchKernelGGL((k_cfl_tail<D, MHD>), dim3(nb), dim3(256), 0, s, c.W, c.ce, c.cflpart, nparts, c.ph, c.cfl_mode, c.d[0], c.d[1],
                        c.d[2], out, run, c.cfl_coeff);
 }
 void launch_cfl_tail(const StepCtx& c, long nparts, unsigned long long* out, bool run, hipStream_t s) {
     StepCtl* r = run ? c.ctl : nullptr;
-    if (c.dim == 2) c.mhd ? cfl_tail_t<2, true>(c, nparts, out, r, s) : cfl_tail_t<2, false>(c, nparts, out, r, s);
+    if (c.dim == 1) c.mhd ? cfl_tail_t<1, true>(c, nparts, out, r, s) : cfl_tail_t<1, false>(c, nparts, out, r, s);
+    else if (c.dim == 2) c.mhd ? cfl_tail_t<2, true>(c, nparts, out, r, s) : cfl_tail_t<2, false>(c, nparts, out, r, s);
     else c.mhd ? cfl_tail_t<3, true>(c, nparts, out, r, s) : cfl_tail_t<3, false>(c, nparts, out, r, s);
+}
+// In a run, the list and the CFL tail in one launch; false (nothing done)
+// where the list does not fit one, or where its shell is large: the launches
+// are then nothing next to their work, and the tail's registers slow the ghost
+// copies.
+template <int D, bool MHD>
+static void bc_tail_t(const BCListArgs& a, const StepCtx& c, long nparts, hipStream_t s) {
+    const unsigned nb = std::min(blocks((long)a.ncell + 3L * a.nface + nparts), 256u);  // grid-stride; few, for the atomics (cfl_t)
+    hipLaunchKernelGGL((k_bc_tail<D, MHD>), dim3(nb), dim3(256), 0, s, a, c.cflpart, (unsigned)nparts, c.ph, c.cfl_mode, c.d[0], c.d[1],
+                       c.d[2], c.ctl, c.cfl_coeff);
+}
+bool launch_bc_tail(BCListArgs& a, const StepCtx& c, long nparts, hipStream_t s) {
+    if (a.npass == 0 || !bc_list_fits(a) || a.ncell >= BC_WHOLE) return false;
+    if (c.dim == 1) c.mhd ? bc_tail_t<1, true>(a, c, nparts, s) : bc_tail_t<1, false>(a, c, nparts, s);
+    else if (c.dim == 2) c.mhd ? bc_tail_t<2, true>(a, c, nparts, s) : bc_tail_t<2, false>(a, c, nparts, s);
+    else c.mhd ? bc_tail_t<3, true>(a, c, nparts, s) : bc_tail_t<3, false>(a, c, nparts, s);
+    return true;
 }
 void launch_cfl(const StepCtx& c, unsigned long long* out, bool run, hipStream_t s) {
     StepCtl* r = run ? c.ctl : nullptr;
@@ -2495,6 +2596,14 @@ static long step_t(const StepCtx& c, hipStream_t s) {
     }
     const Ext& ce = c.ce;
     const int g = ce.g;
+    if constexpr (D == 1) {
+        if (c.fused) {
+            const unsigned nb = (unsigned)((ce.size + STEP1_CELLS - 1) / STEP1_CELLS);
+            hipLaunchKernelGGL((k_step1<MHD, R>), dim3(nb), dim3(256), 0, s, c.W, c.Wn, ce, &c.ctl->t, c.ph, c.err, c.cflpart);
+            mark(c, K_APPLY);
+            return nb;
+        }
+    }
     // half states
     {
         Box all = make_box(D, -g, ce.n[0] + g, -g, ce.n[1] + g, -g, ce.n[2] + g);

@@ -178,6 +178,7 @@ struct BatchArgs {
     bool launch_bc_list(BCListArgs& a, hipStream_t s);                                                          \
     void launch_cfl(const StepCtx& c, unsigned long long* out, bool run, hipStream_t s);                        \
     void launch_cfl_tail(const StepCtx& c, long nparts, unsigned long long* out, bool run, hipStream_t s);      \
+    bool launch_bc_tail(BCListArgs& a, const StepCtx& c, long nparts, hipStream_t s);  /* list and tail, in a run */  \
     void launch_ctl_set(const StepCtx& c, double dt, hipStream_t s);        /* one step of size dt */             \
     void launch_ctl_begin(const StepCtx& c, double left, double tol, hipStream_t s);  /* a run of steps */        \
     void launch_ctl_next(const StepCtx& c, hipStream_t s);                  /* its next step, without CFL */      \
