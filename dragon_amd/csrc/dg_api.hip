@@ -45,8 +45,8 @@ struct dg_grid {
     bool cfl_cached = false;    // cflpart describes the current W (set by a committed step)
     unsigned long long* dev_words = nullptr;   // [1] CFL max bits, [2..3] diagnostics
     unsigned long long* host_words = nullptr;  // pinned mirror
-    StepCtl* ctl = nullptr;                    // device: step sizes, failure word, control of a run of steps
-    StepCtl* host_ctl = nullptr;               // pinned mirror
+    StepCtl* ctl = nullptr;                    // device, behind dev_words: step sizes, failure word, control of a run of steps
+    StepCtl* host_ctl = nullptr;               // its pinned mirror, behind host_words
     bool in_run = false;                       // the launches belong to a run of steps (advance_run)
     std::string err;
     // optional live timing of the step kernels with HIP events
@@ -230,10 +230,12 @@ int dg_create(const dg_desc* desc, dg_grid** out) {
         const long parts = d.dim == 2 ? ct_tiles(d.nx + 1 + 2 * gh, d.ny + 1 + 2 * gh) : 0;
         ok = ok && alloc(&g->cflpart, std::max(parts, nc / 248 + 2));
     }
-    ok = ok && hipMalloc((void**)&g->dev_words, 4 * sizeof(unsigned long long)) == hipSuccess;
-    ok = ok && hipHostMalloc((void**)&g->host_words, 4 * sizeof(unsigned long long), hipHostMallocDefault) == hipSuccess;
-    ok = ok && hipMalloc((void**)&g->ctl, sizeof(StepCtl)) == hipSuccess;
-    ok = ok && hipHostMalloc((void**)&g->host_ctl, sizeof(StepCtl), hipHostMallocDefault) == hipSuccess;
+    // the control words behind the others, in one allocation each
+    const size_t words = 4 * sizeof(unsigned long long);
+    ok = ok && hipMalloc((void**)&g->dev_words, words + sizeof(StepCtl)) == hipSuccess;
+    ok = ok && hipHostMalloc((void**)&g->host_words, words + sizeof(StepCtl), hipHostMallocDefault) == hipSuccess;
+    g->ctl = ok ? (StepCtl*)(g->dev_words + 4) : nullptr;
+    g->host_ctl = ok ? (StepCtl*)(g->host_words + 4) : nullptr;
     if (!ok) {
         dg_destroy(g);
         return DG_ERR_HIP;
@@ -263,8 +265,6 @@ int dg_destroy(dg_grid* g) {
         if (p && hipFree(p) != hipSuccess) rc = DG_ERR_HIP;
     if (g->dev_words && hipFree(g->dev_words) != hipSuccess) rc = DG_ERR_HIP;
     if (g->host_words && hipHostFree(g->host_words) != hipSuccess) rc = DG_ERR_HIP;
-    if (g->ctl && hipFree(g->ctl) != hipSuccess) rc = DG_ERR_HIP;
-    if (g->host_ctl && hipHostFree(g->host_ctl) != hipSuccess) rc = DG_ERR_HIP;
     if (g->ev0 && hipEventDestroy(g->ev0) != hipSuccess) rc = DG_ERR_HIP;
     if (g->ev1 && hipEventDestroy(g->ev1) != hipSuccess) rc = DG_ERR_HIP;
     for (hipEvent_t e : g->evs)
