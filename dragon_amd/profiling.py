@@ -35,20 +35,28 @@ import re
 
 # demangled kernel name -> the kernel class of dg_kernel_time()
 _CLASSES = [
-    (r"k_sweep_(march|wave)<\d, (true|false), (double|float), (\d), false>", lambda m: "pred_sweep_" + "xyz"[int(m.group(4))]),
-    (r"k_sweep_(march|wave)<\d, (true|false), (double|float), (\d), true>", lambda m: "flux_sweep_" + "xyz"[int(m.group(4))]),
+    (r"k_sweep_(march|wave)<\d, (true|false), (double|float), (\d), false[,>]", lambda m: "pred_sweep_" + "xyz"[int(m.group(4))]),
+    (r"k_sweep_(march|wave)<\d, (true|false), (double|float), (\d), true[,>]", lambda m: "flux_sweep_" + "xyz"[int(m.group(4))]),
+    (r"k_sweeps<\d, (true|false), (double|float), false[,>]", "pred_sweeps (all axes)"),
+    (r"k_sweeps<\d, (true|false), (double|float), true[,>]", "flux_sweeps (all axes)"),
+    (r"k_corner_(march|wave)<", "ctu_correct"),
+    (r"k_ct_half2", "ct half step (2D)"),
+    (r"k_ct_final2", "ct + apply (2D)"),
     (r"k_emf[23]<true>", "emf_pred"),
     (r"k_emf[23]<false>", "emf"),
     (r"k_emf3_tiled\(", "emf (predictor + final)"),  # one kernel for both EMFs of the 3D step
     (r"k_faraday<", "faraday (half + final)"),
     (r"k_whalf<", "whalf"),
-    (r"k_apply1?<", "apply"),
-    (r"k_cfl<", "cfl"),
-    (r"k_bc_(cells|faces)", "boundary"),
+    (r"k_(apply1?|apply_axis)<", "apply"),
+    (r"k_step1<", "1D step"),
+    (r"k_split_wave<", "split sweep + apply"),
+    (r"k_cfl(_tail)?<", "cfl"),
+    (r"k_bc_tail<", "boundary + cfl"),
+    (r"k_bc_(cells|faces|list)", "boundary"),
     (r"k_half<", "half_states"),
     (r"k_flux<", "flux (reference-structured path)"),
     (r"k_(correct|ctu_flux|ctu_mhd)<", "ctu_correct"),
-    (r"k_fill_u64", "failure-word reset"),
+    (r"k_(fill_u64|ctl_\w+)", "control words"),
     (r"k_init_B<", "init (initialize_B_fields)"),
     (r"k_divb<", "diagnostic (div B)"),
     (r"k_(aos_to_soa|soa_to_aos)", "layout transfer"),
