@@ -1249,6 +1249,7 @@ static BatchArgs batch_args(const dg_batch* b, int commit, int cls_filter) {
     a.cfl_coeff = b->d.cfl_coeff; a.tol = b->d.timestep_tol > 0 ? b->d.timestep_tol : 1e-14;
     a.cfl_mode = b->d.cfl_mode;
     for (int q = 0; q < 4; q++) a.bc.p[q] = BCPass{q / 2, q % 2, b->bc_kind, 0, {}};
+    for (int q = 0; q < 4; q++) a.bc.heads |= bc_head(a.bc.p[q]) << (8 * q);
     for (int c = 0; c < BATCH_CLASSES; c++) { a.chunk[c] = b->chunk[c]; a.ysw[c] = b->ysw[c]; }
     a.commit = commit; a.cls_filter = cls_filter;
     return a;

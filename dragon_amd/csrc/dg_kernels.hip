@@ -147,7 +147,8 @@ __device__ __forceinline__ double dts(const StepDts* t, int q, bool half = false
 // word before its first load costs Faraday 3%.
 __device__ __forceinline__ bool stopped(const StepDts* t) { return ((DtsPtr)t)->stop != 0; }
 // A run of steps is over: the step before this launch failed, or no time is left.
-__device__ __forceinline__ bool run_over(const StepCtl* c) { return c->t.stop || c->err != ~0ull || !(c->left_next > c->tol); }
+// (All four words read at once: with || they would be a chain of loads.)
+__device__ __forceinline__ bool run_over(const StepCtl* c) { return (c->t.stop != 0) | (c->err != ~0ull) | !(c->left_next > c->tol); }
 
 // ===================================================================== BC
 // One thread per transverse index of a face; it runs the reference's ghost
@@ -358,9 +359,17 @@ __host__ __device__ inline BCShell cell_shell(const Ext& ce, int dim) { return B
 __host__ __device__ inline BCShell face_shell(const Ext& ce, int dim) {
     return BCShell{dim, {ce.n[0] - 1, ce.n[1] - 1, ce.n[2] - 1}, ce.g + 1, ce.g + 1};
 }
+// What the walk needs of pass q (bc_head).
+struct BCHead {
+    int axis, side, kind, gated;
+    __device__ __forceinline__ BCHead(unsigned long long heads, int q) {
+        const unsigned h = (unsigned)(heads >> (8 * q)) & 255u;
+        axis = h & 3; side = h >> 2 & 1; kind = h >> 3 & 3; gated = h >> 5;
+    }
+};
 // Fields [f0, f1) of the t-th ghost cell.  out: the cell's fields after the
 // list, whether a pass writes it or not (f0 = 0).
-__device__ __forceinline__ void bc_list_cell(const BCPass* ps, int np, int dim, const Soa& W, const Ext& ce, unsigned t, int f0, int f1,
+__device__ __forceinline__ void bc_list_cell(unsigned long long heads, const BCPass* ps, int np, int dim, const Soa& W, const Ext& ce, unsigned t, int f0, int f1,
                                              double* out = nullptr) {
     int i, j, k;
     cell_shell(ce, dim).point(t, i, j, k);
@@ -369,7 +378,7 @@ __device__ __forceinline__ void bc_list_cell(const BCPass* ps, int np, int dim, 
     bool hit = false;
     int fixed = -1;  // the pass whose state the cell takes
     for (int q = np - 1; q >= 0 && fixed < 0; q--) {
-        const BCPass& p = ps[q];
+        const BCHead p(heads, q);
         const int ax = p.axis, n = ax == 0 ? ce.n[0] : ax == 1 ? ce.n[1] : ce.n[2], x = ax == 0 ? i : ax == 1 ? j : k;
         if (p.side == 0 ? x >= 0 : x < n) continue;
         hit = true;
@@ -407,7 +416,7 @@ __device__ __forceinline__ void bc_list_cell(const BCPass* ps, int np, int dim, 
     for (int f = 0; f < 8; f++)
         if (f < f1) finish(f, v[f]);
 }
-__device__ __forceinline__ void bc_list_face(const BCPass* ps, int np, int dim, double* const Bc[3], const Ext& ce, const Ext& fe, unsigned t,
+__device__ __forceinline__ void bc_list_face(unsigned long long heads, const BCPass* ps, int np, int dim, double* const Bc[3], const Ext& ce, const Ext& fe, unsigned t,
                                              int c) {
     int i, j, k;
     face_shell(ce, dim).point(t, i, j, k);
@@ -421,7 +430,7 @@ __device__ __forceinline__ void bc_list_face(const BCPass* ps, int np, int dim, 
     int ext = 0, exg = 0;  // extrapolation of the normal component: side + 1, faces beyond the last one kept
     bool hit = false, fixed = false;
     for (int q = np - 1; q >= 0 && !fixed; q--) {
-        const BCPass& p = ps[q];
+        const BCHead p(heads, q);
         const int ax = p.axis, n = ax == 0 ? ce.n[0] : ax == 1 ? ce.n[1] : ce.n[2], x = ax == 0 ? i : ax == 1 ? j : k;
         const bool normal = c == ax;
         int y = x;
@@ -450,7 +459,7 @@ __device__ __forceinline__ void bc_list_face(const BCPass* ps, int np, int dim, 
         }
         hit = true;
         if (p.kind == 3) {
-            v = p.st[F_BX + c];
+            v = ps[q].st[F_BX + c];
             fixed = true;
             ext = 0;  // the extrapolation of equal values
         }
@@ -479,17 +488,17 @@ __device__ __forceinline__ void bc_list_face(const BCPass* ps, int np, int dim, 
 template <bool WHOLE>
 __device__ __forceinline__ void bc_list_body(const BCListArgs& a, const Ext& ce, const Ext& fe, unsigned t) {
     if (WHOLE) {
-        if (t < a.ncell) bc_list_cell(a.p, a.npass, a.dim, a.W, ce, t, 0, a.nf);
+        if (t < a.ncell) bc_list_cell(a.heads, a.p, a.npass, a.dim, a.W, ce, t, 0, a.nf);
         else if (t - a.ncell < a.nface)
-            for (int c = 0; c < 3; c++) bc_list_face(a.p, a.npass, a.dim, a.B, ce, fe, t - a.ncell, c);
+            for (int c = 0; c < 3; c++) bc_list_face(a.heads, a.p, a.npass, a.dim, a.B, ce, fe, t - a.ncell, c);
         return;
     }
     const unsigned cells = a.ncell * (unsigned)a.nf;
     if (t < cells) {
         const int f = (int)(t / a.ncell);
-        bc_list_cell(a.p, a.npass, a.dim, a.W, ce, t % a.ncell, f, f + 1);
+        bc_list_cell(a.heads, a.p, a.npass, a.dim, a.W, ce, t % a.ncell, f, f + 1);
     } else if (t - cells < 3 * a.nface) {
-        bc_list_face(a.p, a.npass, a.dim, a.B, ce, fe, (t - cells) % a.nface, (int)((t - cells) / a.nface));
+        bc_list_face(a.heads, a.p, a.npass, a.dim, a.B, ce, fe, (t - cells) % a.nface, (int)((t - cells) / a.nface));
     }
 }
 template <bool WHOLE>
@@ -670,12 +679,12 @@ KB __global__ void k_bc_tail(BCListArgs a, const double* part, unsigned nparts, 
         if (t >= faces) {
             m = dmax(m, part[t - faces]);
         } else if (t >= a.ncell) {
-            bc_list_face(a.p, a.npass, D, a.B, a.ce, a.fe, (t - a.ncell) % a.nface, (int)((t - a.ncell) / a.nface));
+            bc_list_face(a.heads, a.p, a.npass, D, a.B, a.ce, a.fe, (t - a.ncell) % a.nface, (int)((t - a.ncell) / a.nface));
         } else {
             int i, j, k;
             cell_shell(a.ce, D).point(t, i, j, k);
             double u[8] = {};
-            bc_list_cell(a.p, a.npass, D, a.W, a.ce, t, 0, MHD ? 8 : 5, u);
+            bc_list_cell(a.heads, a.p, a.npass, D, a.W, a.ce, t, 0, MHD ? 8 : 5, u);
             if (i < -1 || i > a.ce.n[0] || (D >= 2 && (j < -1 || j > a.ce.n[1])) || (D >= 3 && (k < -1 || k > a.ce.n[2]))) continue;
             const P<double> w{u[F_RHO], u[F_P], u[F_VX], u[F_VY], u[F_VZ], u[F_BX], u[F_BY], u[F_BZ]};
             m = dmax(m, cfl_speed_w<D, MHD>(w, ph, mode, dx, dy, dz));
@@ -2120,7 +2129,7 @@ KB __global__ void k_apply1(Soa W, Soa Wn, FSoa F, Ext ce, const StepDts* ts, Ph
 // bits).  Bound by latency on the grids 1D problems have: the three separate
 // passes cost 12 us of launches, arrays written and read back, and a CFL scan
 // of every cell.  1024 cells, a frame of 20 steps, with the boundary and the
-// CFL in one launch too: 495 -> 329 us.
+// CFL in one launch too: 495 -> 329 us (308 with bc_head and the early loads).
 constexpr int STEP1_CELLS = 4 * 62;  // per workgroup of four wavefronts
 template <class R> __device__ __forceinline__ U<double> flux_down1(const U<R>& f) {
     return U<double>{__shfl_down(f.rho, 1), __shfl_down(f.E, 1), __shfl_down(f.mx, 1), __shfl_down(f.my, 1),
@@ -2128,22 +2137,21 @@ template <class R> __device__ __forceinline__ U<double> flux_down1(const U<R>& f
 }
 template <bool MHD, class R>
 KS __global__ void k_step1(Soa W, Soa Wn, Ext ce, const StepDts* ts, Phys ph, unsigned long long* err, double* cflpart) {
-    if (stopped(ts)) return;
-    const double dt_dx = dts(ts, 0);
     const int lane = threadIdx.x & 63, g = ce.g, n = ce.n[0];
     const long m = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * 62 + lane - 1;
     const int i = (int)m - g;
     const bool live = m >= 0 && m < ce.size;
-    P<double> w{};
-    P<R> L = pzero<R>(), Rr = pzero<R>();
-    if (live) {
-        w = load_p<double>(W, m, MHD);
-        const P<R> wc = p_cast<R>(w);
-        if (i >= -g + 1 && i < n + g - 1)
-            muscl<MHD, R>(load_p<R>(W, m - 1, MHD), L, wc, Rr, load_p<R>(W, m + 1, MHD), R(dt_dx), R(0), R(0), R(0), ph);
-        else
-            L = Rr = wc;
+    const bool inner = live && i >= -g + 1 && i < n + g - 1;
+    P<double> w{}, wl{}, wr{};
+    if (live) w = load_p<double>(W, m, MHD);
+    if (inner) {
+        wl = load_p<double>(W, m - 1, MHD);
+        wr = load_p<double>(W, m + 1, MHD);
     }
+    if (stopped(ts)) return;  // after the loads, so that they need not wait for it
+    const double dt_dx = dts(ts, 0);
+    P<R> L = p_cast<R>(w), Rr = L;
+    if (inner) muscl<MHD, R>(p_cast<R>(wl), L, p_cast<R>(w), Rr, p_cast<R>(wr), R(dt_dx), R(0), R(0), R(0), ph);
     const P<R> l = shfl_up1(Rr);
     U<R> f = uzero<R>();
     if (live && lane >= 1 && i >= -g + 1) {
@@ -2276,6 +2284,8 @@ static bool bc_list_fits(BCListArgs& a) {
     if (cells * a.nf + fcs * 3 > 2e9) return false;
     a.ncell = cell_shell(a.ce, a.dim).count();
     a.nface = faces ? face_shell(a.ce, a.dim).count() : 0;
+    a.heads = 0;
+    for (int q = 0; q < a.npass; q++) a.heads |= bc_head(a.p[q]) << (8 * q);
     return true;
 }
 bool launch_bc_list(BCListArgs& a, hipStream_t s) {
@@ -2827,8 +2837,8 @@ KB __global__ void kb_bc(BatchArgs A, BlockTable bt, BCPasses bc) {
     BATCH_ITEM(bt)
     const PatchView v = patch_view(A, p);
     const unsigned nc = cell_shell(v.ce, 2).count(), nf = face_shell(v.ce, 2).count(), u = (unsigned)t;
-    if (u < 8 * nc) bc_list_cell(bc.p, 4, 2, v.W, v.ce, u % nc, (int)(u / nc), (int)(u / nc) + 1);
-    else if (u - 8 * nc < 3 * nf) bc_list_face(bc.p, 4, 2, v.B, v.ce, v.fe, (u - 8 * nc) % nf, (int)((u - 8 * nc) / nf));
+    if (u < 8 * nc) bc_list_cell(bc.heads, bc.p, 4, 2, v.W, v.ce, u % nc, (int)(u / nc), (int)(u / nc) + 1);
+    else if (u - 8 * nc < 3 * nf) bc_list_face(bc.heads, bc.p, 4, 2, v.B, v.ce, v.fe, (u - 8 * nc) % nf, (int)((u - 8 * nc) / nf));
 }
 KB __global__ void kb_init_B(BatchArgs A, BlockTable bt) {
     BATCH_ITEM(bt)
