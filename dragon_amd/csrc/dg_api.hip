@@ -120,7 +120,6 @@ static Phys make_phys(const dg_desc& d) {
     const double g = d.gamma;
     p.gamma = g; p.gm1 = g - 1.0;
     p.k1_4pi = 0.25 / M_PI; p.k1_8pi = 0.125 / M_PI; p.sq4pi = std::sqrt(4.0 * M_PI);
-    p.inv_gm1 = 1.0 / p.gm1; p.inv_sq4pi = 1.0 / p.sq4pi;
     p.Gm1_2G = (g - 1.0) / (2.0 * g); p.Gp1_2G = (g + 1.0) / (2.0 * g); p._2G_Gm1 = 2.0 * g / (g - 1.0);
     p.Gm1_2 = (g - 1.0) / 2.0; p._2_Gm1 = 2.0 / (g - 1.0); p._2_Gp1 = 2.0 / (g + 1.0);
     p.Gm1_Gp1 = (g - 1.0) / (g + 1.0); p.Ginv = 1.0 / g;

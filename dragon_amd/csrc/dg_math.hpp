@@ -18,7 +18,6 @@ namespace dg {
 struct Phys {
     double gamma, gm1;          // gamma, gamma - 1.0
     double k1_4pi, k1_8pi, sq4pi;
-    double inv_gm1, inv_sq4pi;  // correctly rounded reciprocals (Den)
     // Exact-solver gamma combinations (Constants.h:33-40)
     double Gm1_2G, Gp1_2G, _2G_Gm1, Gm1_2, _2_Gm1, _2_Gp1, Gm1_Gp1, Ginv;
     int limiter;                // Limiters.cpp dispatch
@@ -44,63 +43,8 @@ enum { RF_OK = 0, RF_BAD_INPUT = 1, RF_BAD_SOLUTION = 2 };
 template <class T> __device__ __forceinline__ T dmin(T a, T b) { return (b < a) ? b : a; }  // std::min
 template <class T> __device__ __forceinline__ T dmax(T a, T b) { return (a < b) ? b : a; }  // std::max
 template <class T> __device__ __forceinline__ T dabs(T a) { return __builtin_fabs(a); }
+__device__ __forceinline__ double dsqrt(double a) { return __builtin_sqrt(a); }
 __device__ __forceinline__ float dsqrt(float a) { return __builtin_sqrtf(a); }
-// FP64 square roots and quotients are a third of the sweeps' instructions, and
-// each quotient starts with a quarter-rate reciprocal.  The compiler's
-// sequences first rescale their operands (for results near the ends of the
-// exponent range) and start from the reciprocal anew for every numerator.
-// Here the operands are used as they are, and quotients by one denominator
-// share its refined reciprocal.  The arithmetic is otherwise the same
-// (Newton steps and one residual correction, each an fma), so the results are
-// the correctly rounded ones, bit for bit, for operands within about
-// 1e-290 .. 1e290; zeros, infinities and NaN give what the operation gives.
-// Measured against the plain operators (a frame of steps, FP64): 2D hydro
-// 1024^2 2216 -> 1976 us, 2D MHD 771 x 530 2486 -> 2285 us, 3D MHD
-// 240 x 200 x 261 19.9 -> 18.0 ms.  The limiters keep the operators: their
-// denominators differ per field and their numerators, products of
-// differences, may be as small as the range's end.
-__device__ __forceinline__ double dsqrt(double a) {
-#ifdef __AMDGCN__
-    const double y = __builtin_amdgcn_rsq(a);
-    double s = a * y, h = 0.5 * y;
-    const double r = __builtin_fma(-h, s, 0.5);
-    s = __builtin_fma(s, r, s);
-    h = __builtin_fma(h, r, h);
-    s = __builtin_fma(__builtin_fma(-s, s, a), h, s);
-    s = __builtin_fma(__builtin_fma(-s, s, a), h, s);
-    return __builtin_amdgcn_class(a, 0x260) ? a : s;  // -0, +0, +inf
-#else
-    return __builtin_sqrt(a);
-#endif
-}
-// Quotients by one denominator.
-template <class T> struct Den {
-    T b;
-    __device__ __forceinline__ explicit Den(T d) : b(d) {}
-    __device__ __forceinline__ Den(T d, double) : b(d) {}
-    __device__ __forceinline__ T q(T a) const { return a / b; }
-};
-template <> struct Den<double> {
-    double b, r;
-    __device__ __forceinline__ explicit Den(double d) : b(d) {
-#ifdef __AMDGCN__
-        r = __builtin_amdgcn_rcp(d);
-        r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
-        r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
-#else
-        r = 0;
-#endif
-    }
-    __device__ __forceinline__ Den(double d, double inv) : b(d), r(inv) {}  // inv: 1/d, correctly rounded
-    __device__ __forceinline__ double q(double a) const {
-#ifdef __AMDGCN__
-        const double y = a * r;
-        return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, y, a), r, y), b, a);
-#else
-        return a / b;
-#endif
-    }
-};
 __device__ __forceinline__ bool fin(double a) { return __builtin_isfinite(a); }
 __device__ __forceinline__ bool fin(float a) { return __builtin_isfinite(a); }
 
@@ -141,25 +85,22 @@ template <bool MHD, class T> __device__ __forceinline__ U<T> umul(U<T> a, T s) {
     return a;
 }
 template <bool MHD, class T> __device__ __forceinline__ U<T> udiv(U<T> a, T s) {
-    const Den<T> d(s);
-    a.rho = d.q(a.rho); a.mx = d.q(a.mx); a.my = d.q(a.my); a.mz = d.q(a.mz); a.E = d.q(a.E);
-    if constexpr (MHD) { a.Bx = d.q(a.Bx); a.By = d.q(a.By); a.Bz = d.q(a.Bz); }
+    a.rho /= s; a.mx /= s; a.my /= s; a.mz /= s; a.E /= s;
+    if constexpr (MHD) { a.Bx /= s; a.By /= s; a.Bz /= s; }
     return a;
 }
 
 // ---- conversions (FluidElement.cpp:35-66)
 template <bool MHD, class T> __device__ __forceinline__ T energy(const P<T>& w, const Phys& ph) {
-    T E = Den<T>(T(ph.gm1), ph.inv_gm1).q(w.p) + (w.rho / 2) * dot3(w.vx, w.vy, w.vz, w.vx, w.vy, w.vz);
+    T E = w.p / T(ph.gm1) + (w.rho / 2) * dot3(w.vx, w.vy, w.vz, w.vx, w.vy, w.vz);
     if constexpr (MHD) E += dot3(w.Bx, w.By, w.Bz, w.Bx, w.By, w.Bz) * T(ph.k1_8pi);
     return E;
 }
-// rho: u.rho; the reference divides by 2 rho (a power of two off, exactly)
-template <bool MHD, class T> __device__ __forceinline__ T pressure(const U<T>& u, const Den<T>& rho, const Phys& ph) {
-    T Et = u.E - T(0.5) * rho.q(dot3(u.mx, u.my, u.mz, u.mx, u.my, u.mz));
+template <bool MHD, class T> __device__ __forceinline__ T pressure(const U<T>& u, const Phys& ph) {
+    T Et = u.E - dot3(u.mx, u.my, u.mz, u.mx, u.my, u.mz) / (2 * u.rho);
     if constexpr (MHD) Et -= dot3(u.Bx, u.By, u.Bz, u.Bx, u.By, u.Bz) * T(ph.k1_8pi);
     return T(ph.gm1) * Et;
 }
-template <bool MHD, class T> __device__ __forceinline__ T pressure(const U<T>& u, const Phys& ph) { return pressure<MHD>(u, Den<T>(u.rho), ph); }
 template <bool MHD, class T> __device__ __forceinline__ U<T> cons(const P<T>& w, const Phys& ph) {
     U<T> u;
     u.rho = w.rho;
@@ -170,17 +111,16 @@ template <bool MHD, class T> __device__ __forceinline__ U<T> cons(const P<T>& w,
 }
 template <bool MHD, class T> __device__ __forceinline__ P<T> prim(const U<T>& u, const Phys& ph) {
     P<T> w;
-    const Den<T> rho(u.rho);
     w.rho = u.rho;
-    w.vx = rho.q(u.mx); w.vy = rho.q(u.my); w.vz = rho.q(u.mz);
-    w.p = pressure<MHD>(u, rho, ph);
+    w.vx = u.mx / u.rho; w.vy = u.my / u.rho; w.vz = u.mz / u.rho;
+    w.p = pressure<MHD>(u, ph);
     if constexpr (MHD) { w.Bx = u.Bx; w.By = u.By; w.Bz = u.Bz; } else { w.Bx = w.By = w.Bz = 0; }
     return w;
 }
 template <bool MHD, class T> __device__ __forceinline__ T enthalpy(const P<T>& w, const Phys& ph) {  // :69-75
     T h = energy<MHD>(w, ph) + w.p;
     if constexpr (MHD) h += dot3(w.Bx, w.By, w.Bz, w.Bx, w.By, w.Bz) * T(ph.k1_8pi);
-    return Den<T>(w.rho).q(h);
+    return h / w.rho;
 }
 template <bool MHD, class T> __device__ __forceinline__ bool physical(const P<T>& w) {  // :82-87
     if constexpr (MHD) { if (!(fin(w.Bx) && fin(w.By) && fin(w.Bz))) return false; }
@@ -195,12 +135,11 @@ template <bool MHD, class T> __device__ __forceinline__ bool physical(const U<T>
 }
 
 // ---- wave speeds (FluidElement.cpp:99-120)
-template <class T> __device__ __forceinline__ T cs(const P<T>& w, const Phys& ph) { return dsqrt(Den<T>(w.rho).q(T(ph.gamma) * w.p)); }
+template <class T> __device__ __forceinline__ T cs(const P<T>& w, const Phys& ph) { return dsqrt(T(ph.gamma) * w.p / w.rho); }
 template <class T> __device__ __forceinline__ T c_fast(const P<T>& w, T Bk, const Phys& ph) {
-    const Den<T> rho(w.rho);
-    T c = dsqrt(rho.q(T(ph.gamma) * w.p));  // cs
-    T a = Den<T>(T(ph.sq4pi), ph.inv_sq4pi).q(dsqrt(rho.q(dot3(w.Bx, w.By, w.Bz, w.Bx, w.By, w.Bz))));
-    T c2 = c * c, a2 = a * a, ak2 = rho.q(Bk * Bk) * T(ph.k1_4pi);
+    T c = cs(w, ph);
+    T a = dsqrt(dot3(w.Bx, w.By, w.Bz, w.Bx, w.By, w.Bz) / w.rho) / T(ph.sq4pi);
+    T c2 = c * c, a2 = a * a, ak2 = (Bk * Bk / w.rho) * T(ph.k1_4pi);
     T s = c2 + a2;
     T disc = dmax(T(0), (s * s) * T(0.25) - ak2 * c2);
     return dsqrt((c2 + a2) * T(0.5) + dsqrt(disc));
@@ -332,8 +271,7 @@ template <bool MHD, class T> __device__ __forceinline__ U<T> hll_s(const P<T>& L
 // Roe average (HLL.cpp:21-37)
 template <bool MHD, class T> __device__ __forceinline__ P<T> roe_avg(const P<T>& L, const P<T>& R, const Phys& ph) {
     T sql = dsqrt(L.rho), sqr = dsqrt(R.rho);
-    const Den<T> sum(sql + sqr);
-    T a = sum.q(sql), b = sum.q(sqr);
+    T a = sql / (sql + sqr), b = sqr / (sql + sqr);
     P<T> w;
     w.rho = sql * sqr;
     w.vx = L.vx * a + R.vx * b; w.vy = L.vy * a + R.vy * b; w.vz = L.vz * a + R.vz * b;
@@ -341,7 +279,7 @@ template <bool MHD, class T> __device__ __forceinline__ P<T> roe_avg(const P<T>&
     else { w.Bx = w.By = w.Bz = 0; }
     T H = a * enthalpy<MHD>(L, ph) + b * enthalpy<MHD>(R, ph);
     T a2 = T(ph.gm1) * (H - dot3(w.vx, w.vy, w.vz, w.vx, w.vy, w.vz) / 2);
-    w.p = Den<T>(T(ph.gamma), ph.Ginv).q(a2 * w.rho);
+    w.p = a2 * w.rho / T(ph.gamma);
     return w;
 }
 template <bool MHD, class T> __device__ U<T> hll(P<T> L, P<T> R, const Phys& ph) {  // HLL.cpp:42-60
@@ -358,8 +296,7 @@ template <bool MHD, class T> __device__ U<T> hll(P<T> L, P<T> R, const Phys& ph)
 }
 template <bool MHD, class T> __device__ U<T> hlle(P<T> L, P<T> R, const Phys& ph) {  // HLL.cpp:61-83
     T sql = dsqrt(L.rho), sqr = dsqrt(R.rho);
-    const Den<T> sum(sql + sqr);
-    T a = sum.q(sql), b = sum.q(sqr);
+    T a = sql / (sql + sqr), b = sqr / (sql + sqr);
     T aL, aR;
     if constexpr (MHD) {
         T Bx = (L.Bx + R.Bx) / 2;
@@ -368,7 +305,7 @@ template <bool MHD, class T> __device__ U<T> hlle(P<T> L, P<T> R, const Phys& ph
     } else {
         aL = cs(L, ph); aR = cs(R, ph);
     }
-    T v = sum.q(R.vx - L.vx);
+    T v = (R.vx - L.vx) / (sql + sqr);
     T d = (a * aL * aL + b * aR * aR) + T(0.5) * (sql * sqr) * v * v;
     d = dsqrt(d);
     T u = a * L.vx + b * R.vx;
@@ -383,47 +320,47 @@ template <class T> __device__ U<T> hllc(const P<T>& L, const P<T>& R, const Phys
     if (sl >= T(0)) return pflux<false>(L, ph);
     if (sr <= T(0)) return pflux<false>(R, ph);
     T pr = R.p + R.rho * R.vx * (R.vx - sr), pl = L.p + L.rho * L.vx * (L.vx - sl);
-    T sc = Den<T>(R.rho * (R.vx - sr) - L.rho * (L.vx - sl)).q(pr - pl);
+    T sc = (pr - pl) / (R.rho * (R.vx - sr) - L.rho * (L.vx - sl));
     const P<T> X = psel(sc > T(0), L, R);
     T sx = sc > T(0) ? sl : sr;
     U<T> UX = cons<false>(X, ph);
     U<T> Us = udiv<false>(umul<false>(UX, sx - X.vx), sx - sc);
     Us.mx = Us.rho * sc;
-    Us.E += Us.rho * (sc - X.vx) * (sc + Den<T>(X.rho * (sx - X.vx)).q(X.p));
+    Us.E += Us.rho * (sc - X.vx) * (sc + X.p / (X.rho * (sx - X.vx)));
     return uadd<false>(flux<false>(UX, X.vx, X.vy, X.vz, ph), umul<false>(usub<false>(Us, UX), sx));
 }
 
 // ---- HLLD (HLLD.cpp), MHD
 template <class T>
-__device__ __forceinline__ void outer_star(U<T>& us, const P<T>& K, T xK, T SK, T SM, const Den<T>& SKM, T pT, T Bx, const Phys& ph) {
+__device__ __forceinline__ void outer_star(U<T>& us, const P<T>& K, T xK, T SK, T SM, T pT, T Bx, const Phys& ph) {
     T Bx2 = (Bx * Bx) * T(ph.k1_4pi);  // HLLD.cpp:21-37
     T den = xK * (SK - SM) - Bx2;
     bool tiny = dabs(den) < T(1e-12);
-    const Den<T> d(den);
-    if (tiny) { us.By = K.By; us.Bz = K.Bz; }
+    if (tiny) { us.Bx = K.Bx; us.By = K.By; us.Bz = K.Bz; }
     else {
         T s = xK * (SK - K.vx) - Bx2;
-        us.By = d.q(K.By * s); us.Bz = d.q(K.Bz * s);
+        us.Bx = K.Bx * s / den; us.By = K.By * s / den; us.Bz = K.Bz * s / den;
     }
     us.Bx = Bx;
     T vsx, vsy, vsz;
-    if (tiny) { vsy = K.vy - T(0); vsz = K.vz - T(0); }
+    if (tiny) { vsx = K.vx - T(0); vsy = K.vy - T(0); vsz = K.vz - T(0); }
     else {
         T s = SM - K.vx;
-        vsy = K.vy - d.q(K.By * Bx * s) * T(ph.k1_4pi);
-        vsz = K.vz - d.q(K.Bz * Bx * s) * T(ph.k1_4pi);
+        vsx = K.vx - K.Bx * Bx * s / den * T(ph.k1_4pi);
+        vsy = K.vy - K.By * Bx * s / den * T(ph.k1_4pi);
+        vsz = K.vz - K.Bz * Bx * s / den * T(ph.k1_4pi);
     }
     vsx = SM;
     us.mx = vsx * us.rho; us.my = vsy * us.rho; us.mz = vsz * us.rho;
     us.E = energy<true>(K, ph) * (SK - K.vx);
     us.E += pT * SM - (K.p + dot3(K.Bx, K.By, K.Bz, K.Bx, K.By, K.Bz) * T(ph.k1_8pi)) * K.vx;
     us.E += Bx * (dot3(K.vx, K.vy, K.vz, K.Bx, K.By, K.Bz) - dot3(vsx, vsy, vsz, us.Bx, us.By, us.Bz)) * T(ph.k1_4pi);
-    us.E = SKM.q(us.E);
+    us.E /= (SK - SM);
 }
 template <class T>
 __device__ __forceinline__ void outer_star_zero(U<T>& us, const P<T>& K, T SK, T SM, T pT, const Phys& ph) {  // :137-150
-    if (dabs(SK - SM) < T(1e-12)) { us.By = K.By; us.Bz = K.Bz; }
-    else { T s = SK - K.vx; const Den<T> d(SK - SM); us.By = d.q(K.By * s); us.Bz = d.q(K.Bz * s); }
+    if (dabs(SK - SM) < T(1e-12)) { us.Bx = K.Bx; us.By = K.By; us.Bz = K.Bz; }
+    else { T s = SK - K.vx, d = SK - SM; us.Bx = K.Bx * s / d; us.By = K.By * s / d; us.Bz = K.Bz * s / d; }
     us.Bx = 0;
     us.mx = SM * us.rho; us.my = K.vy * us.rho; us.mz = K.vz * us.rho;
     us.E = energy<true>(K, ph) * (SK - K.vx);
@@ -432,9 +369,8 @@ __device__ __forceinline__ void outer_star_zero(U<T>& us, const P<T>& K, T SK, T
 }
 template <class T> __device__ __forceinline__ P<T> star_prim(const U<T>& us, T pT, const Phys& ph) {
     P<T> w;
-    const Den<T> rho(us.rho);
     w.rho = us.rho;
-    w.vx = rho.q(us.mx); w.vy = rho.q(us.my); w.vz = rho.q(us.mz);
+    w.vx = us.mx / us.rho; w.vy = us.my / us.rho; w.vz = us.mz / us.rho;
     w.Bx = us.Bx; w.By = us.By; w.Bz = us.Bz;
     w.p = pT - dot3(w.Bx, w.By, w.Bz, w.Bx, w.By, w.Bz) * T(ph.k1_8pi);
     return w;
@@ -481,13 +417,11 @@ template <class T> __device__ U<T> hlld_uniform(P<T> L, P<T> R, const Phys& ph) 
     T pTL = L.p + dot3(L.Bx, L.By, L.Bz, L.Bx, L.By, L.Bz) * T(ph.k1_8pi);
     T pTR = R.p + dot3(R.Bx, R.By, R.Bz, R.Bx, R.By, R.Bz) * T(ph.k1_8pi);
     T xL = L.rho * (SL - L.vx), xR = R.rho * (SR - R.vx);
-    const Den<T> dx(xR - xL);
-    T SM = dx.q((xR * R.vx - xL * L.vx) - (pTR - pTL));
+    T SM = ((xR * R.vx - xL * L.vx) - (pTR - pTL)) / (xR - xL);
     U<T> usL = uzero<T>(), usR = uzero<T>();
-    const Den<T> SLM(SL - SM), SRM(SR - SM);
-    usL.rho = SLM.q(xL);
-    usR.rho = SRM.q(xR);
-    T pT = dx.q(xR * pTL - xL * pTR + xL * xR * (R.vx - L.vx));
+    usL.rho = xL / (SL - SM);
+    usR.rho = xR / (SR - SM);
+    T pT = (xR * pTL - xL * pTR + xL * xR * (R.vx - L.vx)) / (xR - xL);
     P<T> wsL, wsR;
     if (zeroB && !supL && !supR) {  // HLLD_zero_B (HLLD.cpp:152-205)
         wsL = pzero<T>(); wsR = pzero<T>();
@@ -507,11 +441,11 @@ template <class T> __device__ U<T> hlld_uniform(P<T> L, P<T> R, const Phys& ph) 
         T a = sql / (sql + sqr), b = sqr / (sql + sqr);
         return uadd<true>(umul<true>(star_flux(L, usL, SL, ph), a), umul<true>(star_flux(R, usR, SR, ph), b));
     }
-    T SsL = SM - Den<T>(T(ph.sq4pi) * dsqrt(usL.rho)).q(dabs(Bx));
-    T SsR = SM + Den<T>(T(ph.sq4pi) * dsqrt(usR.rho)).q(dabs(Bx));
-    outer_star(usL, L, xL, SL, SM, SLM, pT, Bx, ph);
+    T SsL = SM - dabs(Bx) / (T(ph.sq4pi) * dsqrt(usL.rho));
+    T SsR = SM + dabs(Bx) / (T(ph.sq4pi) * dsqrt(usR.rho));
+    outer_star(usL, L, xL, SL, SM, pT, Bx, ph);
     wsL = star_prim(usL, pT, ph);
-    outer_star(usR, R, xR, SR, SM, SRM, pT, Bx, ph);
+    outer_star(usR, R, xR, SR, SM, pT, Bx, ph);
     wsR = star_prim(usR, pT, ph);
     // region of the face, in the reference's order of tests
     const bool sub = !supL && !supR;
@@ -526,20 +460,20 @@ template <class T> __device__ U<T> hlld_uniform(P<T> L, P<T> R, const Phys& ph) 
     // double-star state (used by dstar faces only)
     const P<T> ws = psel(SM >= T(0), wsL, wsR);
     T sqL = dsqrt(wsL.rho), sqR = dsqrt(wsR.rho);
-    const Den<T> sum(sqL + sqR);
-    T a = sum.q(sqL), b = sum.q(sqR);
+    T a = sqL / (sqL + sqR), b = sqR / (sqL + sqR);
     T sbx = Bx > T(0) ? T(ph.sq4pi) : (Bx < T(0) ? -T(ph.sq4pi) : T(0));
+    T sum = sqL + sqR;
     P<T> wss;
     U<T> uss;
     wss.rho = ws.rho;
     uss.rho = wss.rho;
     wss.vx = SM;
-    wss.vy = wsL.vy * a + wsR.vy * b + sum.q((usR.By - usL.By) * sbx * T(ph.k1_4pi));
-    wss.vz = wsL.vz * a + wsR.vz * b + sum.q((usR.Bz - usL.Bz) * sbx * T(ph.k1_4pi));
+    wss.vy = wsL.vy * a + wsR.vy * b + (usR.By - usL.By) * sbx * T(ph.k1_4pi) / sum;
+    wss.vz = wsL.vz * a + wsR.vz * b + (usR.Bz - usL.Bz) * sbx * T(ph.k1_4pi) / sum;
     uss.mx = wss.vx * uss.rho; uss.my = wss.vy * uss.rho; uss.mz = wss.vz * uss.rho;
     wss.Bx = Bx;
-    wss.By = usR.By * a + usL.By * b + sum.q((wsR.vy - wsL.vy) * sbx * sqL * sqR);
-    wss.Bz = usR.Bz * a + usL.Bz * b + sum.q((wsR.vz - wsL.vz) * sbx * sqL * sqR);
+    wss.By = usR.By * a + usL.By * b + (wsR.vy - wsL.vy) * sbx * sqL * sqR / sum;
+    wss.Bz = usR.Bz * a + usL.Bz * b + (wsR.vz - wsL.vz) * sbx * sqL * sqR / sum;
     uss.Bx = wss.Bx; uss.By = wss.By; uss.Bz = wss.Bz;
     T dE = sbx * (dot3(ws.vx, ws.vy, ws.vz, ws.Bx, ws.By, ws.Bz) - dot3(wss.vx, wss.vy, wss.vz, wss.Bx, wss.By, wss.Bz)) *
            T(ph.k1_4pi) * dsqrt(wss.rho);
@@ -576,13 +510,11 @@ template <class T> __device__ U<T> hlld_branch(P<T> L, P<T> R, const Phys& ph) {
     T pTL = L.p + dot3(L.Bx, L.By, L.Bz, L.Bx, L.By, L.Bz) * T(ph.k1_8pi);
     T pTR = R.p + dot3(R.Bx, R.By, R.Bz, R.Bx, R.By, R.Bz) * T(ph.k1_8pi);
     T xL = L.rho * (SL - L.vx), xR = R.rho * (SR - R.vx);
-    const Den<T> dx(xR - xL);
-    T SM = dx.q((xR * R.vx - xL * L.vx) - (pTR - pTL));
+    T SM = ((xR * R.vx - xL * L.vx) - (pTR - pTL)) / (xR - xL);
     U<T> usL = uzero<T>(), usR = uzero<T>();
-    const Den<T> SLM(SL - SM), SRM(SR - SM);
-    usL.rho = SLM.q(xL);
-    usR.rho = SRM.q(xR);
-    T pT = dx.q(xR * pTL - xL * pTR + xL * xR * (R.vx - L.vx));
+    usL.rho = xL / (SL - SM);
+    usR.rho = xR / (SR - SM);
+    T pT = (xR * pTL - xL * pTR + xL * xR * (R.vx - L.vx)) / (xR - xL);
     P<T> wsL = pzero<T>(), wsR = pzero<T>();
     if (zeroB) {
         if (SM >= T(0)) {
@@ -601,15 +533,15 @@ template <class T> __device__ U<T> hlld_branch(P<T> L, P<T> R, const Phys& ph) {
         T a = sql / (sql + sqr), b = sqr / (sql + sqr);
         return uadd<true>(umul<true>(star_flux(L, usL, SL, ph), a), umul<true>(star_flux(R, usR, SR, ph), b));
     }
-    T SsL = SM - Den<T>(T(ph.sq4pi) * dsqrt(usL.rho)).q(dabs(Bx));
-    T SsR = SM + Den<T>(T(ph.sq4pi) * dsqrt(usR.rho)).q(dabs(Bx));
+    T SsL = SM - dabs(Bx) / (T(ph.sq4pi) * dsqrt(usL.rho));
+    T SsR = SM + dabs(Bx) / (T(ph.sq4pi) * dsqrt(usR.rho));
     if (SsR >= T(0)) {
-        outer_star(usL, L, xL, SL, SM, SLM, pT, Bx, ph);
+        outer_star(usL, L, xL, SL, SM, pT, Bx, ph);
         wsL = star_prim(usL, pT, ph);
         if (ph.hlld_safety && (!physical<true>(wsL) || !physical<true>(usL, ph))) return hlle<true>(L, R, ph);
     }
     if (SsL <= T(0)) {
-        outer_star(usR, R, xR, SR, SM, SRM, pT, Bx, ph);
+        outer_star(usR, R, xR, SR, SM, pT, Bx, ph);
         wsR = star_prim(usR, pT, ph);
         if (ph.hlld_safety && (!physical<true>(wsR) || !physical<true>(usR, ph))) return hlle<true>(L, R, ph);
     }
@@ -617,20 +549,20 @@ template <class T> __device__ U<T> hlld_branch(P<T> L, P<T> R, const Phys& ph) {
     if (SsR <= T(0)) return star_flux(R, usR, SR, ph);
     const P<T> ws = psel(SM >= T(0), wsL, wsR);
     T sqL = dsqrt(wsL.rho), sqR = dsqrt(wsR.rho);
-    const Den<T> sum(sqL + sqR);
-    T a = sum.q(sqL), b = sum.q(sqR);
+    T a = sqL / (sqL + sqR), b = sqR / (sqL + sqR);
     T sbx = Bx > T(0) ? T(ph.sq4pi) : (Bx < T(0) ? -T(ph.sq4pi) : T(0));
+    T sum = sqL + sqR;
     P<T> wss;
     U<T> uss;
     wss.rho = ws.rho;
     uss.rho = wss.rho;
     wss.vx = SM;
-    wss.vy = wsL.vy * a + wsR.vy * b + sum.q((usR.By - usL.By) * sbx * T(ph.k1_4pi));
-    wss.vz = wsL.vz * a + wsR.vz * b + sum.q((usR.Bz - usL.Bz) * sbx * T(ph.k1_4pi));
+    wss.vy = wsL.vy * a + wsR.vy * b + (usR.By - usL.By) * sbx * T(ph.k1_4pi) / sum;
+    wss.vz = wsL.vz * a + wsR.vz * b + (usR.Bz - usL.Bz) * sbx * T(ph.k1_4pi) / sum;
     uss.mx = wss.vx * uss.rho; uss.my = wss.vy * uss.rho; uss.mz = wss.vz * uss.rho;
     wss.Bx = Bx;
-    wss.By = usR.By * a + usL.By * b + sum.q((wsR.vy - wsL.vy) * sbx * sqL * sqR);
-    wss.Bz = usR.Bz * a + usL.Bz * b + sum.q((wsR.vz - wsL.vz) * sbx * sqL * sqR);
+    wss.By = usR.By * a + usL.By * b + (wsR.vy - wsL.vy) * sbx * sqL * sqR / sum;
+    wss.Bz = usR.Bz * a + usL.Bz * b + (wsR.vz - wsL.vz) * sbx * sqL * sqR / sum;
     uss.Bx = wss.Bx; uss.By = wss.By; uss.Bz = wss.Bz;
     T dE = sbx * (dot3(ws.vx, ws.vy, ws.vz, ws.Bx, ws.By, ws.Bz) - dot3(wss.vx, wss.vy, wss.vz, wss.Bx, wss.By, wss.Bz)) *
            T(ph.k1_4pi) * dsqrt(wss.rho);
