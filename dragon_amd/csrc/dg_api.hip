@@ -48,6 +48,7 @@ struct dg_grid {
     StepCtl* ctl = nullptr;                    // device, behind dev_words: step sizes, failure word, control of a run of steps
     StepCtl* host_ctl = nullptr;               // its pinned mirror, behind host_words
     bool in_run = false;                       // the launches belong to a run of steps (advance_run)
+    bool bc_settled = false;                   // a second boundary pass would change nothing the last one left
     std::string err;
     // optional live timing of the step kernels with HIP events
     bool timing = false;
@@ -464,6 +465,7 @@ int dg_apply_boundary(dg_grid* g) { return apply_boundary(g, nullptr, nullptr); 
 // tail: the step of a run whose CFL tail may go with the boundary (*tailed).
 static int apply_boundary(dg_grid* g, const StepCtx* tail, bool* tailed) {
     if (!g) return DG_ERR_ARG;
+    g->bc_settled = false;
     if (g->bc_cb) {  // the caller applies the list itself (host-evaluated elements)
         g->cfl_cached = false;
         const int rc = g->bc_cb(g->bc_user);
@@ -475,7 +477,9 @@ static int apply_boundary(dg_grid* g, const StepCtx* tail, bool* tailed) {
     imp.kind = DG_BC_OUTFLOW; imp.faces = uncovered; imp.corners = 1; imp.gated = 0;
     tm_record(g, -1);
     if (tail) *tailed = apply_list(g, imp, tail);
-    if (!(tail && *tailed) && !apply_list(g, imp, nullptr)) {
+    // in one launch every ghost comes from points that no pass writes
+    g->bc_settled = (tail && *tailed) || apply_list(g, imp, nullptr);
+    if (!g->bc_settled) {
         apply_one(g, imp);
         for (auto& b : g->bcs) apply_one(g, b);
     }
@@ -576,7 +580,10 @@ int dg_step(dg_grid* g, double dt, dg_status* st) {
 // on its input; W is kept, so a failed step commits nothing.
 static int split_step(dg_grid* g, double dt, dg_status* st, bool filled);
 int dg_split_step(dg_grid* g, double dt, dg_status* st) { return split_step(g, dt, st, false); }
-// filled: the grid's boundary has just been applied (and W not changed since).
+// filled: the grid's boundary has just been applied, W not changed since, and
+// the pass before the first sweep would leave every ghost as it is.  (Not so
+// where a pass reads ghosts that another one wrote before or writes later: an
+// axis shorter than its ghosts, an element without corner ghosts.)
 static int split_step(dg_grid* g, double dt, dg_status* st, bool filled) {
     if (!g) return DG_ERR_ARG;
     const int D = g->d.dim;
@@ -757,7 +764,7 @@ static int advance_loop(dg_grid* g, double dt, int check_cfl, long max_steps, dg
         }
         while (true) {
             if (!attempted) {
-                rc = split ? split_step(g, t1, st, !g->bc_cb) : dg_step(g, t1, st);
+                rc = split ? split_step(g, t1, st, g->bc_settled) : dg_step(g, t1, st);
                 if (rc == DG_OK) break;
                 if (rc == DG_ERR_HIP || rc == DG_ERR_ARG || rc == DG_ERR_UNSUPPORTED) return rc;
             }
