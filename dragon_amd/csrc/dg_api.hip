@@ -704,6 +704,28 @@ static int advance_run(dg_grid* g, double left, int check_cfl, int n, int* done,
     return DG_OK;
 }
 
+// Steps of the first run of an advance with a limit on its steps (without one
+// the frame is as long as its time, which may be less than a step, and the
+// first run is one step).  Too few cost another wait, 15 to 20 us; where the
+// time ends first, the others are launched in vain, and a frame of one step
+// must then still not take longer than that step with a wait for the CFL step
+// and one for the failure word.  That holds up to about (FP64 and mixed):
+//   2D / 3D MHD: 7 steps in vain at 160 thousand cells, 4 at 500 thousand, 1.5
+//     at 1.1 million, none at 2 million (18 us each at 128^2, 195 at 96^3)
+//   2D hydro: 5 up to 160 thousand, 6 at 500 thousand, 3 at 1.1 million
+//   1D: 1.6 (13 us each, as long as the step itself); 3D hydro: 1.1
+// With 8 for both kinds up to 2 million cells a frame of one step took 1D 104
+// us, 3D hydro 16^3 332, 2D MHD 128^2 200, 96^3 2197; by its time now 28, 127,
+// 77 and 830.
+static long first_run(const dg_grid* g) {
+    const long n = g->ce.size;
+    const int D = g->d.dim;
+    if (D == 1) return n < 1L << 21 ? 2 : 1;
+    if (D == 3 && !g->d.mhd) return 1;
+    if (n < 150000) return g->d.mhd ? 8 : 4;
+    return n < 600000 ? 4 : n < 1200000 ? 2 : 1;
+}
+
 // Grid::advance_unsplit / advance_split (CFL.cpp:160-238)
 static int advance_loop(dg_grid* g, double dt, int check_cfl, long max_steps, dg_stats* stats, dg_status* st, bool split) {
     dg_stats local{};
@@ -711,14 +733,11 @@ static int advance_loop(dg_grid* g, double dt, int check_cfl, long max_steps, dg
     S.steps = 0; S.failures = 0; S.t_advanced = 0;
     const double tol = g->d.timestep_tol;
     // Steps of a run are launched ahead where a user's boundary, the split
-    // sweeps and the live timing do not need the host between them.  How many:
-    // 8 at first on small grids (a step launched in vain costs a few
-    // microseconds there), one on large ones (a wait is nothing to their
-    // steps, an empty launch of millions of workgroups is not), then what the
-    // last step says is left.
+    // sweeps and the live timing do not need the host between them: first as
+    // many as first_run says, then what the last step says is left.
     const bool runs = !split && !g->bc_cb && !g->timing;
     const long small = 1L << 21;
-    long ahead = g->ce.size < small ? 8 : 1;
+    long ahead = max_steps >= 0 ? first_run(g) : 1;
     while (dt > tol) {
         if (max_steps >= 0 && S.steps >= max_steps) break;
         int rc = DG_OK;
