@@ -1527,7 +1527,9 @@ int dg_batch_autotune(dg_batch* b, int reps, int* chunk_out, double* class_ms) {
         if (!ncls[c]) continue;
         double best = 1e300;
         int pick = b->chunk[c];
-        for (int k : cand) {  // x sweep: faces per walker
+        const int tile = b->chunk[c];  // the present one is a candidate too, the default of few patches being none of the list
+        for (int q = -1; q < (int)(sizeof cand / sizeof *cand); q++) {  // x sweep: faces per walker
+            const int k = q < 0 ? tile : cand[q];
             b->chunk[c] = k;
             if (batch_table(b, BK_PRED_X) || batch_table(b, BK_FLUX_X)) return DG_ERR_HIP;
             float ms = 0;
