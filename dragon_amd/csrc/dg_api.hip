@@ -675,10 +675,11 @@ static int advance_run(dg_grid* g, double left, int check_cfl, int n, int* done,
         StepCtx c = make_ctx(g);
         bool begun = false;
         rc = apply_boundary(g, check_cfl && cached ? &c : nullptr, &begun);
-        if (begun) {}
-        else if (!check_cfl) launch_ctl_next(c, g->s);
-        else if (cached) launch_cfl_tail(c, g->ncflpart, nullptr, true, g->s);
-        else launch_cfl(c, nullptr, true, g->s);
+        if (!begun) {  // the CFL tail did not go with the boundary
+            if (!check_cfl) launch_ctl_next(c, g->s);
+            else if (cached) launch_cfl_tail(c, g->ncflpart, nullptr, true, g->s);
+            else launch_cfl(c, nullptr, true, g->s);
+        }
         g->ncflpart = c.mixed ? p32::launch_step(c, g->s) : p64::launch_step(c, g->s);
         cached = g->cflpart != nullptr;
         std::swap(g->W, g->Wn);

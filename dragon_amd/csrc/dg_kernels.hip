@@ -2259,10 +2259,10 @@ void launch_bc(const BCArgs& a, bool faces, hipStream_t s) {
 }
 
 constexpr unsigned BC_WHOLE = 65536;  // ghost cells from which a thread copies every field of one
-// False where the list does not fit k_bc_list: an axis with a pass and fewer
-// than ng + 2 cells, two passes on one face, a periodic axis with another
-// pass, or more threads than 32 bits count.
-// Whether the list's passes fit one launch; counts its points.
+// Whether the list's passes fit one launch (k_bc_list); counts its points and
+// packs its heads.  They do not: an axis with a pass and fewer than ng + 2
+// cells, two passes on one face, a periodic axis with another pass, or more
+// threads than 32 bits count.
 static bool bc_list_fits(BCListArgs& a) {
     int on[3] = {0, 0, 0}, periodic[3] = {0, 0, 0};
     for (int q = 0; q < a.npass; q++) {
@@ -2288,6 +2288,7 @@ static bool bc_list_fits(BCListArgs& a) {
     for (int q = 0; q < a.npass; q++) a.heads |= bc_head(a.p[q]) << (8 * q);
     return true;
 }
+// False (nothing done) where the list does not fit one launch.
 bool launch_bc_list(BCListArgs& a, hipStream_t s) {
     if (a.npass == 0) return true;
     if (!bc_list_fits(a)) return false;
@@ -2763,9 +2764,9 @@ void ctu_hydro3(const StepCtx& c, hipStream_t s) {
 // Many independent 2D MHD patches (CTU + CT) advanced stage by stage: each
 // launch below covers every active patch through a block table, and runs the
 // same kernel body as the single-grid step over the patch's own arrays.  The
-// step is begin -> boundary passes -> CFL -> dt -> predictor sweeps -> EMF ->
-// half-step faces -> half-step state -> corrector sweeps -> EMF -> Faraday ->
-// apply -> commit, a fixed sequence a graph can replay.  A patch whose
+// step is boundary -> CFL -> dt -> predictor sweeps x, y -> half-step CT ->
+// corrector sweeps x, y -> final CT and apply -> commit, which begins the next
+// step (kb_begin the first), a fixed sequence a graph can replay.  A patch whose
 // attempt fails keeps its state and retries at half the dt in the next step
 // (the dt halving of Grid::advance, CFL.cpp:151-213, one attempt per step).
 struct PatchView {
@@ -2831,8 +2832,13 @@ KB __global__ void kb_begin(BatchArgs A) {
 }
 // The boundary pass of every patch in one launch (bc_list_cell / _face, a
 // thread per ghost cell and field or boundary face and component): the two
-// sides of x, then of y, outflow or periodic.  (Four launches of one pass
-// each took 43 us of the 1.05 ms step of 96 patches.)
+// sides of x, then of y, outflow or periodic.  Sides of 4 cells, the least a
+// patch has, are enough (bc_list_fits asks for ng + 2 for the sake of mirrored
+// points): an outflow ghost comes from cell 0 or n - 1 and its face from faces
+// 0, 1 or n, n - 1, a periodic one from ng = 3 points away from the other end,
+// [n - 3, n) or [0, 3), and none of these is a ghost or, of the faces, one that
+// a pass writes.  (Four launches of one pass each took 43 us of the 1.05 ms step
+// of 96 patches.)
 KB __global__ void kb_bc(BatchArgs A, BlockTable bt, BCPasses bc) {
     BATCH_ITEM(bt)
     const PatchView v = patch_view(A, p);
