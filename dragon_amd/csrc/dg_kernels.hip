@@ -1171,8 +1171,8 @@ __device__ __forceinline__ void sweep_march_body(const SweepArgs& a, long t) {
 // (133 registers, 8 bytes per lane spilled at four, 5-8% faster than three)
 // and the parked corrector (116-118 registers).  1 = the compiler's choice.
 // The FP64 2D hydro corrector is eight registers over three waves: held there
-// it spills 12 bytes per lane.  Hydro 1024^2: 262 -> 250 us per step.  (The 3D
-// hydro one spills 44 to 84: 150 x 128 x 170 2% slower.)
+// it spills 12 bytes per lane.  Hydro 1024^2: 267 -> 261 us per step, 1800^2 760
+// -> 732.  (The 3D hydro one spills 44 to 84: 150 x 128 x 170 2% slower.)
 template <int D, bool MHD, class R, bool FINAL> constexpr bool corrector_2d_hydro() { return D == 2 && !MHD && FINAL && sizeof(R) == 8; }
 template <int D, bool MHD, int AX, class R, bool FINAL, class RS> constexpr int march_min_waves() {
     if (corrector_2d_hydro<D, MHD, R, FINAL>()) return 3;
@@ -1273,7 +1273,8 @@ KS __attribute__((amdgpu_waves_per_eu(wave_min_waves<R>()))) __global__ void k_s
 // in the sweeps above, and corrected and solved in FP64 in both forms.  The
 // half states as arrays (six of them, written once, read by six corner passes
 // and rewritten by six correction passes) cost 420 field accesses a cell where
-// this takes 190: 150 x 128 x 170 FP64 2.5 -> @@ ms a step.
+// this takes 190: 150 x 128 x 170 2.63 -> 2.19 ms a step in FP64, 2.30 -> 1.61
+// mixed.
 template <class R, int AX>
 __device__ __forceinline__ void corner_states(const SweepArgs& a, const int* idx, const P<R>& wl, const P<R>& wc, const P<R>& wr,
                                               P<double>& L1, P<double>& R1, P<double>& L2, P<double>& R2) {
@@ -2465,12 +2466,19 @@ static void sweep(const StepCtx& c, int ax, const Box& b, const FSoa& out, int s
     else { if constexpr (D >= 3) sweep_t<D, MHD, R, FINAL, 2, RS>(c, b, out, stage, s); }
 }
 // The sweeps of all axes: in one launch up to this many workgroups (about 4
-// million cells).  Per step, apart -> together: 3D MHD 24^3 FP64 146 -> 95 us,
-// 64 x 32 x 32 164 -> 136, 128^3 1772 -> 1743, but 160^3 (22 thousand) 3166 ->
-// 3171 and 240 x 200 x 261 8776 -> 9124; 2D MHD 128^2 81 -> 65, 1024^2 557 ->
-// 528, 2048^2 (19 thousand) 1887 -> 1911; 2D hydro 1800^2 762 -> 741; 3D hydro
-// 150 x 128 x 170 (17 thousand) 2054 -> 2010.
-constexpr unsigned MERGE_WORKGROUPS = 18000;
+// million cells; mixed 3D MHD 1.5 million: the two walkers in the one launch
+// take 24 KB of LDS each, three workgroups per CU).  Per step,
+// apart -> together, FP64 / mixed:
+//   3D MHD 24^3 143 -> 84 / 110 -> 72 us, 64 x 32 x 32 187 -> 148 / 136 -> 102,
+//     96^3 (6 thousand mixed) 921 -> 856 / 517 -> 480, 128^3 (13 thousand
+//     mixed) 1949 -> 1890 / 1063 -> 1063, 144^3 2713 -> 2636 / 1413 -> 1439;
+//     160^3 (22 thousand) and up, when it was tried, no faster
+//   2D MHD 128^2 86 -> 60 / 69 -> 52, 1024^2 538 -> 499 / 295 -> 271, 1500^2
+//     1058 -> 1042 / 606 -> 585; 2048^2 (19 thousand) no faster
+//   2D hydro 1024^2 287 -> 259 / 149 -> 130, 1800^2 775 -> 725 / 359 -> 339
+//   3D hydro 64^3 319 -> 299 / 252 -> 238, 150 x 128 x 170 (17 thousand) 2236 ->
+//     2180 / 1599 -> 1598
+template <int D, bool MHD, class R> constexpr unsigned merge_workgroups() { return D == 3 && MHD && sizeof(R) == 4 ? 10000 : 18000; }
 template <int D, bool MHD, class R, bool FINAL, class RS = R>
 static void sweeps(const StepCtx& c, const Box b[3], const Soa out[3], int stage, int kernel_id, hipStream_t s) {
     SweepArgs a[3];
@@ -2478,7 +2486,7 @@ static void sweeps(const StepCtx& c, const Box b[3], const Soa out[3], int stage
     n[0] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 0>(c, b[0], fs(out[0]), stage, a[0]);
     n[1] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 1>(c, b[1], fs(out[1]), stage + 1, a[1]);
     if constexpr (D == 3) n[2] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 2>(c, b[2], fs(out[2]), stage + 2, a[2]);
-    if (n[0] + n[1] + n[2] <= MERGE_WORKGROUPS && !c.march_window) {
+    if (n[0] + n[1] + n[2] <= merge_workgroups<D, MHD, R>() && !c.march_window) {
         hipLaunchKernelGGL((k_sweeps<D, MHD, R, FINAL, RS>), dim3(n[0] + n[1] + n[2]), dim3(256), 0, s, a[0], a[1], a[D == 3 ? 2 : 1], n[0], n[1]);
         mark(c, kernel_id);
         return;
