@@ -1023,8 +1023,11 @@ static constexpr int NOALLOC_MAX_DEVICES = 64;
 static std::atomic<void*> g_scratch_ptr[NOALLOC_MAX_DEVICES] = {};
 static thread_local std::string g_noalloc_err;
 
-// Scratch layout of one step (the arrays dg_create allocates for the same
-// grid, minus the state): doubles from the start of the array.
+// Scratch layout of one step: doubles from the start of the array.  The sizes
+// are those of the reference-structured step where a grid's own step has come
+// to need less (1D: nothing; 3D hydro: six corner fluxes, which take the half
+// states' place, and no T): the limit that callers and dg_noalloc_scratch_bytes
+// see stays as it was.
 struct NoallocLayout {
     long words = 0, F = 0, Fp = -1, HS = -1, T = -1, Bh = -1, E0 = -1, Eh = -1, end = 0;
 };
@@ -1199,8 +1202,8 @@ static int batch_class(int nx, int ny) {
 // faces of all patches per resident walker), at most 6: the patches fill the
 // chip together, and within 5% of the best of 1..16 from 24 to 1000 patches
 // (130 thousand to 16 million zones, both forms).  With 8 to 32 by size class,
-// and the y sweep in segments of 64 lanes, 96 patches in FP64 took 1.05 ms a
-// step against 0.88, 192 mixed 1.10 against 0.97.
+// and the y sweep in segments of 64 lanes, 96 patches in FP64 take 1.10 ms a
+// step against 0.88, 192 mixed 1.04 against 0.90.
 static int batch_chunk(const dg_batch* b) {
     const double resident = b->d.precision == DG_MIXED ? 262144.0 : 131072.0;
     return (int)std::max(1.0, std::min(6.0, std::sqrt(2.0 * (double)b->zones / resident) + 0.5));

@@ -1939,7 +1939,7 @@ KB __global__ void k_apply(Soa W, Soa Wn, FSoa FX, FSoa FY, FSoa FZ, const doubl
 // (2048^2 mixed: 4.2-4.5 TB/s of the 4.8 a copy reaches) and, on small grids, by
 // latency.  Half step / final, against EMF + Faraday + whalf / apply: 2048^2
 // mixed 229 -> 216 / 307 -> 295 us, 771 x 530 FP64 43 -> 28 / 49 -> 32, 128^2 21
-// -> 10 / 23 -> 14; 96 patches FP64 0.88 -> 0.83 ms a step.  (Each thread
+// -> 10 / 23 -> 14; 96 patches FP64 50 us less a step.  (Each thread
 // evaluating its four corners itself, without LDS: 252 / 334 us at 2048^2.)
 struct PtrsCt {  // arguments of the single grid's passes
     Soa W, Wn;
@@ -2399,20 +2399,23 @@ static Box face_box(int D, const Ext& ce, int ax, int along_lo, int along_hi_inc
 // waves per SIMD in FP64, four in FP32), which costs half of c faces' time.
 // With F faces and R resident walkers the sum F/R (1 + 1/2c) + c/2 is least
 // near c = sqrt(F/R); measured, the half round costs a quarter of that, and
-// c = sqrt(2 F/R) lies within 10% of the best of 1..33 at every size tried
-// (64^3 to 240 x 200 x 261, 128^2 to 2048^2, both forms; 33 at 512^3).  With
-// at least 16 faces each, as before, small grids had fewer walkers than the
-// chip holds: x sweeps of 128^2 in FP64 102 -> 16 us, 771 x 530 123 -> 55 us,
-// 64 x 32 x 32 88 -> 18 us, 2048^2 mixed 174 -> 155 us.
-static long march_chunk(long faces, bool fp64) {
+// less where the other axes' sweeps share the launch (sweeps): c = sqrt(k F/R)
+// with k = 2 in a launch of one sweep, 8 in one of all.  Of k = 2, 4, 8, 14 and
+// 24 in shared launches, 8 lies within 5% of the best at every size from 40^3
+// to 160^3 and 256^2 to 2400^2, hydro and MHD, both forms; 2 is up to 16% off
+// (us a step, 2 -> 8: 64^3 MHD mixed 218 -> 195, 96^3 484 -> 468, 1024^2 mixed
+// hydro 134 -> 125, MHD 270 -> 258; FP64 263 -> 253, 502 -> 487).  With at least
+// 16 faces each small grids have fewer walkers than the chip holds (frames,
+// FP64: 128^2 2D MHD 2.03 ms against 0.52, 64 x 32 x 32 1.57 against 0.79).
+static long march_chunk(long faces, bool fp64, bool shared) {
     const double resident = fp64 ? 131072.0 : 262144.0;
-    return std::max(1L, (long)(std::sqrt(2.0 * (double)faces / resident) + 0.5));
+    return std::max(1L, (long)(std::sqrt((shared ? 8.0 : 2.0) * (double)faces / resident) + 0.5));
 }
 
 // Arguments of the sweep of axis AX over the face box b; the workgroups it
-// takes (0: no faces).
+// takes (0: no faces).  shared: in one launch with the other axes'.
 template <int D, bool MHD, bool FP64, bool FINAL, int AX>
-static unsigned sweep_args(const StepCtx& c, const Box& b, const FSoa& out, int stage, SweepArgs& a) {
+static unsigned sweep_args(const StepCtx& c, const Box& b, const FSoa& out, int stage, bool shared, SweepArgs& a) {
     a = SweepArgs{};
     a.W = c.W;
     for (int q = 0; q < 3; q++) {
@@ -2436,7 +2439,7 @@ static unsigned sweep_args(const StepCtx& c, const Box& b, const FSoa& out, int 
         a.chunk = 63;
         return blocks(waves * 64);
     } else {
-        const long chunk = std::min(len, c.march_chunk > 0 ? (long)c.march_chunk : march_chunk(len * ntrans, FP64));
+        const long chunk = std::min(len, c.march_chunk > 0 ? (long)c.march_chunk : march_chunk(len * ntrans, FP64, shared));
         a.chunk = (int)chunk;
         return blocks((len + chunk - 1) / chunk * ntrans);
     }
@@ -2445,7 +2448,7 @@ static unsigned sweep_args(const StepCtx& c, const Box& b, const FSoa& out, int 
 template <int D, bool MHD, class R, bool FINAL, int AX, class RS>
 static void sweep_t(const StepCtx& c, const Box& b, const FSoa& out, int stage, hipStream_t s) {
     SweepArgs a;
-    const unsigned n = sweep_args<D, MHD, sizeof(R) == 8, FINAL, AX>(c, b, out, stage, a);
+    const unsigned n = sweep_args<D, MHD, sizeof(R) == 8, FINAL, AX>(c, b, out, stage, false, a);
     if (!n) return;
     if constexpr (AX == D - 1) {
         hipLaunchKernelGGL((k_sweep_wave<D, MHD, R, AX, FINAL, RS>), dim3(n), dim3(256), 0, s, a);
@@ -2466,27 +2469,25 @@ static void sweep(const StepCtx& c, int ax, const Box& b, const FSoa& out, int s
     else { if constexpr (D >= 3) sweep_t<D, MHD, R, FINAL, 2, RS>(c, b, out, stage, s); }
 }
 // The sweeps of all axes: in one launch up to this many workgroups (about 4
-// million cells; mixed 3D MHD 1.5 million: the two walkers in the one launch
-// take 24 KB of LDS each, three workgroups per CU).  Per step,
-// apart -> together, FP64 / mixed:
-//   3D MHD 24^3 143 -> 84 / 110 -> 72 us, 64 x 32 x 32 187 -> 148 / 136 -> 102,
-//     96^3 (6 thousand mixed) 921 -> 856 / 517 -> 480, 128^3 (13 thousand
-//     mixed) 1949 -> 1890 / 1063 -> 1063, 144^3 2713 -> 2636 / 1413 -> 1439;
-//     160^3 (22 thousand) and up, when it was tried, no faster
-//   2D MHD 128^2 86 -> 60 / 69 -> 52, 1024^2 538 -> 499 / 295 -> 271, 1500^2
-//     1058 -> 1042 / 606 -> 585; 2048^2 (19 thousand) no faster
-//   2D hydro 1024^2 287 -> 259 / 149 -> 130, 1800^2 775 -> 725 / 359 -> 339
-//   3D hydro 64^3 319 -> 299 / 252 -> 238, 150 x 128 x 170 (17 thousand) 2236 ->
-//     2180 / 1599 -> 1598
-template <int D, bool MHD, class R> constexpr unsigned merge_workgroups() { return D == 3 && MHD && sizeof(R) == 4 ? 10000 : 18000; }
+// million cells).  Per step, apart -> together, FP64 / mixed:
+//   3D MHD 24^3 144 -> 84 / 111 -> 72 us, 64 x 32 x 32 189 -> 144 / 137 -> 104,
+//     96^3 922 -> 837 / 519 -> 465, 128^3 1945 -> 1852 / 1069 -> 1033, 160^3 (20
+//     thousand) 3573 -> 3460 / 1838 -> 1848; 176^3 (26 thousand) 4553 -> 4517 /
+//     no difference, and none beyond
+//   2D MHD 128^2 86 -> 60 / 70 -> 53, 1024^2 541 -> 487 / 295 -> 263, 2048^2 (18
+//     thousand) 1906 -> 1859 / 1105 -> 1067, 2400^2 (24 thousand) 2495 -> 2504 /
+//     1439 -> 1408
+//   2D hydro 1024^2 287 -> 253 / 148 -> 122, 2400^2 1243 -> 1200 / 619 -> 610
+//   3D hydro 64^3 320 -> 294 / 252 -> 228, 160^3 2738 -> 2694 / 1976 -> 1926
+constexpr unsigned MERGE_WORKGROUPS = 26000;
 template <int D, bool MHD, class R, bool FINAL, class RS = R>
 static void sweeps(const StepCtx& c, const Box b[3], const Soa out[3], int stage, int kernel_id, hipStream_t s) {
     SweepArgs a[3];
     unsigned n[3] = {0, 0, 0};
-    n[0] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 0>(c, b[0], fs(out[0]), stage, a[0]);
-    n[1] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 1>(c, b[1], fs(out[1]), stage + 1, a[1]);
-    if constexpr (D == 3) n[2] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 2>(c, b[2], fs(out[2]), stage + 2, a[2]);
-    if (n[0] + n[1] + n[2] <= merge_workgroups<D, MHD, R>() && !c.march_window) {
+    n[0] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 0>(c, b[0], fs(out[0]), stage, true, a[0]);
+    n[1] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 1>(c, b[1], fs(out[1]), stage + 1, true, a[1]);
+    if constexpr (D == 3) n[2] = sweep_args<D, MHD, sizeof(R) == 8, FINAL, 2>(c, b[2], fs(out[2]), stage + 2, true, a[2]);
+    if (n[0] + n[1] + n[2] <= MERGE_WORKGROUPS && !c.march_window) {
         hipLaunchKernelGGL((k_sweeps<D, MHD, R, FINAL, RS>), dim3(n[0] + n[1] + n[2]), dim3(256), 0, s, a[0], a[1], a[D == 3 ? 2 : 1], n[0], n[1]);
         mark(c, kernel_id);
         return;
@@ -2524,7 +2525,7 @@ static void hydro3_fluxes(const StepCtx& c, hipStream_t s) {
             const long waves = (ntrans * (len + 1) - 1 + 62) / 63;
             hipLaunchKernelGGL((k_corner_wave<R>), dim3(blocks(waves * 64)), dim3(256), 0, s, a);
         } else {
-            a.chunk = (int)std::min(len, c.march_chunk > 0 ? (long)c.march_chunk : march_chunk(len * ntrans, true));
+            a.chunk = (int)std::min(len, c.march_chunk > 0 ? (long)c.march_chunk : march_chunk(len * ntrans, true, false));
             const long nch = (len + a.chunk - 1) / a.chunk;
             if (ax == 0) hipLaunchKernelGGL((k_corner_march<R, 0>), dim3(blocks(nch * ntrans)), dim3(256), 0, s, a);
             else hipLaunchKernelGGL((k_corner_march<R, 1>), dim3(blocks(nch * ntrans)), dim3(256), 0, s, a);
@@ -2845,8 +2846,8 @@ KB __global__ void kb_begin(BatchArgs A) {
 // points): an outflow ghost comes from cell 0 or n - 1 and its face from faces
 // 0, 1 or n, n - 1, a periodic one from ng = 3 points away from the other end,
 // [n - 3, n) or [0, 3), and none of these is a ghost or, of the faces, one that
-// a pass writes.  (Four launches of one pass each took 43 us of the 1.05 ms step
-// of 96 patches.)
+// a pass writes.  (Four launches of one pass each took 43 us a step of 96
+// patches, this one 20.)
 KB __global__ void kb_bc(BatchArgs A, BlockTable bt, BCPasses bc) {
     BATCH_ITEM(bt)
     const PatchView v = patch_view(A, p);
@@ -3091,8 +3092,8 @@ KB __global__ void k_apply_axis(Soa W, Soa Wn, FSoa F, Ext ce, const StepDts* ts
 // Sweep and update of the contiguous axis in one pass: the lines' cells
 // streamed through wavefronts (sweep_stream_body), 62 of 64 lanes updating
 // their cell from the face below it and the next lane's, so the fluxes stay in
-// registers (1000 x 611 FP64: 44 -> 33 us with the gap between the launches).  Along the strided axes a
-// walker would solve a face more than it has cells: at the lengths that fill
+// registers (1000 x 611 FP64: 11 us less, the gap between the launches included).
+// Along the strided axes a walker would solve a face more than it has cells: at the lengths that fill
 // the chip (3 to 8) that costs what the flux array does.
 template <int D, class R>
 KS __global__ void k_split_wave(SweepArgs a, Soa Wn, SplitCfl cfl) {
@@ -3139,7 +3140,7 @@ static long split_axis_t(const StepCtx& c, const Soa& in, const Soa& out, hipStr
         const SplitCfl cfl{c.cflpart, c.cfl_mode, {c.d[0], c.d[1], c.d[2]}};
         if constexpr (AX == D - 1) {
             SweepArgs a;
-            if (!sweep_args<D, false, sizeof(RT) == 8, false, AX>(cs, b, fs(c.F[AX]), ST_FLUX_X + AX, a)) return 0;
+            if (!sweep_args<D, false, sizeof(RT) == 8, false, AX>(cs, b, fs(c.F[AX]), ST_FLUX_X + AX, false, a)) return 0;
             const unsigned n = blocks((ce.size + 61) / 62 * 64);
             hipLaunchKernelGGL((k_split_wave<D, RT>), dim3(n), dim3(256), 0, s, a, out, cfl);
             return n;

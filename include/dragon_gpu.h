@@ -193,7 +193,12 @@ int dg_timing(dg_grid* g, int enable, double* step_ms, long* steps);
 /* Per-kernel-class device time accumulated while timing is on (events after
  * each launch).  id in [0, count): returns the class name ("boundary", "cfl",
  * "pred_sweep_x", ..., "apply"), total ms and launches; DG_ERR_ARG past the
- * last class.  Instrumentation of this library, no reference counterpart. */
+ * last class.  A launch that does the work of several classes is counted in
+ * one of them: the sweeps of every axis in "pred_sweep_x" and "flux_sweep_x"
+ * where they share a launch (grids up to about 4 million cells), in 2D MHD the
+ * EMF and the half-step faces in "whalf", the EMF and Faraday in "apply", and the
+ * whole 1D step in "apply".  While timing is on, dg_advance waits for each step
+ * and each CFL step.  Instrumentation of this library, no reference counterpart. */
 int dg_kernel_time(dg_grid* g, int id, const char** name, double* ms, long* launches);
 /* Diagnostics: max over interior cells of |div B| * min(dx) / max|B_face| (0 for hydro / 1D). */
 int dg_divb(dg_grid* g, double* out);
@@ -266,8 +271,10 @@ int dg_batch_patch_stats(dg_batch* b, int patch, double* dt_last, long* steps, l
  * wavefronts, 63 cells each, with no segment boundary inside a column.
  * autotune times each candidate on the class's
  * patches (steps not committed), the x tile first, then the y width, and
- * keeps the fastest; class_ms (optional) gets the best time per launch.
- * Results do not depend on either shape. */
+ * keeps the fastest, the shapes the batch has among them; class_ms (optional)
+ * gets the best time per launch.  Results do not depend on either shape in
+ * FP64; in the mixed form the y shapes may differ in the last FP32 digit (the
+ * compiler contracts each copy of the sweep by itself). */
 int dg_batch_set_tiles(dg_batch* b, const int* chunk, int n);
 int dg_batch_get_tiles(const dg_batch* b, int* chunk, int n);
 int dg_batch_set_ysweep(dg_batch* b, const int* width, int n);
