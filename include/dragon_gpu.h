@@ -272,9 +272,7 @@ int dg_batch_patch_stats(dg_batch* b, int patch, double* dt_last, long* steps, l
  * autotune times each candidate on the class's
  * patches (steps not committed), the x tile first, then the y width, and
  * keeps the fastest, the shapes the batch has among them; class_ms (optional)
- * gets the best time per launch.  Results do not depend on either shape in
- * FP64; in the mixed form the y shapes may differ in the last FP32 digit (the
- * compiler contracts each copy of the sweep by itself). */
+ * gets the best time per launch.  Results do not depend on either shape. */
 int dg_batch_set_tiles(dg_batch* b, const int* chunk, int n);
 int dg_batch_get_tiles(const dg_batch* b, int* chunk, int n);
 int dg_batch_set_ysweep(dg_batch* b, const int* width, int n);
