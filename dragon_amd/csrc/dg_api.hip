@@ -746,7 +746,7 @@ static int advance_loop(dg_grid* g, double dt, int check_cfl, long max_steps, dg
         bool attempted = false;  // t1 was tried and failed
         if (runs) {
             long n = max_steps >= 0 ? std::min(max_steps - S.steps, ahead) : ahead;
-            n = std::max(1L, std::min<long>(n, CTL_RING));
+            n = check_cfl ? std::max(1L, std::min<long>(n, CTL_RING)) : 1;  // without CFL a step takes all the time left
             int done;
             rc = advance_run(g, dt, check_cfl, (int)n, &done, &attempted);
             if (rc) return rc;

@@ -42,3 +42,30 @@ def test_one_step_frame(name):
     print(f"{name}: one by one {apart * 1e6:.0f} us, a frame {frame * 1e6:.0f} us")
     assert gg.advance(dt) == (1, 0)
     assert frame <= 1.5 * apart
+
+
+@pytest.mark.parametrize("name", ["sod_1024", "ot_128", "turb_96"])
+def test_one_step_without_cfl(name):
+    """Without the CFL check one step takes all the time, whatever the limit
+    on steps."""
+    gg = gpu_grid(PROBLEMS[name]())
+    gg.advance(1e9, True, 2)
+    gg.apply_boundary()
+    dt = 0.1 * gg.cfl_time()
+
+    def median(f):
+        t = []
+        for _ in range(15):
+            t0 = time.perf_counter()
+            f()
+            t.append(time.perf_counter() - t0)
+        return np.median(t[3:])
+
+    def one_by_one():
+        gg.apply_boundary()
+        gg.unsplit_step(dt)
+
+    apart, frame = median(one_by_one), median(lambda: gg.advance(dt, False, 20))
+    print(f"{name}: one by one {apart * 1e6:.0f} us, a frame {frame * 1e6:.0f} us")
+    assert gg.advance(dt, False, 20) == (1, 0)
+    assert frame <= 1.5 * apart
