@@ -13,6 +13,8 @@ def test_tuning_keeps_the_untuned_tile_where_it_is_best():
     a step, the next best tile 102."""
     b, _ = build(0, [(60, 60, 4.0, 0.1, 1.5)])
     assert b.tiles()[0] == 1
+    b.run(200)  # the clock is up before anything is timed
+    b.sync()
     tiles, _ = b.autotune(reps=40)
     assert tiles[0] == 1
 
